@@ -193,6 +193,7 @@ struct WorkBufs {
     DevBuf tA, tB, tC; // per-target chunk buffers, C x P complex
     DevBuf pairs;      // chunk pair list
     DevBuf t0trace;    // S x P complex: summed type-0 target histograms
+    DevBuf dpart;      // S x splits x nr FP64 complex: partial direct sinc sums
     DevBuf shots;      // S erp_shot
     DevBuf prisms;
     DevBuf out;        // S x nr complex (device output staging)

@@ -3086,144 +3086,235 @@ __global__ void k_pair_targets_rows(int* __restrict__ ptgt, const int* __restric
 
 // ---------------------------------------------------------------------------
 // NoConv direct sums (reflRadarSignal / refrRadarSignal, radar_kernels.cu:
-// 58-159, 201-299): one thread per (shot, bin), facets streamed through LDS.
+// 58-159, 201-299): out[j] = sum_k c_k sinc((r_j - R_k) / res) over the terms
+// of a shot (its facets; or its type-0 targets times its facets).
+//
+// Bound by the evaluations, nr per term.  With a = r / res, b = R / res,
+//   sinc(a - b) = (sin(pi a) cos(pi b) - cos(pi a) sin(pi b)) / (pi (a - b)),
+// so with p = c cos(pi b) / pi and q = c sin(pi b) / pi, formed once per
+// term, a bin needs only w = 1 / (a - b) and the sums of p w and q w; the
+// sine and cosine of the bin are applied once at the end.  An evaluation is
+// then ten FP64 instructions (one reciprocal for two bins) instead of a
+// division, a phasor and a sine.  Everything is FP64: the two sums cancel to
+// |a - b| of their size near a bin's own range, down to the 1e-6 below which
+// the sinc is taken as 1.
+// Measured at 16 shots of 1000 bins, 8.8e3 facets and 9 targets each
+// (1.4e9 evaluations): a run takes 1.08 ms, against 29.3 ms with one thread
+// per bin evaluating phasor and sinc of every term, and every bin block
+// repeating the terms' geometry.
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(NT) k_refl_direct(
-    float2* __restrict__ refl, const erp_shot* __restrict__ shots, const int* __restrict__ Vs,
-    const int64_t* __restrict__ rec_base, Rec rec, KPar kp) {
-    const int s = blockIdx.y;
-    const int ir = blockIdx.x * NT + threadIdx.x;
-    const ShotK sh = load_shot(shots, s);
-    const int V = Vs[s];
-    const int64_t r0 = rec_base[s];
-    __shared__ double it_s[NT];
-    __shared__ float fre_s[NT];
-    const double r = (double)sh.rst + (double)ir * kp.drd;
-    const bool lossless = kp.mode & ERP_MODE_LOSSLESS;
-    (void)lossless;
-    // FP64 sums: V terms of either sign per bin (sinc sidelobes of facets at
-    // other ranges) cancel to a bin far smaller than its largest terms
-    double ax = 0.0, ay = 0.0;
-    for (int k0 = 0; k0 < V; k0 += NT) {
-        const int k = k0 + threadIdx.x;
-        if (k < V) {
-            it_s[threadIdx.x] = rec.itd[r0 + k];
-            fre_s[threadIdx.x] = rec.F[r0 + k];  // fRe stored in F for this mode
-        }
-        __syncthreads();
-        const int m = min(NT, V - k0);
-        for (int j = 0; j < m; ++j) {
-            const double itd = it_s[j];
-            const float dl = (float)((r - itd) / (double)kp.rng_res);
-            const float2 ph = phasor_cycles(-2.0 * itd * kp.inv_cyc);
-            const float sc = sinc_f(dl) * fre_s[j];
-            ax += (double)(ph.x * sc);
-            ay += (double)(ph.y * sc);
-        }
-        __syncthreads();
-    }
-    if (ir < kp.nr) refl[(size_t)s * kp.nr + ir] = make_float2((float)ax, (float)ay);
+constexpr int DS_BINS = 4;             // bins per thread
+constexpr int DS_TILE = NT * DS_BINS;  // bins per workgroup
+constexpr int DS_MIN_ITEMS = 4;        // term groups (of NT) worth a workgroup of their own
+// Partial rows a shot's terms are split into at most: enough workgroups for
+// one shot to fill the device, 1 MB of partial rows per shot.
+__host__ __device__ inline int direct_splits_max(int nr) {
+    const int n = 65536 / nr;
+    return n < 1 ? 1 : (n > 64 ? 64 : n);
+}
+// The splits of a shot with `items` term groups.  They depend on the shot
+// alone, so its sums do not depend on the batch it runs in.
+__device__ __forceinline__ int direct_splits(long long items, int nr) {
+    const long long n = (items + DS_MIN_ITEMS - 1) / DS_MIN_ITEMS;
+    const int m = direct_splits_max(nr);
+    return n < 1 ? 1 : (n > m ? m : (int)n);
 }
 
-__global__ void __launch_bounds__(NT) k_refr0_direct(
-    float2* __restrict__ refr, const float* __restrict__ tg, int64_t Tpad,
+// the term of facet record rr and the target at (tx, ty, tz): range R and
+// complex amplitude (refrRadarSignal)
+__device__ __forceinline__ void refr0_term(const Rec& rec, int64_t rr, double tx, double ty,
+                                           double tz, int V, const ShotK& sh,
+                                           const erp_prism* __restrict__ prisms, int np,
+                                           const KPar& kp, double* R, double2* c) {
+    const float fx = rec.geo[rr], fy = rec.geo[rec.cap + rr], fz = rec.geo[2 * rec.cap + rr];
+    const float nx = rec.geo[3 * rec.cap + rr], ny = rec.geo[4 * rec.cap + rr],
+                nz = rec.geo[5 * rec.cap + rr];
+    const float ux = rec.geo[6 * rec.cap + rr], uy = rec.geo[7 * rec.cap + rr],
+                uz = rec.geo[8 * rec.cap + rr];
+    const float vx = rec.geo[9 * rec.cap + rr], vy = rec.geo[10 * rec.cap + rr],
+                vz = rec.geo[11 * rec.cap + rr];
+    const double Itd = rec.itd[rr];
+    const double dx = tx - fx, dy = ty - fy, dz = tz - fz;
+    const double Ttd = dist3(dx, dy, dz);
+    const double invd = 1.0 / Ttd;
+    const double ix = dx * invd, iy = dy * invd, iz = dz * invd;
+    const float Ix = (float)ix, Iy = (float)iy, Iz = (float)iz;
+    const float2 csT = cos_sin_ref(ix, iy, iz, nx, ny, nz);
+    const float cT = csT.x, sT = csT.y;
+    float expo = 0.f, tot = 0.f;
+    for (int p = 0; p < np; ++p) {
+        const float d = prism_len(fx, fy, fz, Ix, Iy, Iz, prisms[p], (float)Ttd);
+        tot += d;
+        expo += prisms[p].alpha * d;
+    }
+    expo += kp.alpha2 * ((float)Ttd - tot);
+    const float kc = kp.ks * cT;
+    float EI = expf(-4.f * expo) * rec.fRfrC[rr] * expf(-4.f * kc * kc);
+    float EO = EI;
+    float Iu = Ix * ux + Iy * uy + Iz * uz;
+    float Iv = Ix * vx + Iy * vy + Iz * vz;
+    if (!kp.ortho) {
+        const float2 e = uv_dots_exact(ix, iy, iz, ux, uy, uz, vx, vy, vz);
+        Iu = e.x;
+        Iv = e.y;
+    }
+    const float Iph = rec.ang[rec.cap + rr], Rth = rec.ang[2 * rec.cap + rr];
+    const float Tth = atan2f(sT, cT);
+    const float Tph = atan2f(Iu, Iv);
+    const float si = sinf(Rth - Tth), dph = Iph - Tph;
+    const float a1 = sinc_f(kp.fs_lam * si * cosf(dph)), a2 = sinc_f(kp.fs_lam * si * sinf(dph));
+    const float vi = kp.fs2_lam * a1 * a2;
+    EI *= vi * vi;
+    const float sR = kp.sqrt_e2e1 * sinf(ERP_PI_F - Tth);
+    const float RrTh = (sR > 1.f) ? 1e4f : asinf(sR);
+    const float so = sinf(RrTh), dpo = Tph - Iph;
+    const float b1 = sinc_f(kp.fs_lam * so * cosf(dpo)), b2 = sinc_f(kp.fs_lam * so * sinf(dpo));
+    const float vo = kp.fs2_lam * b1 * b2;
+    EO *= vo * vo;
+    const double sl = Itd + Ttd;
+    const double sl2 = sl * sl;
+    const float req = (float)((double)V * ((double)(kp.P * sh.grefr * sh.grefr * kp.fs * kp.fs *
+                                                   kp.fs * kp.fs) /
+                                           (ERP_FOURPI5_SQ * sl2 * sl2)));
+    // refrRadarSignal passes d_Tth to rerad_funct (sim.cu:930-934)
+    const float amp = rerad_f(kp.rerad, Tth) * EI * EO * req;
+    const double rngt = madd_nc(sl - Ttd, Ttd, kp.cc2);
+    const float2 ph = phasor_cycles(-2.0 * rngt * kp.inv_cyc);
+    *R = rngt;
+    *c = make_double2((double)ph.x * amp, (double)ph.y * amp);
+}
+
+// Partial sums of one shot: workgroup (bin tile, split, shot) takes its
+// share of the shot's term groups in order.  REFR: the type-0 targets'
+// terms, else the facets' own (reflRadarSignal).
+template <bool REFR>
+__global__ void __launch_bounds__(NT) k_direct_part(
+    double2* __restrict__ part, const float* __restrict__ tg, int64_t Tpad,
     const int* __restrict__ list0, const int* __restrict__ tcnt, int Tcap,
     const erp_shot* __restrict__ shots, const int* __restrict__ Vs,
     const int64_t* __restrict__ rec_base, Rec rec, const erp_prism* __restrict__ prisms, int np,
     KPar kp) {
-    const int s = blockIdx.y;
-    const int ir = blockIdx.x * NT + threadIdx.x;
+    const int s = blockIdx.z, sp = blockIdx.y, tid = threadIdx.x;
+    const int V = Vs[s], nr = kp.nr;
+    const int groups = (V + NT - 1) / NT;
+    const long long items = (long long)groups * (REFR ? tcnt[2 * s + 1] : 1);
+    const int nsp = direct_splits(items, nr);
+    if (sp >= nsp) return;
+    const long long per = (items + nsp - 1) / nsp;
+    const long long i0 = per * sp, i1 = min(i0 + per, items);
     const ShotK sh = load_shot(shots, s);
-    const int V = Vs[s];
-    const int n0 = tcnt[2 * s + 1];
     const int64_t r0 = rec_base[s];
-    __shared__ double rng_s[NT];
-    __shared__ float rc_s[NT];
-    const double r = (double)sh.rst + (double)ir * kp.drd;
-    double ax = 0.0, ay = 0.0;  // FP64 sums, as in k_refl_direct
-    for (int ti = 0; ti < n0; ++ti) {
-        const int t = list0[(size_t)s * Tcap + ti];
-        const double tx = tg[t], ty = tg[Tpad + t], tz = tg[2 * Tpad + t];
-        for (int k0 = 0; k0 < V; k0 += NT) {
-            const int k = k0 + threadIdx.x;
-            if (k < V) {
-                const int64_t rr = r0 + k;
-                const float fx = rec.geo[rr], fy = rec.geo[rec.cap + rr], fz = rec.geo[2 * rec.cap + rr];
-                const float nx = rec.geo[3 * rec.cap + rr], ny = rec.geo[4 * rec.cap + rr],
-                            nz = rec.geo[5 * rec.cap + rr];
-                const double Itd = rec.itd[rr];
-                const double dx = tx - fx, dy = ty - fy, dz = tz - fz;
-                const double Ttd = dist3(dx, dy, dz);
-                const double invd = 1.0 / Ttd;
-                const double ix = dx * invd, iy = dy * invd, iz = dz * invd;
-                const float Ix = (float)ix, Iy = (float)iy, Iz = (float)iz;
-                const float2 csT = cos_sin_ref(ix, iy, iz, nx, ny, nz);
-                const float cT = csT.x;
-                float expo = 0.f, tot = 0.f;
-                for (int p = 0; p < np; ++p) {
-                    const float d = prism_len(fx, fy, fz, Ix, Iy, Iz, prisms[p], (float)Ttd);
-                    tot += d;
-                    expo += prisms[p].alpha * d;
-                }
-                expo += kp.alpha2 * ((float)Ttd - tot);
-                const float kc = kp.ks * cT;
-                const float fRfrC = rec.fRfrC[rr];
-                float EI = expf(-4.f * expo) * fRfrC * expf(-4.f * kc * kc);
-                float EO = EI;
-                {
-                    float Iu = Ix * rec.geo[6 * rec.cap + rr] + Iy * rec.geo[7 * rec.cap + rr] +
-                               Iz * rec.geo[8 * rec.cap + rr];
-                    float Iv = Ix * rec.geo[9 * rec.cap + rr] + Iy * rec.geo[10 * rec.cap + rr] +
-                               Iz * rec.geo[11 * rec.cap + rr];
-                    const float sT = csT.y;
-                    if (!kp.ortho) {
-                        const float2 e = uv_dots_exact(
-                            ix, iy, iz, rec.geo[6 * rec.cap + rr], rec.geo[7 * rec.cap + rr],
-                            rec.geo[8 * rec.cap + rr], rec.geo[9 * rec.cap + rr],
-                            rec.geo[10 * rec.cap + rr], rec.geo[11 * rec.cap + rr]);
-                        Iu = e.x;
-                        Iv = e.y;
-                    }
-                    const float Iph = rec.ang[rec.cap + rr], Rth = rec.ang[2 * rec.cap + rr];
-                    const float Tth = atan2f(sT, cT);
-                    const float Tph = atan2f(Iu, Iv);
-                    const float si = sinf(Rth - Tth), dph = Iph - Tph;
-                    const float a1 = sinc_f(kp.fs_lam * si * cosf(dph)),
-                                a2 = sinc_f(kp.fs_lam * si * sinf(dph));
-                    const float vi = kp.fs2_lam * a1 * a2;
-                    EI *= vi * vi;
-                    const float sR = kp.sqrt_e2e1 * sinf(ERP_PI_F - Tth);
-                    const float RrTh = (sR > 1.f) ? 1e4f : asinf(sR);
-                    const float so = sinf(RrTh), dpo = Tph - Iph;
-                    const float b1 = sinc_f(kp.fs_lam * so * cosf(dpo)),
-                                b2 = sinc_f(kp.fs_lam * so * sinf(dpo));
-                    const float vo = kp.fs2_lam * b1 * b2;
-                    EO *= vo * vo;
-                }
-                const double sl = Itd + Ttd;
-                const double sl2 = sl * sl;
-                const float req = (float)((double)V * ((double)(kp.P * sh.grefr * sh.grefr * kp.fs *
-                                                               kp.fs * kp.fs * kp.fs) /
-                                                       (ERP_FOURPI5_SQ * sl2 * sl2)));
-                // refrRadarSignal passes d_Tth to rerad_funct (sim.cu:930-934)
-                rc_s[threadIdx.x] =
-                    rerad_f(kp.rerad, atan2f(csT.y, cT)) * EI * EO * req;
-                rng_s[threadIdx.x] = madd_nc(sl - Ttd, Ttd, kp.cc2);
-            }
-            __syncthreads();
-            const int m = min(NT, V - k0);
-            for (int j = 0; j < m; ++j) {
-                const double rngt = rng_s[j];
-                const float dl = (float)((r - rngt) / (double)kp.rng_res);
-                const float2 ph = phasor_cycles(-2.0 * rngt * kp.inv_cyc);
-                const float sc = sinc_f(dl) * rc_s[j];
-                ax += (double)(ph.x * sc);
-                ay += (double)(ph.y * sc);
-            }
-            __syncthreads();
-        }
+    __shared__ double2 s_bp[NT], s_pq[NT];  // (b, p.x), (p.y, q.x)
+    __shared__ double s_qy[NT];
+    const double inv_res = 1.0 / (double)kp.rng_res;
+    const int j0 = blockIdx.x * DS_TILE + tid;
+    double a[DS_BINS], px[DS_BINS], py[DS_BINS], qx[DS_BINS], qy[DS_BINS];
+#pragma unroll
+    for (int k = 0; k < DS_BINS; ++k) {
+        a[k] = ((double)sh.rst + (double)(j0 + k * NT) * kp.drd) * inv_res;
+        px[k] = py[k] = qx[k] = qy[k] = 0.0;
     }
-    if (ir < kp.nr) refr[(size_t)s * kp.nr + ir] = make_float2((float)ax, (float)ay);
+    for (long long it = i0; it < i1; ++it) {
+        const int ti = REFR ? (int)(it / groups) : 0;
+        const int k0 = (int)(it - (long long)ti * groups) * NT;
+        if (k0 + tid < V) {
+            const int64_t rr = r0 + k0 + tid;
+            double R;
+            double2 c;
+            if (REFR) {
+                const int t = list0[(size_t)s * Tcap + ti];
+                refr0_term(rec, rr, tg[t], tg[Tpad + t], tg[2 * Tpad + t], V, sh, prisms, np, kp,
+                           &R, &c);
+            } else {
+                R = rec.itd[rr];
+                const float f = rec.F[rr];  // fRe, stored in F for this mode
+                const float2 ph = phasor_cycles(-2.0 * R * kp.inv_cyc);
+                c = make_double2((double)ph.x * f, (double)ph.y * f);
+            }
+            const double b = R * inv_res;
+            double sn, cs;
+            sincospi(b, &sn, &cs);
+            sn *= 0.31830988618379067;
+            cs *= 0.31830988618379067;
+            s_bp[tid] = make_double2(b, c.x * cs);
+            s_pq[tid] = make_double2(c.y * cs, c.x * sn);
+            s_qy[tid] = c.y * sn;
+        }
+        __syncthreads();
+        const int m = min(NT, V - k0);
+        for (int j = 0; j < m; ++j) {
+            const double2 bp = s_bp[j], pq = s_pq[j];
+            const double q1 = s_qy[j];
+#pragma unroll
+            for (int k = 0; k < DS_BINS; k += 2) {
+                const double d0 = a[k] - bp.x, d1 = a[k + 1] - bp.x;
+                // 1 / (d0 d1): the hardware FP32 reciprocal and one Newton
+                // step in FP64 (1e-13)
+                const double dd = d0 * d1;
+                const double y = (double)__builtin_amdgcn_rcpf((float)dd);
+                const double w = fma(fma(-dd, y, 1.0), y, y);
+                double w0 = d1 * w, w1 = d0 * w;
+                if (fmin(fabs(d0), fabs(d1)) < 1e-6) {
+                    // a range on a bin: sinc = 1 there, i.e. its c = pi (p
+                    // cos + q sin) added through the bin's own sine and cosine
+                    auto hit = [&](double ak, double d, double& ww, int e) {
+                        if (fabs(d) < 1e-6) {
+                            double sn, cs;
+                            sincospi(ak, &sn, &cs);
+                            const double cx = M_PI * (bp.y * cs + pq.y * sn),
+                                         cy = M_PI * (pq.x * cs + q1 * sn);
+                            px[e] += cx * sn;
+                            py[e] += cy * sn;
+                            qx[e] -= cx * cs;
+                            qy[e] -= cy * cs;
+                            ww = 0.0;
+                        } else {
+                            ww = 1.0 / d;
+                        }
+                    };
+                    hit(a[k], d0, w0, k);
+                    hit(a[k + 1], d1, w1, k + 1);
+                }
+                px[k] = fma(bp.y, w0, px[k]);
+                py[k] = fma(pq.x, w0, py[k]);
+                qx[k] = fma(pq.y, w0, qx[k]);
+                qy[k] = fma(q1, w0, qy[k]);
+                px[k + 1] = fma(bp.y, w1, px[k + 1]);
+                py[k + 1] = fma(pq.x, w1, py[k + 1]);
+                qx[k + 1] = fma(pq.y, w1, qx[k + 1]);
+                qy[k + 1] = fma(q1, w1, qy[k + 1]);
+            }
+        }
+        __syncthreads();
+    }
+    double2* row = part + ((size_t)s * direct_splits_max(nr) + sp) * nr;
+#pragma unroll
+    for (int k = 0; k < DS_BINS; ++k) {
+        const int j = j0 + k * NT;
+        if (j >= nr) continue;
+        double sn, cs;
+        sincospi(a[k], &sn, &cs);
+        row[j] = make_double2(sn * px[k] - cs * qx[k], sn * py[k] - cs * qy[k]);
+    }
+}
+
+// a shot's partial rows added in order (tcnt null: the facets' own terms)
+__global__ void __launch_bounds__(NT) k_direct_sum(float2* __restrict__ out,
+                                                   const double2* __restrict__ part,
+                                                   const int* __restrict__ Vs,
+                                                   const int* __restrict__ tcnt, int nr) {
+    const int s = blockIdx.y, j = blockIdx.x * NT + threadIdx.x;
+    if (j >= nr) return;
+    const long long items = (long long)((Vs[s] + NT - 1) / NT) * (tcnt ? tcnt[2 * s + 1] : 1);
+    const int nsp = direct_splits(items, nr);
+    const double2* row = part + (size_t)s * direct_splits_max(nr) * nr + j;
+    double ax = 0.0, ay = 0.0;
+    for (int sp = 0; sp < nsp; ++sp) {
+        const double2 v = row[(size_t)sp * nr];
+        ax += v.x;
+        ay += v.y;
+    }
+    out[(size_t)s * nr + j] = make_float2((float)ax, (float)ay);
 }
 
 // ---------------------------------------------------------------------------
@@ -3803,6 +3894,8 @@ int64_t erp_footprint_impl(const erp_params* par, int64_t F, int64_t T, int64_t 
     b += S * F * 136 + 2560;                  // facet records (136 B per facet-shot)
     b += S * P * 8 * 3 + S * M * 8;           // surface, spectral sum, type-0 rows; Bluestein
     b += S * nr * (16 + 8 + 16) + S * 4;      // FP64 surface bins, reflected, refracted
+    if (spec && !(par->mode & ERP_MODE_CONVOLUTION))
+        b += S * nr * 16 * direct_splits_max((int)nr);  // partial sinc sums
     if (T > 0) {
         const int64_t nbuf = spec ? 4 : 3;
         int64_t C = std::max<int64_t>(1, kPairRowBytes / (P * 8 * nbuf));
@@ -4009,6 +4102,8 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
                 buf(W.blu, sizeof(float2) * s * planM.N, "Bluestein rows");
             }
             if (any_t0) buf(W.t0trace, sizeof(float2) * s * P, "type-0 traces");
+            if (spec && !conv)
+                buf(W.dpart, sizeof(double2) * s * nr * direct_splits_max(nr), "partial sinc sums");
             if (T > 0) {
                 buf(W.tlist, sizeof(int) * s * (size_t)T * 2, "target lists");
                 buf(W.tcnt, sizeof(int) * s * 2, "target counts");
@@ -4077,6 +4172,9 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
         W.blu.ensure(sizeof(float2) * (size_t)Smax * planM.N);
     }
     if (any_t0) W.t0trace.ensure(sizeof(float2) * (size_t)Smax * P);
+    if (spec && !conv)
+        W.dpart.ensure(sizeof(double2) * (size_t)std::min<int64_t>(Smax, ns) * nr *
+                       direct_splits_max(nr));
     if (T > 0) {
         W.tlist.ensure(sizeof(int) * (size_t)Smax * T * 2);
         W.tcnt.ensure(sizeof(int) * (size_t)Smax * 2);
@@ -4338,9 +4436,15 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
             have_refl = true;
         } else if (spec && !conv) {
             PT_.begin(ERP_STAGE_OTHER, st, 0.0);
-            hipLaunchKernelGGL(k_refl_direct, dim3((nr + NT - 1) / NT, S), dim3(NT), 0, st, refl,
-                               dshots, dV, dbase, rec, kp);
-            ERP_CHECK_LAUNCH("k_refl_direct");
+            hipLaunchKernelGGL(k_direct_part<false>,
+                               dim3((nr + DS_TILE - 1) / DS_TILE, direct_splits_max(nr), S), dim3(NT),
+                               0, st, W.dpart.as<double2>(), (const float*)nullptr, (int64_t)0,
+                               (const int*)nullptr, (const int*)nullptr, 0, dshots, dV, dbase, rec,
+                               (const erp_prism*)nullptr, 0, kp);
+            ERP_CHECK_LAUNCH("k_direct_part");
+            hipLaunchKernelGGL(k_direct_sum, dim3((nr + NT - 1) / NT, S), dim3(NT), 0, st, refl,
+                               W.dpart.as<double2>(), dV, (const int*)nullptr, nr);
+            ERP_CHECK_LAUNCH("k_direct_sum");
             PT_.end(st);
             have_refl = true;
         }
@@ -4597,11 +4701,16 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
             if (n0 > 0) {
                 PT_.begin(ERP_STAGE_OTHER, st, (double)n0);
                 if (!conv) {
-                    hipLaunchKernelGGL(k_refr0_direct, dim3((nr + NT - 1) / NT, S), dim3(NT), 0, st,
-                                       refr0, targets->xyzn.as<float>(), Tpad, list0,
-                                       W.tcnt.as<int>(), Tcap, dshots, dV, dbase, rec, dpr,
-                                       (int)nprisms, kp);
-                    ERP_CHECK_LAUNCH("k_refr0_direct");
+                    hipLaunchKernelGGL(k_direct_part<true>,
+                                       dim3((nr + DS_TILE - 1) / DS_TILE, direct_splits_max(nr), S),
+                                       dim3(NT), 0, st, W.dpart.as<double2>(),
+                                       targets->xyzn.as<float>(), Tpad, list0, W.tcnt.as<int>(),
+                                       Tcap, dshots, dV, dbase, rec, dpr, (int)nprisms, kp);
+                    ERP_CHECK_LAUNCH("k_direct_part");
+                    hipLaunchKernelGGL(k_direct_sum, dim3((nr + NT - 1) / NT, S), dim3(NT), 0, st,
+                                       refr0, W.dpart.as<double2>(), dV,
+                                       (const int*)W.tcnt.as<int>(), nr);
+                    ERP_CHECK_LAUNCH("k_direct_sum");
                 } else {
                     float2* t0 = W.t0trace.as<float2>();
                     zero(t0, (size_t)S * P, st);
