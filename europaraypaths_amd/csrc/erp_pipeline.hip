@@ -47,6 +47,7 @@ constexpr int FPT = FB / NT;   // facets per thread (8)
 constexpr int WPB = NT / 64;   // waves per block
 constexpr int MASKW = FB / 64; // mask words per block (32)
 constexpr int SWIN = 2048;     // surface LDS window (bins)
+constexpr int LWIN = 1024;     // that of the surface kernel without records
 constexpr int TWIN = 4096;     // target LDS window (bins)
 constexpr int NTT = 512;       // threads per workgroup of the target kernels
 // (shot, target) pairs per target launch: their P-point rows take at most
@@ -1211,6 +1212,208 @@ __global__ void __launch_bounds__(NT) k_surface(
             vx = v.x;
             vy = v.y;
         }
+        const int b = base + k;
+        if (b < nr && (vx != 0.0 || vy != 0.0)) glb_add2d(row, b, vx, vy);
+    }
+}
+
+// The surface echo alone: surfacePT of every lit facet into FP64 bins, for
+// runs that keep no facet records (no targets), in the product's arithmetic
+// without ERP_RUN_DETERMINISTIC.  k_surface evaluates the same terms with
+// correctly rounded roots and divisions, which the records and the bounds of
+// the target kernels need.
+//
+// Bound by VALU issue: at 60 degrees every facet of a mesh is lit, a term
+// needs about 100 instructions and reads 48 bytes.  So, as in the target
+// kernels: range and 1 / range by one FP64 Newton step from the hardware
+// reciprocal root, the oracle's exact root and division only within 1e-7 bin
+// of a bin edge (bin indices stay identical), hardware sine, exponential
+// and reciprocal on reduced arguments, sqrt(fRe) formed directly, the
+// azimuth from unnormalised projections (only their ratio enters).  No
+// bounds, no ranks; only the bins a block's terms reach are cleared and
+// flushed.  Shots are the fast grid dimension: the workgroups that read one
+// facet block run together and find it in their L2.
+// Measured on the 2048 x 2048 mesh at 60 degrees, 50 shots (1.9e8 terms):
+// k_surface took 4.2 ms per launch, this kernel 1.15 ms; VALU 82 % busy with
+// 142 instructions per facet (176 with vector addresses for the loads, 1.28
+// ms).  Windows of 1024 bins instead of 2048 and the next facet's loads
+// ahead of the arithmetic gave 1.38 to 1.28 ms.
+template <bool REDUCE>
+__global__ void __launch_bounds__(NT) k_surface_lean(
+    const float* __restrict__ mesh, int64_t Fpad, const erp_shot* __restrict__ shots,
+    const unsigned long long* __restrict__ mask, const int* __restrict__ cnt, int nblk, KPar kp,
+    double2* __restrict__ srow, int64_t shot0, int tile_nx, int shot_fast) {
+    const int s = shot_fast ? blockIdx.x : blockIdx.y, blk = shot_fast ? blockIdx.y : blockIdx.x;
+    if (cnt[(size_t)s * nblk + blk] == 0) return;  // dark block (uniform exit)
+    const unsigned long long* mw = mask + ((size_t)s * nblk + blk) * MASKW;
+    __shared__ double swin[2 * LWIN];
+    __shared__ int b_s[2];
+    if (threadIdx.x < 2) b_s[threadIdx.x] = threadIdx.x ? -1 : 0x7FFFFFFF;
+    const ShotK sh = load_shot(shots, s);
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const bool lossless = kp.mode & ERP_MODE_LOSSLESS;
+    const bool incoh = kp.mode & ERP_MODE_INCOHERENT;
+    const double rst = (double)sh.rst, x0 = -rst * kp.inv_dr, two_cyc = 2.0 * kp.inv_cyc;
+    // amplitude without G1 / Dmax / Itd^2 and the loss; the four factors pi
+    // of the two pi-sincs squared
+    const float amp0 = kp.sqrtP * kp.lam * kp.lam * sh.grefr * kp.invK * kp.Dmax *
+                       (0.0102659823f * 0.0625f);
+    // exp(-2 (alpha1 Itd + (ks cI)^2)) as exp2
+    constexpr float m2l2e = -2.f * 1.44269504088896341f;
+    // pi-sincs from half their arguments h in revolutions, sin(2 pi |h|) / |h|
+    // (the four factors 2 in amp0); REDUCE: |h| may pass 256, up to which the
+    // hardware sine's own reduction is exact enough
+    const float hL = 0.5f * kp.piLlam;
+    auto pisinc = [](float h, float* num, float* den) {
+        const float ha = fmaxf(fabsf(h), 5e-7f);
+        *num = __builtin_amdgcn_sinf(REDUCE ? ha - rintf(ha) : ha);
+        *den = ha;
+    };
+    const float la = m2l2e * kp.alpha1, lk = m2l2e * kp.ks * kp.ks;
+
+    int bq[FPT];
+    float wq[FPT];
+    float2 cq[FPT];
+    int bmin = 0x7FFFFFFF, bmax = -1;
+    // facet_of(blk, q NT + threadIdx.x) = f0 + fv + q fstep, f0 uniform: the
+    // attribute loads take scalar bases and one 32-bit offset
+    int64_t f0 = (int64_t)blk * FB;
+    int fv = threadIdx.x, fstep = NT;
+    if (tile_nx) {
+        const int tpr = tile_nx / 64, trow = blk / tpr, tcol = blk - trow * tpr;
+        f0 = (int64_t)trow * 32 * tile_nx + (int64_t)tcol * 64;
+        fv = wv * tile_nx + lane;
+        fstep = WPB * tile_nx;
+    }
+    // (in scalar registers for good: folded into the offset sums again, they
+    // would cost a 64-bit vector addition per load)
+    typedef __attribute__((address_space(1))) const char* gbytes;
+    gbytes mp[12];
+#pragma unroll
+    for (int a = 0; a < 12; ++a) {
+        mp[a] = (gbytes)(mesh + (size_t)a * Fpad + f0);
+        asm("" : "+s"(mp[a]));
+    }
+    // the next facet's attributes are loaded before this one's arithmetic
+    float gq[2][12];
+    bool lit[FPT];
+#pragma unroll
+    for (int q = 0; q < FPT; ++q)
+        lit[q] = (mw[__builtin_amdgcn_readfirstlane(q * WPB + wv)] >> lane) & 1ull;
+    auto load = [&](int q) {
+        if (!lit[q]) return;
+        const unsigned off = (unsigned)(fv + q * fstep) * 4u;
+#pragma unroll
+        for (int a = 0; a < 12; ++a)
+            gq[q & 1][a] = *(__attribute__((address_space(1))) const float*)(mp[a] + off);
+    };
+    load(0);
+#pragma unroll
+    for (int q = 0; q < FPT; ++q) {
+        bq[q] = -1;
+        if (q + 1 < FPT) load(q + 1);
+        if (!lit[q]) continue;
+        const float(&g)[12] = gq[q & 1];
+        const double dx = (double)g[0] - sh.sx, dy = (double)g[1] - sh.sy,
+                     dz = (double)g[2] - sh.sz;
+        const double t2 = fma(dx, dx, fma(dy, dy, dz * dz));
+        const float rs = __builtin_amdgcn_rsqf((float)t2);
+        const double rd = (double)rs, hr = 0.5 * rd;
+        const double y0 = t2 * rd;
+        const double Itd = fma(fma(-y0, y0, t2), hr, y0);
+        const double xq = fma(Itd, kp.inv_dr, x0);
+        int b = (int)xq;
+        double w = xq - (double)b;
+        bool valid = (xq > -1.0) && (xq < (double)kp.nr);
+        if (w < 1e-7 || w > 1.0 - 1e-7) valid = bin_of(dist3(dx, dy, dz), rst, kp.drd, kp.nr, &b, &w);
+        if (!valid) continue;
+        // -I.n in FP64 (the sine near normal incidence needs it)
+        const double invd = rd * fma(-y0, hr, 1.5);
+        const double c0 = -fma(dx, (double)g[3], fma(dy, (double)g[4], dz * (double)g[5])) * invd;
+        const double cc = fmin(1.0, fmax(-1.0, c0));
+        const float cI = (float)cc, sI = __builtin_amdgcn_sqrtf((float)((1.0 - cc) * (1.0 + cc)));
+        const float fx = (float)dx, fy = (float)dy, fz = (float)dz;
+        float Iu = fx * g[6] + fy * g[7] + fz * g[8];
+        float Iv = fx * g[9] + fy * g[10] + fz * g[11];
+        if (!kp.ortho) {
+            const float2 e = uv_dots_exact(dx, dy, dz, g[6], g[7], g[8], g[9], g[10], g[11]);
+            Iu = e.x;
+            Iv = e.y;
+        }
+        // sin(Ith) (cos Iph, sin Iph); (sI, 0) where both projections vanish
+        const float r2 = Iu * Iu + Iv * Iv;
+        const bool az = r2 > 0.f;
+        const float ri = sI * __builtin_amdgcn_rsqf(az ? r2 : 1.f);
+        float n1, d1, n2, d2;
+        pisinc(hL * (az ? Iv * ri : sI), &n1, &d1);
+        pisinc(hL * (Iu * ri), &n2, &d2);
+        const float sc = n1 * n2 * __builtin_amdgcn_rcpf(d1 * d2);
+        float amp = amp0 * (sc * sc) * (rs * rs);
+        if (!lossless) {
+            // Snell and Fresnel (pol 0); past the critical angle cos(1e4)
+            const float sR = kp.sqrt_e1e2 * sI;
+            const float cR = sR > 1.0f ? cosf(1e4f)
+                                       : __builtin_amdgcn_sqrtf(fmaxf(0.f, 1.f - sR * sR));
+            const float rho = (kp.nu2 * cI - kp.nu1 * cR) *
+                              __builtin_amdgcn_rcpf(kp.nu2 * cI + kp.nu1 * cR);
+            amp *= fabsf(rho) * __builtin_amdgcn_exp2f(fmaf(lk * cI, cI, la * (float)Itd));
+        }
+        float2 ph;
+        if (incoh) {
+            float sn, cs;
+            sincospif(2.0f * incoherent_u(kp.seed, shot0 + s, f0 + fv + q * fstep), &sn, &cs);
+            ph = make_float2(cs, sn);
+        } else {
+            ph = phasor_rc_hw(Itd, two_cyc);
+        }
+        bq[q] = b;
+        wq[q] = (float)w;
+        cq[q] = make_float2(ph.x * amp, ph.y * amp);
+        bmin = min(bmin, b);
+        bmax = max(bmax, b);
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        bmin = min(bmin, __shfl_xor(bmin, o));
+        bmax = max(bmax, __shfl_xor(bmax, o));
+    }
+    __syncthreads();
+    if (lane == 0) {
+        atomicMin(&b_s[0], bmin);
+        atomicMax(&b_s[1], bmax);
+    }
+    __syncthreads();
+    const int base = b_s[0], nr = kp.nr;
+    if (base == 0x7FFFFFFF) return;  // no term within the bins
+    const int span = min(LWIN, b_s[1] + 2 - base);
+    for (int k = threadIdx.x; k < span; k += NT) swin[k] = swin[LWIN + k] = 0.0;
+    __syncthreads();
+    double2* row = srow + (size_t)s * nr;
+#pragma unroll
+    for (int q = 0; q < FPT; ++q) {
+        const int b = bq[q];
+        if (b < 0) continue;
+        // split in FP64, the window's precision: c1 = c w, c0 = c - c1
+        const double w = wq[q], cx = cq[q].x, cy = cq[q].y;
+        const double c1x = cx * w, c1y = cy * w;
+        const int k0 = b - base;
+        if (k0 < LWIN) {
+            atomicAdd(&swin[k0], cx - c1x);
+            atomicAdd(&swin[LWIN + k0], cy - c1y);
+        } else {
+            glb_add2d(row, b, cx - c1x, cy - c1y);
+        }
+        if (b + 1 < nr) {
+            if (k0 + 1 < LWIN) {
+                atomicAdd(&swin[k0 + 1], c1x);
+                atomicAdd(&swin[LWIN + k0 + 1], c1y);
+            } else {
+                glb_add2d(row, b + 1, c1x, c1y);
+            }
+        }
+    }
+    __syncthreads();
+    for (int k = threadIdx.x; k < span; k += NT) {
+        const double vx = swin[k], vy = swin[LWIN + k];
         const int b = base + k;
         if (b < nr && (vx != 0.0 || vy != 0.0)) glb_add2d(row, b, vx, vy);
     }
@@ -4382,12 +4585,23 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
         PT_.begin(ERP_STAGE_SURFACE, st, Vsum);
         if (do_trace) zero(W.srow.as<float2>(), srow_f2, st);
         const int write = (need_rec && Vtot > 0) ? 1 : 0;
-        hipLaunchKernelGGL(k_surface, dim3(nblk, S), dim3(NT), 0, st, mesh->soa.as<float>(),
-                           mesh->Fpad, F, dshots, dmask, W.off.as<int>(), dV, dbase, nblk, kp, rec,
-                           write, do_trace ? 1 : 0, srow, s0, dbounds, det ? 1 : 0, smax,
-                           tile_nx, ph, acc, (const TrackK*)nullptr, (const RowK*)nullptr, brk,
-                           T > 0 ? W.bbox.as<float4>() : nullptr);
-        ERP_CHECK_LAUNCH("k_surface");
+        if (T == 0 && !spec && !det && ph == PH_F64 && acc == ACC_F64) {
+            // no targets: nothing reads records or bounds (shots are the fast
+            // dimension where the blocks fit the other one)
+            const int shot_fast = nblk <= 65535 ? 1 : 0;
+            hipLaunchKernelGGL(kp.piLlam <= 512.f ? k_surface_lean<false> : k_surface_lean<true>,
+                               shot_fast ? dim3(S, nblk) : dim3(nblk, S), dim3(NT), 0, st,
+                               mesh->soa.as<float>(), mesh->Fpad, dshots, dmask, W.cnt.as<int>(),
+                               nblk, kp, srow, s0, tile_nx, shot_fast);
+            ERP_CHECK_LAUNCH("k_surface_lean");
+        } else {
+            hipLaunchKernelGGL(k_surface, dim3(nblk, S), dim3(NT), 0, st, mesh->soa.as<float>(),
+                               mesh->Fpad, F, dshots, dmask, W.off.as<int>(), dV, dbase, nblk, kp, rec,
+                               write, do_trace ? 1 : 0, srow, s0, dbounds, det ? 1 : 0, smax,
+                               tile_nx, ph, acc, (const TrackK*)nullptr, (const RowK*)nullptr, brk,
+                               T > 0 ? W.bbox.as<float4>() : nullptr);
+            ERP_CHECK_LAUNCH("k_surface");
+        }
         if (T > 0) {
             hipLaunchKernelGGL(k_shot_sphere, dim3(S), dim3(256), 0, st, dbounds,
                                (const float4*)W.bbox.as<float4>(), (const int*)W.cnt.as<int>(),
