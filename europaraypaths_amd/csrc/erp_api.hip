@@ -308,9 +308,12 @@ void erp_ctx_destroy(erp_ctx* ctx) {
     stop_slots(ctx);
     if (ctx->stream) hipStreamSynchronize(ctx->stream);
     for (auto* c : ctx->chirps) delete c;
-    for (auto* b : ctx->blues) delete b;
+    for (auto* b : ctx->bands) {
+        b->tab.release();
+        delete b;
+    }
     ctx->chirps.clear();
-    ctx->blues.clear();
+    ctx->bands.clear();
     release_work(ctx->work);
     mt_state_free(ctx->mt);
     ctx->mt = nullptr;
@@ -560,7 +563,7 @@ int erp_run_tracks(erp_ctx* ctx, const erp_track* tracks, int64_t ntracks, uint3
                                                   " belong to another context"};
         }
         set_device(ctx);
-        // the cached range kernel spectra and Bluestein tables the batches
+        // the cached range kernel spectra and band tables the batches
         // point to stay in the cache while the run holds them
         ctx->active.fetch_add(1);
         struct Hold {

@@ -25,6 +25,8 @@
 // and rounded once.
 #include "erp_internal.h"
 
+#include <cmath>
+
 namespace {
 
 constexpr int NT = 256;         // threads per workgroup
@@ -386,12 +388,19 @@ __global__ void __launch_bounds__(NT) k_tfft_cols_fwd(float2* __restrict__ data,
     }
 }
 
-__global__ void __launch_bounds__(NT) k_tfft_rows_conv(const float2* __restrict__ src,
-                                                       float2* __restrict__ dst, int N1,
+// (src and dst may be the same rows.  trk: each row with its track's surface
+// spectrum, a track without one giving zeros.)
+__global__ void __launch_bounds__(NT) k_tfft_rows_conv(const float2* src, float2* dst, int N1,
                                                        int log2N1, int N2,
                                                        const float2* __restrict__ G,
                                                        const float2* __restrict__ tw,
-                                                       const float2* __restrict__ it) {
+                                                       const float2* __restrict__ it,
+                                                       const TrackK* __restrict__ trk,
+                                                       const RowK* __restrict__ rk) {
+    if (trk) {
+        if (rk[blockIdx.y].shot < 0) return;
+        G = trk[rk[blockIdx.y].trk].g_surf;
+    }
     __shared__ float2 s[NPTS];
     __shared__ float2 twl[TWL];
     const int RT = NPTS / N1;
@@ -401,8 +410,9 @@ __global__ void __launch_bounds__(NT) k_tfft_rows_conv(const float2* __restrict_
     for (int i = threadIdx.x; i < NPTS; i += NT) s[sw(i)] = src[off + i];
     __syncthreads();
     lds_fft(s, N1, log2N1, RT, false, tws);
-    const float2* Gr = G + (size_t)r0 * N1;
-    for (int i = threadIdx.x; i < NPTS; i += NT) s[sw(i)] = cmul(s[sw(i)], Gr[i]);
+    const float2* Gr = G ? G + (size_t)r0 * N1 : nullptr;
+    for (int i = threadIdx.x; i < NPTS; i += NT)
+        s[sw(i)] = Gr ? cmul(s[sw(i)], Gr[i]) : make_float2(0.f, 0.f);
     __syncthreads();
     lds_fft(s, N1, log2N1, RT, true, tws);
     for (int i = threadIdx.x; i < NPTS; i += NT)
@@ -483,8 +493,10 @@ __global__ void __launch_bounds__(NT) k_tfft_rows_mac(const float2* __restrict__
 }
 
 // Single-pass sizes (P <= 4096): the whole chain for one pair in one
-// workgroup; writes the product X_p Z_p.
-__global__ void __launch_bounds__(NT) k_tfft_small(const float2* __restrict__ A, int P, int log2P,
+// workgroup; writes the product X_p Z_p, X_p the spectrum of A_p or, with B
+// (the specular method's outward trace), of B_p.  pbase null: whole rows.
+__global__ void __launch_bounds__(NT) k_tfft_small(const float2* __restrict__ A,
+                                                   const float2* __restrict__ B, int P, int log2P,
                                                    const int* __restrict__ pbase,
                                                    const int* __restrict__ pwin, int nr,
                                                    const float2* __restrict__ G,
@@ -492,7 +504,7 @@ __global__ void __launch_bounds__(NT) k_tfft_small(const float2* __restrict__ A,
                                                    const float2* __restrict__ tw) {
     __shared__ float2 s[NPTS];
     const int p = blockIdx.x;
-    const int base = pbase[p], win = pwin[p];
+    const int base = pbase ? pbase[p] : -1, win = pbase ? pwin[p] : 0;
     const float2* a = A + (size_t)p * P;
     for (int n = threadIdx.x; n < P; n += NT) {
         const bool live = (n < nr) && (base < 0 || (n >= base && n < base + win));
@@ -525,10 +537,354 @@ __global__ void __launch_bounds__(NT) k_tfft_small(const float2* __restrict__ A,
     }
     __syncthreads();
     lds_fft(s, P, log2P, 1, false, tw);
+    if (B) {
+        // hold Z, transform the outward trace
+        const float2* b = B + (size_t)p * P;
+#pragma unroll
+        for (int q = 0; q < PPT; ++q) {
+            const int n = threadIdx.x + q * NT;
+            if (n < P) xr[q] = s[sw(n)];
+        }
+        __syncthreads();
+        for (int n = threadIdx.x; n < P; n += NT)
+            s[sw(n)] = n < nr ? b[n] : make_float2(0.f, 0.f);
+        __syncthreads();
+        lds_fft(s, P, log2P, 1, false, tw);
+    }
 #pragma unroll
     for (int q = 0; q < PPT; ++q) {
         const int n = threadIdx.x + q * NT;
         if (n < P) prod[(size_t)p * P + n] = cmul(xr[q], s[sw(n)]);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Per-shot stages: the surface echo's range compression and the band crop of
+// the summed target spectra.  A batch has few rows (its shots), so these are
+// bound by launches and by the latency of one workgroup's transform, not by
+// bytes: sizes that fit one workgroup run in one launch, two-pass sizes in
+// three and five, each transform reading its input and writing its result
+// where the next step wants it.
+// Replaces seven launches of the range compression and fifteen of a Bluestein
+// DFT_L, crop and IDFT_L: one shot of 700 bins 464 -> 373 us per call, 24
+// shots of 1500 bins (specular) 866 -> 660 us, six short tracks 9.93 -> 9.02
+// ms.
+// ---------------------------------------------------------------------------
+// bin n of a surface row: FP64, or fixed point times inv
+__device__ __forceinline__ float2 surf_bin(const double2* __restrict__ row, int n, int det,
+                                           double inv) {
+    const double2 v = row[n];
+    if (det)
+        return make_float2((float)det_unfix(__double_as_longlong(v.x), inv),
+                           (float)det_unfix(__double_as_longlong(v.y), inv));
+    return make_float2((float)v.x, (float)v.y);
+}
+__device__ __forceinline__ double surf_inv(int det, const unsigned* __restrict__ smax,
+                                           const int* __restrict__ Vs, int s) {
+    if (!det) return 0.0;
+    const double sc = det_scale((double)Vs[s], (double)__uint_as_float(smax[s]));
+    return sc > 0.0 ? 1.0 / sc : 0.0;
+}
+
+// P <= 4096: one workgroup per row
+__global__ void __launch_bounds__(NT) k_conv_small(float2* __restrict__ out,
+                                                   const double2* __restrict__ srow, int nr,
+                                                   int det, const unsigned* __restrict__ smax,
+                                                   const int* __restrict__ Vs, int P, int log2P,
+                                                   const float2* __restrict__ G,
+                                                   const TrackK* __restrict__ trk,
+                                                   const RowK* __restrict__ rk,
+                                                   const float2* __restrict__ tw) {
+    __shared__ float2 s[NPTS];
+    const int r = blockIdx.x;
+    if (trk) {
+        if (rk[r].shot < 0) return;
+        G = trk[rk[r].trk].g_surf;
+        if (!G) {
+            for (int n = threadIdx.x; n < nr; n += NT)
+                out[(size_t)r * nr + n] = make_float2(0.f, 0.f);
+            return;
+        }
+    }
+    const double inv = surf_inv(det, smax, Vs, r);
+    const double2* row = srow + (size_t)r * nr;
+    for (int n = threadIdx.x; n < P; n += NT)
+        s[sw(n)] = n < nr ? surf_bin(row, n, det, inv) : make_float2(0.f, 0.f);
+    __syncthreads();
+    lds_fft(s, P, log2P, 1, false, tw);
+    for (int n = threadIdx.x; n < P; n += NT) s[sw(n)] = cmul(s[sw(n)], G[n]);
+    __syncthreads();
+    lds_fft(s, P, log2P, 1, true, tw);
+    for (int n = threadIdx.x; n < nr; n += NT) out[(size_t)r * nr + n] = s[sw(n + nr)];
+}
+
+// two-pass, first column pass from the surface bins
+__global__ void __launch_bounds__(NT) k_conv_cols_in(float2* __restrict__ data,
+                                                     const double2* __restrict__ srow, int nr,
+                                                     int det, const unsigned* __restrict__ smax,
+                                                     const int* __restrict__ Vs, int N1, int N2,
+                                                     int log2N2, const float2* __restrict__ tw,
+                                                     const float2* __restrict__ it) {
+    __shared__ float2 s[NPTS];
+    __shared__ float2 twl[TWL];
+    const int CT = NPTS / N2, c0 = blockIdx.x * CT, rw = blockIdx.y;
+    float2* g = data + (size_t)rw * N1 * N2;
+    const double2* row = srow + (size_t)rw * nr;
+    const float2* tws = stage_ladder(twl, tw, N2);
+    const double inv = surf_inv(det, smax, Vs, rw);
+    for (int idx = threadIdx.x; idx < NPTS; idx += NT) {
+        const int r = idx / CT, c = idx - r * CT;
+        const int n = r * N1 + c0 + c;
+        s[sw(c * N2 + r)] = n < nr ? surf_bin(row, n, det, inv) : make_float2(0.f, 0.f);
+    }
+    __syncthreads();
+    lds_fft(s, N2, log2N2, CT, false, tws);
+    for (int idx = threadIdx.x; idx < NPTS; idx += NT) {
+        const int r = idx / CT, c = idx - r * CT;
+        g[(size_t)r * N1 + c0 + c] = cmul(s[sw(c * N2 + r)], it[(size_t)r * N1 + c0 + c]);
+    }
+}
+
+// two-pass, last column pass (inverse): keeps [nr, 2 nr)
+__global__ void __launch_bounds__(NT) k_conv_cols_out(float2* __restrict__ out, int nr,
+                                                      const float2* __restrict__ data, int N1,
+                                                      int N2, int log2N2,
+                                                      const float2* __restrict__ tw) {
+    __shared__ float2 s[NPTS];
+    __shared__ float2 twl[TWL];
+    const int CT = NPTS / N2, c0 = blockIdx.x * CT, rw = blockIdx.y;
+    const float2* tws = stage_ladder(twl, tw, N2);
+    load_cols(s, data + (size_t)rw * N1 * N2, N1, N2, c0);
+    __syncthreads();
+    lds_fft(s, N2, log2N2, CT, true, tws);
+    for (int idx = threadIdx.x; idx < NPTS; idx += NT) {
+        const int r = idx / CT, c = idx - r * CT;
+        const int j = r * N1 + c0 + c - nr;
+        if (j >= 0 && j < nr) out[(size_t)rw * nr + j] = s[sw(c * N2 + r)];
+    }
+}
+
+// band kernels D[2 d] and D[2 d - 1] at e = P / 2 + d, |d| < nr (BandTables);
+// 2 K + 1 frequencies are kept: D[t] = sin(pi (2K+1) t / L) / (L sin(pi t / L))
+__global__ void k_band_gen(float2* __restrict__ tab, int P, int nr, int K) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= 2 * P) return;
+    const int odd = i >= P, d = (i - odd * P) - P / 2;
+    const long long L = 2 * (long long)nr - 1, t = 2 * (long long)d - odd;
+    float v = 0.f;
+    if (d > -nr && d < nr && K >= 0) {
+        if (t % L == 0) {
+            v = (float)((double)(2 * K + 1) / (double)L);
+        } else {
+            const double a = sinpi((double)(((2LL * K + 1) * t) % (2 * L)) / (double)L);
+            const double b = sinpi((double)(t % (2 * L)) / (double)L);
+            v = (float)(a / ((double)L * b));
+        }
+    }
+    tab[i] = make_float2(v, 0.f);
+}
+__global__ void k_band_scale(float2* __restrict__ tab, int n, float sc) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) tab[i] = make_float2(tab[i].x * sc, tab[i].y * sc);
+}
+
+// Where a row's samples go (the combine step of combineRadarSignals,
+// radar_kernels.cu:302-311): a run's output, or its track's radargram
+struct FinalOut {
+    const float2* refl;
+    const float2* add;
+    const int* Vs;
+    float2* out;
+    int32_t* nvalid;
+    const TrackK* trk;
+    const RowK* rk;
+};
+// false: a padding row of a multi-track batch
+__device__ __forceinline__ bool final_row(const FinalOut& fo, int r, int nr, float2** o,
+                                          const float2** tab) {
+    if (fo.trk) {
+        const RowK row = fo.rk[r];
+        if (row.shot < 0) return false;
+        const TrackK& t = fo.trk[row.trk];
+        *o = t.out + (size_t)row.shot * nr;
+        *tab = t.band;
+        if (t.nvalid && blockIdx.x == 0 && threadIdx.x == 0) t.nvalid[row.shot] = fo.Vs[r];
+    } else {
+        *o = fo.out + (size_t)r * nr;
+        if (fo.nvalid && blockIdx.x == 0 && threadIdx.x == 0) fo.nvalid[r] = fo.Vs[r];
+    }
+    return true;
+}
+__device__ __forceinline__ float2 final_value(const FinalOut& fo, size_t i, bool live, float2 v) {
+    if (!live) return make_float2(0.f, 0.f);
+    if (fo.refl) v = cadd(fo.refl[i], v);
+    if (fo.add) v = cadd(v, fo.add[i]);
+    return v;
+}
+
+// P <= 4096: the whole stage of one row in one workgroup
+__global__ void __launch_bounds__(NT) k_final_small(const float2* __restrict__ S, int P, int log2P,
+                                                    int nr, const float2* tab, FinalOut fo,
+                                                    const float2* __restrict__ tw) {
+    __shared__ float2 s[NPTS];
+    const int r = blockIdx.y;
+    float2* o;
+    if (!final_row(fo, r, nr, &o, &tab)) return;
+    const float2* x = S + (size_t)r * P;
+    for (int n = threadIdx.x; n < P; n += NT) s[sw(n)] = x[n];
+    __syncthreads();
+    lds_fft(s, P, log2P, 1, true, tw);
+    // even and odd samples of c (2 nr - 1 of them), P / 2 each
+    constexpr int H = PPT / 2;
+    float2 ce[H], co[H], acc[PPT];
+#pragma unroll
+    for (int q = 0; q < H; ++q) {
+        const int l = threadIdx.x + q * NT;
+        ce[q] = l < nr ? s[sw(2 * l)] : make_float2(0.f, 0.f);
+        co[q] = l < nr - 1 ? s[sw(2 * l + 1)] : make_float2(0.f, 0.f);
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < H; ++q) {
+            const int l = threadIdx.x + q * NT;
+            if (l < P / 2) {
+                s[sw(l)] = h ? co[q] : ce[q];
+                s[sw(l + P / 2)] = make_float2(0.f, 0.f);
+            }
+        }
+        __syncthreads();
+        lds_fft(s, P, log2P, 1, false, tw);
+#pragma unroll
+        for (int q = 0; q < PPT; ++q) {
+            const int n = threadIdx.x + q * NT;
+            if (n < P) {
+                const float2 v = cmul(s[sw(n)], tab[(size_t)h * P + n]);
+                acc[q] = h ? cadd(acc[q], v) : v;
+            }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < PPT; ++q) {
+        const int n = threadIdx.x + q * NT;
+        if (n < P) s[sw(n)] = acc[q];
+    }
+    __syncthreads();
+    lds_fft(s, P, log2P, 1, true, tw);
+    const bool live = fo.Vs[r] > 0;
+    for (int n = threadIdx.x; n < nr; n += NT)
+        o[n] = final_value(fo, (size_t)r * nr + n, live, s[sw(P / 2 + n)]);
+}
+
+// two-pass: column IFFT of S, c's even samples to eo[0, P / 2), odd to [P / 2, P)
+__global__ void __launch_bounds__(NT) k_final_split(float2* __restrict__ eo,
+                                                    const float2* __restrict__ S, int nr, int N1,
+                                                    int N2, int log2N2,
+                                                    const float2* __restrict__ tw) {
+    __shared__ float2 s[NPTS];
+    __shared__ float2 twl[TWL];
+    const int CT = NPTS / N2, c0 = blockIdx.x * CT;
+    const size_t off = (size_t)blockIdx.y * N1 * N2;
+    const float2* tws = stage_ladder(twl, tw, N2);
+    load_cols(s, S + off, N1, N2, c0);
+    __syncthreads();
+    lds_fft(s, N2, log2N2, CT, true, tws);
+    for (int idx = threadIdx.x; idx < NPTS; idx += NT) {
+        const int r = idx / CT, c = idx - r * CT;
+        const int n = r * N1 + c0 + c;
+        if (n < 2 * nr - 1)
+            eo[off + (size_t)(n & 1) * (N1 * N2 / 2) + (n >> 1)] = s[sw(c * N2 + r)];
+    }
+}
+// column FFT of the even (blockIdx.y even) and odd samples of a row
+__global__ void __launch_bounds__(NT) k_final_cols(float2* __restrict__ ev, float2* __restrict__ od,
+                                                   const float2* __restrict__ eo, int nr, int N1,
+                                                   int N2, int log2N2,
+                                                   const float2* __restrict__ tw,
+                                                   const float2* __restrict__ it) {
+    __shared__ float2 s[NPTS];
+    __shared__ float2 twl[TWL];
+    const int CT = NPTS / N2, c0 = blockIdx.x * CT, h = blockIdx.y & 1;
+    const size_t P = (size_t)N1 * N2, off = (size_t)(blockIdx.y >> 1) * P;
+    const float2* x = eo + off + h * (P / 2);
+    float2* g = (h ? od : ev) + off;
+    const float2* tws = stage_ladder(twl, tw, N2);
+    for (int idx = threadIdx.x; idx < NPTS; idx += NT) {
+        const int r = idx / CT, c = idx - r * CT;
+        const int n = r * N1 + c0 + c;
+        s[sw(c * N2 + r)] = n < nr - h ? x[n] : make_float2(0.f, 0.f);
+    }
+    __syncthreads();
+    lds_fft(s, N2, log2N2, CT, false, tws);
+    for (int idx = threadIdx.x; idx < NPTS; idx += NT) {
+        const int r = idx / CT, c = idx - r * CT;
+        g[(size_t)r * N1 + c0 + c] = cmul(s[sw(c * N2 + r)], it[(size_t)r * N1 + c0 + c]);
+    }
+}
+// row FFTs of both, times the band kernels, summed, row IFFT (+ conj twiddle)
+// into ev
+__global__ void __launch_bounds__(NT) k_final_rows(float2* __restrict__ ev,
+                                                   const float2* __restrict__ od, int N1,
+                                                   int log2N1, int N2,
+                                                   const float2* __restrict__ tab, FinalOut fo,
+                                                   const float2* __restrict__ tw,
+                                                   const float2* __restrict__ it) {
+    __shared__ float2 s[NPTS];
+    __shared__ float2 twl[TWL];
+    if (fo.trk) {
+        const RowK row = fo.rk[blockIdx.y];
+        if (row.shot < 0) return;
+        tab = fo.trk[row.trk].band;
+    }
+    const int RT = NPTS / N1, r0 = blockIdx.x * RT;
+    const size_t P = (size_t)N1 * N2, off = (size_t)blockIdx.y * P + (size_t)r0 * N1;
+    const float2* tws = stage_ladder(twl, tw, N1);
+    float2 acc[PPT];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const float2* x = (h ? od : ev) + off;
+        for (int i = threadIdx.x; i < NPTS; i += NT) s[sw(i)] = x[i];
+        __syncthreads();
+        lds_fft(s, N1, log2N1, RT, false, tws);
+        const float2* t = tab + h * P + (size_t)r0 * N1;
+#pragma unroll
+        for (int q = 0; q < PPT; ++q) {
+            const int i = threadIdx.x + q * NT;
+            const float2 v = cmul(s[sw(i)], t[i]);
+            acc[q] = h ? cadd(acc[q], v) : v;
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int q = 0; q < PPT; ++q) s[sw(threadIdx.x + q * NT)] = acc[q];
+    __syncthreads();
+    lds_fft(s, N1, log2N1, RT, true, tws);
+    for (int i = threadIdx.x; i < NPTS; i += NT)
+        ev[off + i] = cmul(s[sw(i)], conjf2(it[(size_t)r0 * N1 + i]));
+}
+// last column IFFT; output i at P / 2 + i
+__global__ void __launch_bounds__(NT) k_final_out(const float2* __restrict__ ev, int nr, int N1,
+                                                  int N2, int log2N2, FinalOut fo,
+                                                  const float2* __restrict__ tw) {
+    __shared__ float2 s[NPTS];
+    __shared__ float2 twl[TWL];
+    const int CT = NPTS / N2, c0 = blockIdx.x * CT, rw = blockIdx.y;
+    float2* o;
+    const float2* unused;
+    if (!final_row(fo, rw, nr, &o, &unused)) return;
+    const float2* tws = stage_ladder(twl, tw, N2);
+    load_cols(s, ev + (size_t)rw * N1 * N2, N1, N2, c0);
+    __syncthreads();
+    lds_fft(s, N2, log2N2, CT, true, tws);
+    const bool live = fo.Vs[rw] > 0;
+    const int half = N1 * N2 / 2;
+    for (int idx = threadIdx.x; idx < NPTS; idx += NT) {
+        const int r = idx / CT, c = idx - r * CT;
+        const int j = r * N1 + c0 + c - half;
+        if (j >= 0 && j < nr)
+            o[j] = final_value(fo, (size_t)rw * nr + j, live, s[sw(c * N2 + r)]);
     }
 }
 
@@ -1205,14 +1561,15 @@ FftPlan fft_plan(int N) {
 static const float2* inter_table(erp_ctx* ctx, const FftPlan& p, hipStream_t s);
 
 // The ladder table and the inter-pass tables of every two-pass size a run
-// can use (up to the 2^17-point Bluestein transforms of nr = 32767): built
-// once per context, so that no run allocates a table (1.9 MB in all).
+// can use (up to the 2^16-point transforms of nr = 32767): built once per
+// context, so that no run allocates a table (0.9 MB in all; a terrain's
+// larger transforms add theirs on first use).
 void fft_init_twiddles(erp_ctx* ctx) {
     ctx->twiddle.ensure(sizeof(float2) * (size_t)LADN);
     hipLaunchKernelGGL(k_twiddle_init, dim3(LADN / 256), dim3(256), 0, ctx->stream,
                        ctx->twiddle.as<float2>());
     ERP_CHECK_LAUNCH("k_twiddle_init");
-    for (int n = 2 * NPTS; n <= (1 << 17); n *= 2) inter_table(ctx, fft_plan(n), ctx->stream);
+    for (int n = 2 * NPTS; n <= (1 << 16); n *= 2) inter_table(ctx, fft_plan(n), ctx->stream);
 }
 
 // inter-pass twiddle table of a two-pass plan (cached per size in the context)
@@ -1280,8 +1637,8 @@ void target_spectra_fused(erp_ctx* ctx, const FftPlan& p, float2* A, float2* Y,
     const float2* tw = ctx->twiddle.as<float2>();
     const int P = p.N;
     if (!p.two_pass) {
-        hipLaunchKernelGGL(k_tfft_small, dim3(n), dim3(NT), 0, st, A, P, p.log2N, pbase, pwin, nr,
-                           G, work, tw);
+        hipLaunchKernelGGL(k_tfft_small, dim3(n), dim3(NT), 0, st, A,
+                           (const float2*)nullptr, P, p.log2N, pbase, pwin, nr, G, work, tw);
         ERP_CHECK_LAUNCH("k_tfft_small");
         // groups are unused here: sum the per-pair products per shot segment
         hipLaunchKernelGGL(k_sum_rows, dim3(std::max(1, P / 256), nseg), dim3(256), 0, st, S,
@@ -1297,7 +1654,7 @@ void target_spectra_fused(erp_ctx* ctx, const FftPlan& p, float2* A, float2* Y,
                        pbase, pwin, nr, tw, it);
     ERP_CHECK_LAUNCH("k_tfft_cols_fwd");
     hipLaunchKernelGGL(k_tfft_rows_conv, dim3(p.N2 / RT, n), dim3(NT), 0, st, A, Y, p.N1, l1,
-                       p.N2, G, tw, it);
+                       p.N2, G, tw, it, (const TrackK*)nullptr, (const RowK*)nullptr);
     ERP_CHECK_LAUNCH("k_tfft_rows_conv");
     hipLaunchKernelGGL(k_tfft_cols_shift, dim3(p.N1 / CT, n), dim3(NT), 0, st, Y, p.N1, p.N2, l2,
                        nr / p.N1, tw, it);
@@ -1308,6 +1665,100 @@ void target_spectra_fused(erp_ctx* ctx, const FftPlan& p, float2* A, float2* Y,
     hipLaunchKernelGGL(k_sum_rows, dim3(std::max(1, P / 256), nseg), dim3(256), 0, st, S, work,
                        gseg_shot, gseg_beg, gseg_end, P, scale, 0, 0);
     ERP_CHECK_LAUNCH("k_sum_rows");
+}
+
+void target_spectra_small(erp_ctx* ctx, const FftPlan& p, const float2* A, const float2* B, int nr,
+                          int n, const float2* G, float2* prod, const int* seg_shot,
+                          const int* seg_beg, const int* seg_end, int nseg, float2* S,
+                          hipStream_t st) {
+    if (p.two_pass) throw ErpError{ERP_E_INVALID, "target_spectra_small needs a single-pass size"};
+    hipLaunchKernelGGL(k_tfft_small, dim3(n), dim3(NT), 0, st, A, B, p.N, p.log2N,
+                       (const int*)nullptr, (const int*)nullptr, nr, G, prod,
+                       ctx->twiddle.as<float2>());
+    ERP_CHECK_LAUNCH("k_tfft_small");
+    hipLaunchKernelGGL(k_sum_rows, dim3(std::max(1, p.N / 256), nseg), dim3(256), 0, st, S, prod,
+                       seg_shot, seg_beg, seg_end, p.N, 1.0f, 0, 0);
+    ERP_CHECK_LAUNCH("k_sum_rows");
+}
+
+void surface_conv_rows(erp_ctx* ctx, const FftPlan& p, const double2* srow, int nr, int rows,
+                       bool det, const unsigned* smax, const int* Vs, const float2* G,
+                       float2* work, float2* out, const TrackK* trk, const RowK* rk,
+                       hipStream_t st) {
+    if (rows <= 0) return;
+    const float2* tw = ctx->twiddle.as<float2>();
+    const int d = det ? 1 : 0;
+    if (!p.two_pass) {
+        hipLaunchKernelGGL(k_conv_small, dim3(rows), dim3(NT), 0, st, out, srow, nr, d, smax, Vs,
+                           p.N, p.log2N, G, trk, rk, tw);
+        ERP_CHECK_LAUNCH("k_conv_small");
+        return;
+    }
+    const int CT = NPTS / p.N2, RT = NPTS / p.N1;
+    const float2* it = inter_table(ctx, p, st);
+    hipLaunchKernelGGL(k_conv_cols_in, dim3(p.N1 / CT, rows), dim3(NT), 0, st, work, srow, nr, d,
+                       smax, Vs, p.N1, p.N2, ilog2(p.N2), tw, it);
+    ERP_CHECK_LAUNCH("k_conv_cols_in");
+    hipLaunchKernelGGL(k_tfft_rows_conv, dim3(p.N2 / RT, rows), dim3(NT), 0, st, work, work, p.N1,
+                       ilog2(p.N1), p.N2, G, tw, it, trk, rk);
+    ERP_CHECK_LAUNCH("k_tfft_rows_conv");
+    hipLaunchKernelGGL(k_conv_cols_out, dim3(p.N1 / CT, rows), dim3(NT), 0, st, out, nr, work,
+                       p.N1, p.N2, ilog2(p.N2), tw);
+    ERP_CHECK_LAUNCH("k_conv_cols_out");
+}
+
+void build_band(erp_ctx* ctx, const FftPlan& p, float2* tab, int nr, float smpl, float B,
+                hipStream_t st) {
+    // the largest kept frequency index of cropSpectrum (elementary_kernels.cu:
+    // 258-278): freq = k smpl / L, kept unless |freq| > B
+    const int L = 2 * nr - 1, kmax = L / 2;
+    auto kept = [&](int k) {
+        return !(std::fabs(((double)k * (double)smpl) / (double)L) > (double)B);
+    };
+    const double g = std::floor((double)B * L / (double)smpl);
+    int K = g >= kmax ? kmax : g >= 0.0 ? (int)g : 0;  // (a NaN starts at 0)
+    while (K < kmax && kept(K + 1)) ++K;
+    while (K >= 0 && !kept(K)) --K;
+    const int n = 2 * p.N;
+    hipLaunchKernelGGL(k_band_gen, dim3((n + 255) / 256), dim3(256), 0, st, tab, p.N, nr, K);
+    ERP_CHECK_LAUNCH("k_band_gen");
+    fft_forward(ctx, p, tab, 2, st);
+    hipLaunchKernelGGL(k_band_scale, dim3((n + 255) / 256), dim3(256), 0, st, tab, n,
+                       1.0f / (float)p.N / (float)p.N);
+    ERP_CHECK_LAUNCH("k_band_scale");
+}
+
+void shot_final_rows(erp_ctx* ctx, const FftPlan& p, float2* S, float2* work, int nr, int rows,
+                     const float2* tab, const float2* refl, const float2* add, const int* Vs,
+                     float2* out, int32_t* nvalid, const TrackK* trk, const RowK* rk,
+                     hipStream_t st) {
+    if (rows <= 0) return;
+    const float2* tw = ctx->twiddle.as<float2>();
+    const FinalOut fo{refl, add, Vs, out, nvalid, trk, rk};
+    if (!p.two_pass) {
+        hipLaunchKernelGGL(k_final_small, dim3(1, rows), dim3(NT), 0, st, S, p.N, p.log2N, nr, tab,
+                           fo, tw);
+        ERP_CHECK_LAUNCH("k_final_small");
+        return;
+    }
+    const int CT = NPTS / p.N2, RT = NPTS / p.N1, l1 = ilog2(p.N1), l2 = ilog2(p.N2);
+    const float2* it = inter_table(ctx, p, st);
+    float2* od = work + (size_t)rows * p.N;
+    hipLaunchKernelGGL(k_fft_rows, dim3(p.N2 / RT, rows), dim3(NT), 0, st, S, p.N1, l1, p.N2, 1,
+                       tw, it);
+    ERP_CHECK_LAUNCH("k_fft_rows");
+    hipLaunchKernelGGL(k_final_split, dim3(p.N1 / CT, rows), dim3(NT), 0, st, work, S, nr, p.N1,
+                       p.N2, l2, tw);
+    ERP_CHECK_LAUNCH("k_final_split");
+    hipLaunchKernelGGL(k_final_cols, dim3(p.N1 / CT, 2 * rows), dim3(NT), 0, st, S, od, work, nr,
+                       p.N1, p.N2, l2, tw, it);
+    ERP_CHECK_LAUNCH("k_final_cols");
+    hipLaunchKernelGGL(k_final_rows, dim3(p.N2 / RT, rows), dim3(NT), 0, st, S, od, p.N1, l1, p.N2,
+                       tab, fo, tw, it);
+    ERP_CHECK_LAUNCH("k_final_rows");
+    hipLaunchKernelGGL(k_final_out, dim3(p.N1 / CT, rows), dim3(NT), 0, st, S, nr, p.N1, p.N2, l2,
+                       fo, tw);
+    ERP_CHECK_LAUNCH("k_final_out");
 }
 
 int target_half_slice() { return SLICE; }

@@ -155,7 +155,7 @@ struct FftPlan {
     bool two_pass = false;
 };
 
-// Per-(nr, dr, res) chirp spectra and per-L Bluestein tables
+// Per-(nr, dr, res) chirp spectra
 struct ChirpKey {
     int nr;
     float dr, res;
@@ -173,12 +173,20 @@ struct ChirpSpec {
     DevBuf wl;    // the natural one in the layout of k_tpair_wl (first use)
 };
 
-struct BlueTables {
-    int L = 0, M = 0;
+// Band crop and decimation of a shot's summed spectrum (convolveComplex's
+// cropSpectrum + takeEveryOtherComplex, elementary_kernels.cu:187-194,
+// 258-353).  DFT_L, crop to |freq| <= B, IDFT_L and keeping every second
+// sample of the L = 2 nr - 1 samples c is a convolution with the band's real
+// L-periodic kernel D:
+//     out[i] = sum_j c[j] D[2 i - j],   i < nr,
+// i.e. (j even and odd apart) two linear convolutions of nr points with
+// D[2 d] and D[2 d - 1], which fit the P >= 2 nr - 1 point transforms.
+// tab: the spectra of those two kernels (output i at P / 2 + i), P complex64
+// each in fft_forward's order, scaled by 1 / P^2 (the two inverses).
+struct BandTables {
+    int nr = 0, P = 0;
     float smpl = 0, B = 0;
-    DevBuf w;     // L complex64: exp(-i pi n^2 / L)
-    DevBuf Bw;    // M complex64: FFT_M of the conjugate chirp, scaled 1/M
-    DevBuf mask;  // L uint8: crop mask (1 = keep)
+    DevBuf tab;
 };
 
 struct WorkBufs {
@@ -189,7 +197,7 @@ struct WorkBufs {
     DevBuf srow;       // S x nr FP64 / fixed-point surface bins + S per-shot maxima
     DevBuf refl;       // S x nr complex
     DevBuf shotS;      // S x P complex: per-shot spectral accumulator
-    DevBuf blu;        // S x M complex: Bluestein workspace
+    DevBuf blu;        // S x 2P complex: workspace of the band crop
     DevBuf tA, tB, tC; // per-target chunk buffers, C x P complex
     DevBuf pairs;      // chunk pair list
     DevBuf t0trace;    // S x P complex: summed type-0 target histograms
@@ -239,11 +247,11 @@ struct erp_ctx {
     DevBuf twiddle;  // ladder table of the LDS FFT stages (65536 complex64)
     std::vector<std::pair<int, DevBuf*>> inter;  // inter-pass twiddles per size
     std::vector<ChirpSpec*> chirps;
-    std::vector<BlueTables*> blues;
+    std::vector<BandTables*> bands;
     WorkBufs work;
     std::mutex mu;        // serialises the synchronous entry points
-    // guards inter / chirps / blues (shared by all streams); recursive because
-    // building a chirp or Bluestein table runs FFTs that look up inter tables
+    // guards inter / chirps / bands (shared by all streams); recursive because
+    // building a chirp or band table runs FFTs that look up inter tables
     std::recursive_mutex cache_mu;
     int num_cu = 0;
     // asynchronous jobs: worker slots, each with its own thread, stream and
@@ -306,6 +314,34 @@ void target_sum_half(const FftPlan& p, const float2* work, float2* partial, cons
                      const float* seg_scale = nullptr, bool seq = false, bool wl = false);
 // natural-order copy of a forward spectrum produced by fft_forward
 void fft_natural_order(const FftPlan& p, const float2* src, float2* dst, hipStream_t st);
+// Surface range compression of `rows` rows: FP64 bins srow (nr per row; det:
+// fixed point, scaled by its row's V and smax) -> out (nr per row), by the
+// spectrum G, or each row's track's (trk, rk; a track without one gets
+// zeros).  work: rows x P, unused by single-pass sizes.
+struct TrackK;
+struct RowK;
+void surface_conv_rows(erp_ctx* ctx, const FftPlan& p, const double2* srow, int nr, int rows,
+                       bool det, const unsigned* smax, const int* Vs, const float2* G,
+                       float2* work, float2* out, const TrackK* trk, const RowK* rk,
+                       hipStream_t st);
+// spectra of the band kernels of (nr, smpl, B) into tab (2 P complex64)
+void build_band(erp_ctx* ctx, const FftPlan& p, float2* tab, int nr, float smpl, float B,
+                hipStream_t st);
+// Last stage of typed targets: each row's summed spectrum S (P, overwritten)
+// -> c = IFFT(S), cropped to the band and decimated, plus refl and add
+// (either may be null), zero where Vs is 0, into out and nvalid (or, with
+// trk, each row's place in its track's radargram).  work: rows x 2P, unused
+// by single-pass sizes.
+void shot_final_rows(erp_ctx* ctx, const FftPlan& p, float2* S, float2* work, int nr, int rows,
+                     const float2* tab, const float2* refl, const float2* add, const int* Vs,
+                     float2* out, int32_t* nvalid, const TrackK* trk, const RowK* rk,
+                     hipStream_t st);
+// Specular typed targets of single-pass sizes: prod[p] = FFT(B_p) FFT(z_p),
+// z_p the range-compressed window of A_p, summed per segment into S
+void target_spectra_small(erp_ctx* ctx, const FftPlan& p, const float2* A, const float2* B, int nr,
+                          int n, const float2* G, float2* prod, const int* seg_shot,
+                          const int* seg_beg, const int* seg_end, int nseg, float2* S,
+                          hipStream_t st);
 void target_spectra_fused(erp_ctx* ctx, const FftPlan& p, float2* A, float2* Y,
                           const int* pbase, const int* pwin, int nr, int n, const float2* G,
                           float2* work, int ngroups, const int* gbeg, const int* gend,
@@ -338,6 +374,80 @@ void mesh_from_heights(const double* heights, int64_t nx, int64_t ny, double fs,
 // ny x nx FP64 heights of a synthetic terrain into device memory h (see
 // erp_mesh_from_terrain; erp_terrain.hip); synchronous on st
 void terrain_heights(erp_ctx* ctx, const erp_terrain& t, double* h, hipStream_t st);
+
+// Kernel-side parameter block (derived once per run on the host).
+struct KPar {
+    float lam, fs, P, ks, eps1, eps2, nu1, nu2, alpha1, alpha2, rng_res, dr;
+    float c, c1, c2;
+    float piLlam;      // PI_F*fs/lam (facet_G's sinc argument scale)
+    float Dmax;        // 4*PI_F*fs^2/lam^2
+    float fs_lam;      // fs/lam (facetReradiation)
+    float fs2_lam;     // fs*fs/lam
+    float nf;          // sqrt(eps_2) in float (accumulateTarget's n)
+    int ortho;         // every facet frame (u, v, n) orthonormal (see sc_angles)
+    float sqrtP;
+    float invK;        // 1/(4*3.14159)^2
+    float sqrt_e1e2;   // sqrt(eps_1/eps_2)
+    float sqrt_e2e1;   // sqrt(eps_2/eps_1)
+    double drd, inv_dr, cos_ap, n_d, inv_cyc, lam_d;
+    // c1/c2 and c/c2 (genRefrPhasor, refrRadarSignal) divided in FP64: a
+    // float quotient is off by up to 6e-8, i.e. 5e-5 rad of phase over a
+    // 300 m refracted leg at 60 MHz
+    double c1c2, cc2;
+    // second subsurface medium below z = zi (has3 = 0: none): dn = n3 - n2,
+    // tsq = sqrt(1 - rho23^2) (amplitude factor of a crossing path),
+    // n_lo / n_hi = min / max(n2, n3) (window bounds)
+    int has3;
+    double zi, dn, n_lo, n_hi;
+    float tsq;
+    double B, smpl;
+    int nr, P_fft, rerad;
+    int row_live;      // entries of a pair row the spectral chain reads: P_fft / 2
+                       // for the per-pair LDS chain, P_fft otherwise
+    uint32_t mode;
+    uint64_t seed;
+    int win_shift;     // 0; > 0 only to test the target kernel's window check
+};
+
+// Multi-track batches (erp_run_tracks): the rows of a batch are shots of
+// several tracks of one range length; every kernel that reads a track's
+// data takes it from that track's descriptor instead of its arguments.
+struct TrackK {
+    KPar kp;
+    const float* mesh;             // 12 x Fpad SoA
+    int64_t Fpad, F;
+    int nblk, tile_nx, frame_ok;
+    const float* tg;               // 6 x Tpad targets
+    int64_t Tpad;
+    int T;
+    const unsigned char* ttype;
+    const float2* g_surf;          // surface range kernel spectrum (fft order)
+    const float2* g_targ_nat;      // target range kernel spectrum (natural order, or
+                                   // in the layout of k_tpair_wl where it runs)
+    const float2* band;            // band tables of the track (BandTables::tab)
+    float2* out;                   // the track's radargram, ns x nr (device)
+    int32_t* nvalid;               // its illuminated counts (device) or null
+    float tscale;                  // -1 / sqrt(P): outward trace of a target
+};
+struct RowK {
+    int trk;   // track of the row
+    int shot;  // the row's shot index within its track
+};
+
+// Deterministic accumulation: every term is rounded once to a signed 64-bit
+// fixed-point value v * 2^E and summed with integer atomics, which are exact
+// and so independent of the order in which threads and workgroups arrive.
+// E is chosen from a bound M >= |component| of every term and the number of
+// terms n that can reach one bin: |sum| * 2^E <= 2 n M 2^E <= 2^61.
+__device__ __forceinline__ double det_scale(double n, double M) {
+    if (!(M > 0.0)) return 0.0;
+    int e;
+    frexp(2.0 * n * M, &e);  // 2 n M < 2^e
+    return ldexp(1.0, 61 - e);
+}
+__device__ __forceinline__ double det_unfix(unsigned long long u, double inv_scale) {
+    return (double)(long long)u * inv_scale;
+}
 
 inline int next_pow2(int64_t n) {
     int p = 1;

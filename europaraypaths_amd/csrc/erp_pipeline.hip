@@ -23,8 +23,8 @@
 //                  767-892) over all illuminated facets, LDS window histogram.
 //   target spectra: FFT, x chirp(2 res), IFFT, window, FFT, and the product
 //                  with the outward trace's spectrum summed over the shot's
-//                  targets in the frequency domain; one inverse + Bluestein
-//                  DFT_L / crop / IDFT_L per shot replaces the reference's
+//                  targets in the frequency domain; one inverse and one band
+//                  convolution per shot (shot_final_rows) replace the reference's
 //                  per-target convolveComplex (elementary_kernels.cu:258-353).
 //   k_finalize     refl + refr -> output (combineRadarSignals, radar_kernels.cu:
 //                  302-311).
@@ -68,70 +68,9 @@ constexpr int NTF = 512;       // threads of k_target_accum_fast (two workgroups
 // at more than twice the rate of FP32 ones (ds_add_f32) on gfx950 and remove
 // FP32 accumulation error from the bins.
 
-// Kernel-side parameter block (derived once per run on the host).
-struct KPar {
-    float lam, fs, P, ks, eps1, eps2, nu1, nu2, alpha1, alpha2, rng_res, dr;
-    float c, c1, c2;
-    float piLlam;      // PI_F*fs/lam (facet_G's sinc argument scale)
-    float Dmax;        // 4*PI_F*fs^2/lam^2
-    float fs_lam;      // fs/lam (facetReradiation)
-    float fs2_lam;     // fs*fs/lam
-    float nf;          // sqrt(eps_2) in float (accumulateTarget's n)
-    int ortho;         // every facet frame (u, v, n) orthonormal (see sc_angles)
-    float sqrtP;
-    float invK;        // 1/(4*3.14159)^2
-    float sqrt_e1e2;   // sqrt(eps_1/eps_2)
-    float sqrt_e2e1;   // sqrt(eps_2/eps_1)
-    double drd, inv_dr, cos_ap, n_d, inv_cyc, lam_d;
-    // c1/c2 and c/c2 (genRefrPhasor, refrRadarSignal) divided in FP64: a
-    // float quotient is off by up to 6e-8, i.e. 5e-5 rad of phase over a
-    // 300 m refracted leg at 60 MHz
-    double c1c2, cc2;
-    // second subsurface medium below z = zi (has3 = 0: none): dn = n3 - n2,
-    // tsq = sqrt(1 - rho23^2) (amplitude factor of a crossing path),
-    // n_lo / n_hi = min / max(n2, n3) (window bounds)
-    int has3;
-    double zi, dn, n_lo, n_hi;
-    float tsq;
-    double B, smpl;
-    int nr, P_fft, rerad;
-    int row_live;      // entries of a pair row the spectral chain reads: P_fft / 2
-                       // for the per-pair LDS chain, P_fft otherwise
-    uint32_t mode;
-    uint64_t seed;
-    int win_shift;     // 0; > 0 only to test the target kernel's window check
-};
-
 struct ShotK {
     double sx, sy, sz;
     float snx, sny, snz, rst, grefl, grefr;
-};
-
-// Multi-track batches (erp_run_tracks): the rows of a batch are shots of
-// several tracks of one range length; every kernel that reads a track's
-// data takes it from that track's descriptor instead of its arguments.
-struct TrackK {
-    KPar kp;
-    const float* mesh;             // 12 x Fpad SoA
-    int64_t Fpad, F;
-    int nblk, tile_nx, frame_ok;
-    const float* tg;               // 6 x Tpad targets
-    int64_t Tpad;
-    int T;
-    const unsigned char* ttype;
-    const float2* g_surf;          // surface range kernel spectrum (fft order)
-    const float2* g_targ_nat;      // target range kernel spectrum (natural order, or
-                                   // in the layout of k_tpair_wl where it runs)
-    const float2* blue_w;          // Bluestein tables of the track's band
-    const float2* blue_Bw;
-    const unsigned char* blue_mask;
-    float2* out;                   // the track's radargram, ns x nr (device)
-    int32_t* nvalid;               // its illuminated counts (device) or null
-    float tscale;                  // -1 / sqrt(P): outward trace of a target
-};
-struct RowK {
-    int trk;   // track of the row
-    int shot;  // the row's shot index within its track
 };
 
 __device__ __forceinline__ ShotK load_shot(const erp_shot* __restrict__ shots, int s) {
@@ -702,17 +641,6 @@ __device__ __forceinline__ void glb_add2d(double2* row, int idx, double x, doubl
     atomicAdd(&row[idx].y, y);
 }
 
-// Deterministic accumulation: every term is rounded once to a signed 64-bit
-// fixed-point value v * 2^E and summed with integer atomics, which are exact
-// and so independent of the order in which threads and workgroups arrive.
-// E is chosen from a bound M >= |component| of every term and the number of
-// terms n that can reach one bin: |sum| * 2^E <= 2 n M 2^E <= 2^61.
-__device__ __forceinline__ double det_scale(double n, double M) {
-    if (!(M > 0.0)) return 0.0;
-    int e;
-    frexp(2.0 * n * M, &e);  // 2 n M < 2^e
-    return ldexp(1.0, 61 - e);
-}
 __device__ __forceinline__ unsigned long long det_fix(float v, double scale) {
     return (unsigned long long)__double2ll_rn((double)v * scale);
 }
@@ -806,9 +734,6 @@ __device__ __forceinline__ void glb_add2_fix(unsigned long long* row, int idx, f
                                              double scale) {
     atomicAdd(&row[2 * idx], det_fix(v.x, scale));
     atomicAdd(&row[2 * idx + 1], det_fix(v.y, scale));
-}
-__device__ __forceinline__ double det_unfix(unsigned long long u, double inv_scale) {
-    return (double)(long long)u * inv_scale;
 }
 
 // Scale of a shot's fixed-point type-0 row: V facets times n0 type-0
@@ -1439,9 +1364,8 @@ __global__ void k_fix_rows(float2* __restrict__ dst, const unsigned long long* _
     }
 }
 
-// surface rows (FP64 or fixed point, stride nr) -> FP32 rows of the FFT
-// buffer (stride P); bins nr..P-1 are left as they are (zero)
-__global__ void k_surf_rows(float2* __restrict__ psurf, int P, const double2* __restrict__ srow,
+// surface rows (FP64 or fixed point) -> FP32 rows (ERP_RUN_RAW_SURFACE)
+__global__ void k_surf_rows(float2* __restrict__ out, const double2* __restrict__ srow,
                             int nr, int S, int det, const unsigned* __restrict__ smax,
                             const int* __restrict__ Vs) {
     const int s = blockIdx.y;
@@ -1461,7 +1385,7 @@ __global__ void k_surf_rows(float2* __restrict__ psurf, int P, const double2* __
         } else {
             o = make_float2((float)v.x, (float)v.y);
         }
-        psurf[(size_t)s * P + b] = o;
+        out[(size_t)s * nr + b] = o;
     }
 }
 
@@ -1494,17 +1418,6 @@ __global__ void k_window(float2* __restrict__ out, int ostride, const float2* __
             v.y *= scale;
         }
         out[(size_t)r * ostride + j] = v;
-    }
-}
-
-// out[r][j] = in[r][j], j < ncols
-__global__ void k_copy_rows(float2* __restrict__ out, int ostride, const float2* __restrict__ in,
-                            int istride, int ncols, int rows) {
-    const size_t n = (size_t)ncols * rows;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (size_t)gridDim.x * blockDim.x) {
-        const int r = (int)(i / ncols), j = (int)(i - (size_t)r * ncols);
-        out[(size_t)r * ostride + j] = in[(size_t)r * istride + j];
     }
 }
 
@@ -1555,36 +1468,6 @@ __global__ void k_scale(float2* __restrict__ p, int n, float s) {
     if (i < n) {
         p[i].x *= s;
         p[i].y *= s;
-    }
-}
-
-// Bluestein tables for DFT_L: w[n] = exp(-i pi n^2 / L); b[m] = conj(w[|m|])
-// circularly in M; crop mask of cropSpectrum (elementary_kernels.cu:258-278).
-__global__ void k_blue_tables(float2* __restrict__ w, float2* __restrict__ b,
-                              unsigned char* __restrict__ mask, int L, int M, double smpl,
-                              double Bw) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < L) {
-        const long long q = ((long long)i * i) % (2LL * L);
-        double sn, cs;
-        sincospi(-(double)q / (double)L, &sn, &cs);
-        w[i] = make_float2((float)cs, (float)sn);
-        const double freq = (i <= L / 2) ? ((double)i * smpl) / (double)L
-                                         : ((double)(i - L) * smpl) / (double)L;
-        mask[i] = (fabs(freq) > Bw) ? 0 : 1;
-    }
-    if (i < M) {
-        int m = -1;
-        if (i < L) m = i;
-        else if (i > M - L) m = M - i;
-        float2 v = make_float2(0.f, 0.f);
-        if (m >= 0) {
-            const long long q = ((long long)m * m) % (2LL * L);
-            double sn, cs;
-            sincospi((double)q / (double)L, &sn, &cs);
-            v = make_float2((float)cs, (float)sn);
-        }
-        b[i] = v;
     }
 }
 
@@ -3106,61 +2989,11 @@ __global__ void k_accum_spectra(float2* __restrict__ S, const float2* __restrict
     }
 }
 
-// Bluestein step 1: a[n] = c[n] * cscale * w[n] (n < L), 0 for L <= n < M
-__global__ void k_blue_in(float2* __restrict__ a, int M, const float2* __restrict__ c, int P,
-                          const float2* __restrict__ w, int L, float cscale, int rows) {
-    const size_t n = (size_t)M * rows;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (size_t)gridDim.x * blockDim.x) {
-        const int r = (int)(i / M), k = (int)(i - (size_t)r * M);
-        float2 v = make_float2(0.f, 0.f);
-        if (k < L) {
-            float2 x = c[(size_t)r * P + k];
-            x.x *= cscale;
-            x.y *= cscale;
-            v = cmul(x, w[k]);
-        }
-        a[i] = v;
-    }
-}
-
-// Bluestein step 2 (between DFT_L and IDFT_L): a[n] = mask[n] conj(conv[n])
-__global__ void k_blue_mid(float2* __restrict__ a, int M, const unsigned char* __restrict__ mask,
-                           int L, int rows) {
-    const size_t n = (size_t)M * rows;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (size_t)gridDim.x * blockDim.x) {
-        const int k = (int)(i % M);
-        float2 v = make_float2(0.f, 0.f);
-        if (k < L && mask[k]) {
-            v = a[i];
-            v.y = -v.y;
-        }
-        a[i] = v;
-    }
-}
-
-// Bluestein output + decimation: refr[i] = conj(w[2i] conv2[2i]) / L
-__global__ void k_blue_out(float2* __restrict__ refr, int nr, const float2* __restrict__ a,
-                           int M, const float2* __restrict__ w, float invL, int rows,
-                           const int* __restrict__ live) {
-    const size_t n = (size_t)nr * rows;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (size_t)gridDim.x * blockDim.x) {
-        const int r = (int)(i / nr), j = (int)(i - (size_t)r * nr);
-        float2 v = make_float2(0.f, 0.f);
-        if (live[r]) {
-            v = cmul(w[2 * j], a[(size_t)r * M + 2 * j]);
-            v = make_float2(v.x * invL, -v.y * invL);
-        }
-        refr[i] = v;
-    }
-}
-
-// out = refl + refr (+ type-0 conv), zeros for shots with V == 0
+// out = refl (+ type-0 targets) where no typed target is in the aperture,
+// zeros for shots with V == 0
 __global__ void k_finalize(float2* __restrict__ out, const float2* __restrict__ refl,
-                           const float2* __restrict__ refr, const float2* __restrict__ refr0,
-                           const int* __restrict__ Vs, int nr, int rows,
+                           const float2* __restrict__ refr0, const int* __restrict__ Vs, int nr,
+                           int rows,
                            int32_t* __restrict__ nvalid) {
     const size_t n = (size_t)nr * rows;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
@@ -3169,9 +3002,8 @@ __global__ void k_finalize(float2* __restrict__ out, const float2* __restrict__ 
         float2 v = make_float2(0.f, 0.f);
         if (Vs[r] > 0) {
             const float2 a = refl ? refl[i] : make_float2(0.f, 0.f);
-            const float2 b = refr ? refr[i] : make_float2(0.f, 0.f);
             const float2 c = refr0 ? refr0[i] : make_float2(0.f, 0.f);
-            v = make_float2(a.x + b.x + c.x, a.y + b.y + c.y);
+            v = make_float2(a.x + c.x, a.y + c.y);
         }
         out[i] = v;
         if (nvalid && (i % nr) == 0) nvalid[r] = Vs[r];
@@ -3182,76 +3014,11 @@ __global__ void k_finalize(float2* __restrict__ out, const float2* __restrict__ 
 // multi-track batches: the row-wise forms of the per-shot kernels above,
 // each row taking its track's tables from the track descriptors
 // ---------------------------------------------------------------------------
-// dst[r][k] = src[r][k] * table[k]: which = 0 the track's surface range
-// kernel spectrum (none: a track without a surface echo gets zeros),
-// which = 1 its Bluestein spectrum
-__global__ void k_mul_spec_rows(float2* __restrict__ dst, const float2* __restrict__ src, int P,
-                                int rows, const TrackK* __restrict__ trk,
-                                const RowK* __restrict__ rk, int which) {
-    const size_t n = (size_t)P * rows;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (size_t)gridDim.x * blockDim.x) {
-        const TrackK& t = trk[rk[i / P].trk];
-        const float2* spec = which == 0 ? t.g_surf : t.blue_Bw;
-        dst[i] = spec ? cmul(src[i], spec[i & (size_t)(P - 1)]) : make_float2(0.f, 0.f);
-    }
-}
-
-__global__ void k_blue_in_rows(float2* __restrict__ a, int M, const float2* __restrict__ c, int P,
-                               int L, float cscale, int rows, const TrackK* __restrict__ trk,
-                               const RowK* __restrict__ rk) {
-    const size_t n = (size_t)M * rows;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (size_t)gridDim.x * blockDim.x) {
-        const int r = (int)(i / M), k = (int)(i - (size_t)r * M);
-        float2 v = make_float2(0.f, 0.f);
-        if (k < L) {
-            float2 x = c[(size_t)r * P + k];
-            x.x *= cscale;
-            x.y *= cscale;
-            v = cmul(x, trk[rk[r].trk].blue_w[k]);
-        }
-        a[i] = v;
-    }
-}
-
-__global__ void k_blue_mid_rows(float2* __restrict__ a, int M, int L, int rows,
-                                const TrackK* __restrict__ trk, const RowK* __restrict__ rk) {
-    const size_t n = (size_t)M * rows;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (size_t)gridDim.x * blockDim.x) {
-        const int r = (int)(i / M), k = (int)(i - (size_t)r * M);
-        float2 v = make_float2(0.f, 0.f);
-        if (k < L && trk[rk[r].trk].blue_mask[k]) {
-            v = a[i];
-            v.y = -v.y;
-        }
-        a[i] = v;
-    }
-}
-
-__global__ void k_blue_out_rows(float2* __restrict__ refr, int nr, const float2* __restrict__ a,
-                                int M, float invL, int rows, const int* __restrict__ live,
-                                const TrackK* __restrict__ trk, const RowK* __restrict__ rk) {
-    const size_t n = (size_t)nr * rows;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (size_t)gridDim.x * blockDim.x) {
-        const int r = (int)(i / nr), j = (int)(i - (size_t)r * nr);
-        float2 v = make_float2(0.f, 0.f);
-        if (live[r]) {
-            v = cmul(trk[rk[r].trk].blue_w[2 * j], a[(size_t)r * M + 2 * j]);
-            v = make_float2(v.x * invL, -v.y * invL);
-        }
-        refr[i] = v;
-    }
-}
-
-// out = refl + refr (refr null: no target in the batch) into each row's
-// place in its track's radargram (rows of shot -1 pad a batch and write
-// nothing)
-__global__ void k_finalize_rows(const float2* __restrict__ refl, const float2* __restrict__ refr,
-                                const int* __restrict__ Vs, int nr, int rows,
-                                const TrackK* __restrict__ trk, const RowK* __restrict__ rk) {
+// out = refl into each row's place in its track's radargram (a group without
+// targets; rows of shot -1 pad a batch and write nothing)
+__global__ void k_finalize_rows(const float2* __restrict__ refl, const int* __restrict__ Vs,
+                                int nr, int rows, const TrackK* __restrict__ trk,
+                                const RowK* __restrict__ rk) {
     const size_t n = (size_t)nr * rows;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
          i += (size_t)gridDim.x * blockDim.x) {
@@ -3259,12 +3026,7 @@ __global__ void k_finalize_rows(const float2* __restrict__ refl, const float2* _
         const RowK row = rk[r];
         if (row.shot < 0) continue;
         const TrackK& t = trk[row.trk];
-        float2 v = make_float2(0.f, 0.f);
-        if (Vs[r] > 0) {
-            const float2 b = refr ? refr[i] : make_float2(0.f, 0.f);
-            v = make_float2(refl[i].x + b.x, refl[i].y + b.y);
-        }
-        t.out[(size_t)row.shot * nr + j] = v;
+        t.out[(size_t)row.shot * nr + j] = Vs[r] > 0 ? refl[i] : make_float2(0.f, 0.f);
         if (t.nvalid && j == 0) t.nvalid[row.shot] = Vs[r];
     }
 }
@@ -3640,40 +3402,28 @@ const float2* get_chirp(erp_ctx* ctx, int nr, float dr, float res, int kind, flo
     return c->wl.as<float2>();
 }
 
-// Bluestein tables of b (L, M, smpl, B set; w, Bw and mask sized) built on st
-void build_blue(erp_ctx* ctx, BlueTables* b, hipStream_t st) {
-    hipLaunchKernelGGL(k_blue_tables, dim3((b->M + 255) / 256), dim3(256), 0, st,
-                       b->w.as<float2>(), b->Bw.as<float2>(), b->mask.as<unsigned char>(), b->L,
-                       b->M, (double)b->smpl, (double)b->B);
-    ERP_CHECK_LAUNCH("k_blue_tables");
-    FftPlan pm = fft_plan(b->M);
-    fft_forward(ctx, pm, b->Bw.as<float2>(), 1, st);
-    hipLaunchKernelGGL(k_scale, dim3((b->M + 255) / 256), dim3(256), 0, st, b->Bw.as<float2>(),
-                       b->M, 1.0f / (float)b->M);
-    ERP_CHECK_LAUNCH("k_scale");
-}
-
-BlueTables* get_blue(erp_ctx* ctx, int L, float smpl, float B, hipStream_t st) {
+// band tables of (nr, smpl, B), cached per context
+const float2* get_band(erp_ctx* ctx, int nr, float smpl, float B, const FftPlan& plan,
+                       hipStream_t st) {
     std::lock_guard<std::recursive_mutex> lk(ctx->cache_mu);
-    for (BlueTables* b : ctx->blues)
-        if (b->L == L && b->smpl == smpl && b->B == B) return b;
-    BlueTables* b = new BlueTables();
-    b->L = L;
-    b->M = next_pow2(2 * (int64_t)L - 1);
+    for (BandTables* b : ctx->bands)
+        if (b->nr == nr && b->smpl == smpl && b->B == B) return b->tab.as<float2>();
+    BandTables* b = new BandTables();
+    b->nr = nr;
+    b->P = plan.N;
     b->smpl = smpl;
     b->B = B;
-    b->w.ensure(sizeof(float2) * (size_t)L);
-    b->Bw.ensure(sizeof(float2) * (size_t)b->M);
-    b->mask.ensure((size_t)L);
-    build_blue(ctx, b, st);
-    if (ctx->blues.size() > 8 && ctx->active.load() == 0) {
+    b->tab.ensure(sizeof(float2) * 2 * (size_t)plan.N);
+    build_band(ctx, plan, b->tab.as<float2>(), nr, smpl, B, st);
+    if (ctx->bands.size() > 8 && ctx->active.load() == 0) {
         ERP_HIP_TRY(hipStreamSynchronize(st));
-        delete ctx->blues.front();
-        ctx->blues.erase(ctx->blues.begin());
+        ctx->bands.front()->tab.release();
+        delete ctx->bands.front();
+        ctx->bands.erase(ctx->bands.begin());
     }
-    ctx->blues.push_back(b);
+    ctx->bands.push_back(b);
     ERP_HIP_TRY(hipStreamSynchronize(st));
-    return b;
+    return b->tab.as<float2>();
 }
 
 void zero(float2* p, size_t n, hipStream_t st) {
@@ -4088,14 +3838,13 @@ TargetAccumFn pick_target_accum(bool det, int ph, int acc, bool s3) {
 int64_t erp_footprint_impl(const erp_params* par, int64_t F, int64_t T, int64_t ns) {
     const int64_t nr = par->nr;
     const int64_t P = next_pow2(2 * nr - 1);
-    const int64_t M = next_pow2(2 * (2 * nr - 1) - 1);
     const int64_t S = std::max<int64_t>(1, std::min<int64_t>(ns, kShotsPerBatch));
     const int64_t nblk = (F + FB - 1) / FB;
     const bool spec = par->mode & ERP_MODE_SPECULAR;
     int64_t b = 0;
     b += S * nblk * (MASKW * 8 + 8);          // mask + counts + offsets
     b += S * F * 136 + 2560;                  // facet records (136 B per facet-shot)
-    b += S * P * 8 * 3 + S * M * 8;           // surface, spectral sum, type-0 rows; Bluestein
+    b += S * P * 8 * 5;                       // surface, spectral sum, type-0 rows; band crop
     b += S * nr * (16 + 8 + 16) + S * 4;      // FP64 surface bins, reflected, refracted
     if (spec && !(par->mode & ERP_MODE_CONVOLUTION))
         b += S * nr * 16 * direct_splits_max((int)nr);  // partial sinc sums
@@ -4147,14 +3896,7 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
                        "(sim.cu:431-439,778 otherwise write past the chirp buffer)"};
     const int64_t F = mesh->F;
     const int64_t T = targets ? targets->T : 0;
-    bool any_typed = false, any_t0 = false;
-    std::vector<unsigned char> htype;
-    if (T > 0) {
-        htype.resize(T);
-        ERP_HIP_TRY(hipMemcpyAsync(htype.data(), targets->type.p, T, hipMemcpyDeviceToHost, st));
-        ERP_HIP_TRY(hipStreamSynchronize(st));
-        for (auto t : htype) (t ? any_typed : any_t0) = true;
-    }
+    const bool any_t0 = T > 0 && targets->n0 > 0, any_typed = T > 0 && targets->n0 < T;
     if (any_typed && !(conv && lin))
         throw ErpError{ERP_E_UNSUPPORTED,
                        "targets of type != 0 need convolution and convolution_linear "
@@ -4181,7 +3923,6 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
     KPar kp = make_kpar(p, P);
     kp.ortho = mesh->frame_ok ? 1 : 0;
     kp.win_shift = (int)ctx->tune_shift;
-    const int L = 2 * nr - 1;
     const int nblk = (int)((F + FB - 1) / FB);
     // facet order of the surface kernels: tiles where a wide aperture lights
     // most of the mesh (each block's ranges then stay within its window);
@@ -4223,24 +3964,15 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
     float2* g_circ = (arena && any_t0 && conv && !lin)
                          ? arena->take_n<float2>((size_t)P, "circular chirp spectrum")
                          : nullptr;
-    BlueTables* blue = nullptr;
-    BlueTables blue_local;
-    FftPlan planM;
+    const float2* band = nullptr;
     if (any_typed) {
         if (arena) {
-            blue = &blue_local;
-            blue->L = L;
-            blue->M = next_pow2(2 * (int64_t)L - 1);
-            blue->smpl = p.smpl;
-            blue->B = p.B;
-            arena->lend(blue->w, sizeof(float2) * (size_t)L, "Bluestein chirp");
-            arena->lend(blue->Bw, sizeof(float2) * (size_t)blue->M, "Bluestein spectrum");
-            arena->lend(blue->mask, (size_t)L, "band mask");
-            build_blue(ctx, blue, st);
+            float2* tab = arena->take_n<float2>(2 * (size_t)P, "band tables");
+            build_band(ctx, planP, tab, nr, p.smpl, p.B, st);
+            band = tab;
         } else {
-            blue = get_blue(ctx, L, p.smpl, p.B, st);
+            band = get_band(ctx, nr, p.smpl, p.B, planP, st);
         }
-        planM = fft_plan(blue->M);
     }
 
     // batch size: bounded by memory of per-shot buffers
@@ -4299,10 +4031,10 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
             buf(W.psurf, sizeof(float2) * s * P, "surface traces");
             buf(W.srow, sizeof(float2) * (s * nr * 2 + (s + 1) / 2), "surface bins");
             buf(W.refl, sizeof(float2) * s * nr, "reflected traces");
-            buf(W.out, sizeof(float2) * s * nr * 2, "refracted traces");
+            if (any_t0) buf(W.out, sizeof(float2) * s * nr, "refracted traces");
             if (any_typed) {
                 buf(W.shotS, sizeof(float2) * s * P, "spectral sums");
-                buf(W.blu, sizeof(float2) * s * planM.N, "Bluestein rows");
+                buf(W.blu, sizeof(float2) * s * 2 * P, "band crop rows");
             }
             if (any_t0) buf(W.t0trace, sizeof(float2) * s * P, "type-0 traces");
             if (spec && !conv)
@@ -4369,10 +4101,10 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
     double2* srow = W.srow.as<double2>();
     unsigned* smax = reinterpret_cast<unsigned*>(srow + (size_t)Smax * nr);
     W.refl.ensure(sizeof(float2) * (size_t)Smax * nr);
-    W.out.ensure(sizeof(float2) * (size_t)Smax * nr * 2);  // refr + refr0
+    if (any_t0) W.out.ensure(sizeof(float2) * (size_t)Smax * nr);  // type-0 targets
     if (any_typed) {
         W.shotS.ensure(sizeof(float2) * (size_t)Smax * P);
-        W.blu.ensure(sizeof(float2) * (size_t)Smax * planM.N);
+        W.blu.ensure(sizeof(float2) * (size_t)Smax * 2 * P);
     }
     if (any_t0) W.t0trace.ensure(sizeof(float2) * (size_t)Smax * P);
     if (spec && !conv)
@@ -4411,8 +4143,7 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
     int64_t* dbase = W.tcount.as<int64_t>();
     unsigned long long* dmask = W.Vd.as<unsigned long long>();
     Bounds* dbounds = W.bounds.as<Bounds>();
-    float2* refr = W.out.as<float2>();
-    float2* refr0 = refr + (size_t)Smax * nr;
+    float2* refr0 = W.out.as<float2>();
 
     // S: shots of the current batch (an allocation-free run may take fewer
     // than Smax when their facet records do not fit the region)
@@ -4577,7 +4308,6 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
         }
 
         // 3: fused surface kernel
-        zero(W.psurf.as<float2>(), (size_t)S * P, st);
         hipLaunchKernelGGL(k_init_bounds, dim3(1), dim3(64), 0, st, dbounds, S);
         ERP_CHECK_LAUNCH("k_init_bounds");
         double Vsum = 0;
@@ -4618,18 +4348,18 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
                                (float4*)nullptr);
             ERP_CHECK_LAUNCH("k_surface");
         }
-        if (do_trace) {
-            hipLaunchKernelGGL(k_surf_rows, dim3((nr + 255) / 256, S), dim3(256), 0, st,
-                               W.psurf.as<float2>(), P, srow, nr, S, det ? 1 : 0, smax, dV);
-            ERP_CHECK_LAUNCH("k_surf_rows");
-        }
         PT_.end(st);
 
         if (flags & ERP_RUN_RAW_SURFACE) {
             // debug_surface: the raw surface phasor trace, no range compression
-            hipLaunchKernelGGL(k_copy_rows, dim3(grid_for((size_t)nr * S)), dim3(256), 0, st,
-                               out_dev + (size_t)s0 * nr, nr, W.psurf.as<float2>(), P, nr, S);
-            ERP_CHECK_LAUNCH("k_copy_rows");
+            if (do_trace) {
+                hipLaunchKernelGGL(k_surf_rows, dim3((nr + 255) / 256, S), dim3(256), 0, st,
+                                   out_dev + (size_t)s0 * nr, srow, nr, S, det ? 1 : 0, smax,
+                                   dV);
+                ERP_CHECK_LAUNCH("k_surf_rows");
+            } else {
+                zero(out_dev + (size_t)s0 * nr, (size_t)S * nr, st);
+            }
             if (nvalid_dev)
                 ERP_HIP_TRY(hipMemcpyAsync(nvalid_dev + s0, dV, sizeof(int) * S,
                                            hipMemcpyDeviceToDevice, st));
@@ -4641,13 +4371,12 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
         bool have_refl = false;
         if (!spec || (conv && lin)) {
             PT_.begin(ERP_STAGE_SURFACE_CONV, st, (double)S);
-            if (mode & ERP_MODE_DISABLE_SURFACE && !spec) {
-                zero(refl, (size_t)S * nr, st);
-            } else {
-                window_conv(ctx, planP, W.psurf.as<float2>(), S, g_surf, refl, nr, st);
+            if (!(mode & ERP_MODE_DISABLE_SURFACE && !spec)) {
+                surface_conv_rows(ctx, planP, srow, nr, S, det, smax, dV, g_surf,
+                                  W.psurf.as<float2>(), refl, nullptr, nullptr, st);
+                have_refl = true;
             }
             PT_.end(st);
-            have_refl = true;
         } else if (spec && !conv) {
             PT_.begin(ERP_STAGE_OTHER, st, 0.0);
             hipLaunchKernelGGL(k_direct_part<false>,
@@ -4859,6 +4588,12 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
                         PT_.end(st);
                         continue;
                     }
+                    if (spec && !planP.two_pass) {
+                        target_spectra_small(ctx, planP, A, Bs, nr, n, g_targ, Z, dseg, dseg + S,
+                                             dseg + 2 * S, nseg, Sacc, st);
+                        PT_.end(st);
+                        continue;
+                    }
                     // X = FFT(A); y = IFFT(X * g_targ); Ptarg = window(y); Z = FFT(Ptarg)
                     fft_forward(ctx, planP, A, n, st);
                     hipLaunchKernelGGL(k_mul_spec, dim3(grid_for((size_t)P * n)), dim3(256), 0,
@@ -4881,31 +4616,6 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
                     ERP_CHECK_LAUNCH("k_accum_spectra");
                     PT_.end(st);
                 }
-                // per shot: c = IFFT(S)/P; Bluestein DFT_L, crop, IDFT_L, decimate
-                PT_.begin(ERP_STAGE_SHOT_FINAL, st, (double)S);
-                fft_inverse(ctx, planP, Sacc, S, st);
-                float2* bu = W.blu.as<float2>();
-                const int M = planM.N;
-                hipLaunchKernelGGL(k_blue_in, dim3(grid_for((size_t)M * S)), dim3(256), 0, st, bu,
-                                   M, Sacc, P, blue->w.as<float2>(), L, 1.0f / (float)P, S);
-                ERP_CHECK_LAUNCH("k_blue_in");
-                fft_forward(ctx, planM, bu, S, st);
-                hipLaunchKernelGGL(k_mul_spec, dim3(grid_for((size_t)M * S)), dim3(256), 0, st, bu,
-                                   bu, blue->Bw.as<float2>(), M, S);
-                ERP_CHECK_LAUNCH("k_mul_spec");
-                fft_inverse(ctx, planM, bu, S, st);
-                hipLaunchKernelGGL(k_blue_mid, dim3(grid_for((size_t)M * S)), dim3(256), 0, st, bu,
-                                   M, blue->mask.as<unsigned char>(), L, S);
-                ERP_CHECK_LAUNCH("k_blue_mid");
-                fft_forward(ctx, planM, bu, S, st);
-                hipLaunchKernelGGL(k_mul_spec, dim3(grid_for((size_t)M * S)), dim3(256), 0, st, bu,
-                                   bu, blue->Bw.as<float2>(), M, S);
-                ERP_CHECK_LAUNCH("k_mul_spec");
-                fft_inverse(ctx, planM, bu, S, st);
-                hipLaunchKernelGGL(k_blue_out, dim3(grid_for((size_t)nr * S)), dim3(256), 0, st,
-                                   refr, nr, bu, M, blue->w.as<float2>(), 1.0f / (float)L, S, dV);
-                ERP_CHECK_LAUNCH("k_blue_out");
-                PT_.end(st);
                 have_refr = true;
             }
 
@@ -4999,12 +4709,21 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
             }
         }
 
-        // 8: combine
-        hipLaunchKernelGGL(k_finalize, dim3(grid_for((size_t)nr * S)), dim3(256), 0, st,
-                           out_dev + (size_t)s0 * nr, have_refl ? W.refl.as<float2>() : nullptr,
-                           have_refr ? refr : nullptr, have_refr0 ? refr0 : nullptr, dV, nr, S,
-                           nvalid_dev ? nvalid_dev + s0 : nullptr);
-        ERP_CHECK_LAUNCH("k_finalize");
+        // 8: typed targets' band crop, combine
+        int32_t* nv = nvalid_dev ? nvalid_dev + s0 : nullptr;
+        const float2* r0 = have_refr0 ? refr0 : nullptr;
+        if (have_refr) {
+            PT_.begin(ERP_STAGE_SHOT_FINAL, st, (double)S);
+            shot_final_rows(ctx, planP, W.shotS.as<float2>(), W.blu.as<float2>(), nr, S, band,
+                            have_refl ? refl : nullptr, r0, dV, out_dev + (size_t)s0 * nr, nv,
+                            nullptr, nullptr, st);
+            PT_.end(st);
+        } else {
+            hipLaunchKernelGGL(k_finalize, dim3(grid_for((size_t)nr * S)), dim3(256), 0, st,
+                               out_dev + (size_t)s0 * nr, have_refl ? refl : nullptr, r0, dV, nr,
+                               S, nv);
+            ERP_CHECK_LAUNCH("k_finalize");
+        }
     }
     if (check_win) check_windows(W.oow.as<int>(), st);
 }
@@ -5015,15 +4734,15 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
 // The (track, shot) rows of several tracks of one range length run in
 // batches of R rows: every launch of a batch covers all its rows, and each
 // row takes its mesh, targets, parameters, range kernel spectra and
-// Bluestein tables from its track's descriptor (TrackK).  Per batch:
+// band tables from its track's descriptor (TrackK).  Per batch:
 //   A1  aperture masks and counts of the R rows
 //       -> illuminated counts to the host: facet record bases
 //   A2  surface kernel, surface range compression, target selection
 //       -> pair counts to the host: pair lists, cut into launches of C
 //   chunk (per launch of C pairs) pair resolution, facet x target
 //       accumulation, per-pair LDS chain, slice and row sums
-//   tail  Bluestein crop and decimation of every row, then each row's trace
-//       into its track's radargram
+//   tail  band crop and decimation of every row, plus its surface echo, into
+//       its track's radargram
 // Each of the four sequences has fixed launch shapes (a short last batch is
 // padded with rows of shot -1, a short launch exits past its pair count on
 // the device), so it is captured once as a HIP graph and replayed; the
@@ -5057,7 +4776,7 @@ constexpr int kMtRowsMax = 256;
 
 struct MtState {
     MtKey key;
-    DevBuf trk, rows, shots, cnt, off, V, mask, bounds, base, psurf, srow, refl, refr, Sacc, blu,
+    DevBuf trk, rows, shots, cnt, off, V, mask, bounds, base, psurf, srow, refl, Sacc, blu,
         list, tcnt, A, Z, tabs, dtabs, rec;
     // shot-pair kernel: union masks, counts, offsets, sizes, first records
     // and first rows per block of two rows; work items and their count
@@ -5073,7 +4792,7 @@ struct MtState {
     void release() {
         reset_graphs();
         DevBuf* b[] = {&trk, &rows, &shots, &cnt, &off, &V, &mask, &bounds, &base, &psurf, &srow,
-                       &refl, &refr, &Sacc, &blu, &list, &tcnt, &A, &Z, &tabs, &dtabs, &rec,
+                       &refl, &Sacc, &blu, &list, &tcnt, &A, &Z, &tabs, &dtabs, &rec,
                        &umask, &ucnt, &uoff, &U, &ubase, &brows, &items, &bbox};
         for (DevBuf* d : b) d->release();
         key = MtKey{};
@@ -5142,9 +4861,6 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
     if (!target_half_supported(planP, nr))
         throw ErpError{ERP_E_INVALID, "multi-track batch: range length without a pair chain"};
     const int tkind = nr < P / 2 ? 2 : 0;  // the cropped pair chain's kernel placement
-    const int L = 2 * nr - 1;
-    const FftPlan planM = fft_plan(next_pow2(2 * (int64_t)L - 1));
-    const int M = planM.N;
     const int ntr = (int)trk_idx.size();
 
     // track descriptors
@@ -5191,15 +4907,12 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
         nrows += t.ns;
     }
 
-    // Bluestein tables of every track once any has targets: the tail runs
-    // over all rows of a batch (a row without targets crops a zero sum)
+    // band tables of every track once any has targets: the tail runs over all
+    // rows of a batch (a row without targets crops a zero sum)
     if (targ)
         for (int k = 0; k < ntr; ++k) {
             const erp_params& p = *tracks[trk_idx[k]].par;
-            const BlueTables* b = get_blue(ctx, L, p.smpl, p.B, st);
-            tk[k].blue_w = b->w.as<float2>();
-            tk[k].blue_Bw = b->Bw.as<float2>();
-            tk[k].blue_mask = b->mask.as<unsigned char>();
+            tk[k].band = get_band(ctx, nr, p.smpl, p.B, planP, st);
         }
 
     // shapes
@@ -5246,9 +4959,8 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
     m.srow.ensure(sizeof(float2) * srow_f2);
     m.refl.ensure(sizeof(float2) * r * nr);
     if (targ) {
-        m.refr.ensure(sizeof(float2) * r * nr);
         m.Sacc.ensure(sizeof(float2) * r * P);
-        m.blu.ensure(sizeof(float2) * r * M);
+        m.blu.ensure(sizeof(float2) * r * 2 * P);
         m.list.ensure(sizeof(int) * r * (size_t)Tcap * 2);
         m.tcnt.ensure(sizeof(int) * r * 2);
         m.bbox.ensure(sizeof(float4) * 2 * r * nblk_max);
@@ -5451,7 +5163,6 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
                                    brk.rec.itd, (int64_t)m.key.reccap);
                 ERP_CHECK_LAUNCH("k_fill_itd");
             }
-            zero(m.psurf.as<float2>(), r * P, st);
             hipLaunchKernelGGL(k_init_bounds, dim3((R + 63) / 64), dim3(64), 0, st, dbounds, R);
             ERP_CHECK_LAUNCH("k_init_bounds");
             zero(m.srow.as<float2>(), srow_f2, st);
@@ -5476,19 +5187,9 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
                                    2, smax, 0, 0, 0, dtrk, drows, BlkRec{}, (float4*)nullptr);
                 ERP_CHECK_LAUNCH("k_surface");
             }
-            hipLaunchKernelGGL(k_surf_rows, dim3((nr + 255) / 256, R), dim3(256), 0, st,
-                               m.psurf.as<float2>(), P, srow, nr, R, det ? 1 : 0, smax, dV);
-            ERP_CHECK_LAUNCH("k_surf_rows");
             // reflected signal: each row with its track's range kernel
-            float2* ps = m.psurf.as<float2>();
-            fft_forward(ctx, planP, ps, R, st);
-            hipLaunchKernelGGL(k_mul_spec_rows, dim3(grid_for(r * P)), dim3(256), 0, st, ps, ps,
-                               P, R, dtrk, drows, 0);
-            ERP_CHECK_LAUNCH("k_mul_spec_rows");
-            fft_inverse(ctx, planP, ps, R, st);
-            hipLaunchKernelGGL(k_window, dim3(grid_for(r * nr)), dim3(256), 0, st,
-                               m.refl.as<float2>(), nr, ps, P, nr, R, 1.0f, 0);
-            ERP_CHECK_LAUNCH("k_window");
+            surface_conv_rows(ctx, planP, srow, nr, R, det, smax, dV, nullptr,
+                              m.psurf.as<float2>(), m.refl.as<float2>(), dtrk, drows, st);
             if (targ) {
                 hipLaunchKernelGGL(k_target_select, dim3(R), dim3(1024), 0, st,
                                    (const float*)nullptr, (int64_t)0, 0,
@@ -5498,8 +5199,7 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
                 zero(m.Sacc.as<float2>(), r * P, st);
             } else {
                 hipLaunchKernelGGL(k_finalize_rows, dim3(grid_for(r * nr)), dim3(256), 0, st,
-                                   m.refl.as<float2>(), (const float2*)nullptr, dV, nr, R, dtrk,
-                                   drows);
+                                   m.refl.as<float2>(), dV, nr, R, dtrk, drows);
                 ERP_CHECK_LAUNCH("k_finalize_rows");
             }
         });
@@ -5645,36 +5345,11 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
             PT_.end(st);
         }
 
-        // tail: per row c = IFFT(S)/P; Bluestein DFT_L, crop, IDFT_L, decimate;
-        // then refl + refr into the track's radargram
+        // tail: each row's band crop, plus its echo, into the track's radargram
         PT_.begin(ERP_STAGE_SHOT_FINAL, st, (double)nb);
         mt_launch(m.gTail, direct, st, [&] {
-            float2* Sacc = m.Sacc.as<float2>();
-            float2* bu = m.blu.as<float2>();
-            fft_inverse(ctx, planP, Sacc, R, st);
-            hipLaunchKernelGGL(k_blue_in_rows, dim3(grid_for(r * M)), dim3(256), 0, st, bu, M,
-                               Sacc, P, L, 1.0f / (float)P, R, dtrk, drows);
-            ERP_CHECK_LAUNCH("k_blue_in_rows");
-            fft_forward(ctx, planM, bu, R, st);
-            hipLaunchKernelGGL(k_mul_spec_rows, dim3(grid_for(r * M)), dim3(256), 0, st, bu, bu,
-                               M, R, dtrk, drows, 1);
-            ERP_CHECK_LAUNCH("k_mul_spec_rows");
-            fft_inverse(ctx, planM, bu, R, st);
-            hipLaunchKernelGGL(k_blue_mid_rows, dim3(grid_for(r * M)), dim3(256), 0, st, bu, M,
-                               L, R, dtrk, drows);
-            ERP_CHECK_LAUNCH("k_blue_mid_rows");
-            fft_forward(ctx, planM, bu, R, st);
-            hipLaunchKernelGGL(k_mul_spec_rows, dim3(grid_for(r * M)), dim3(256), 0, st, bu, bu,
-                               M, R, dtrk, drows, 1);
-            ERP_CHECK_LAUNCH("k_mul_spec_rows");
-            fft_inverse(ctx, planM, bu, R, st);
-            hipLaunchKernelGGL(k_blue_out_rows, dim3(grid_for(r * nr)), dim3(256), 0, st,
-                               m.refr.as<float2>(), nr, bu, M, 1.0f / (float)L, R, dV, dtrk,
-                               drows);
-            ERP_CHECK_LAUNCH("k_blue_out_rows");
-            hipLaunchKernelGGL(k_finalize_rows, dim3(grid_for(r * nr)), dim3(256), 0, st,
-                               m.refl.as<float2>(), m.refr.as<float2>(), dV, nr, R, dtrk, drows);
-            ERP_CHECK_LAUNCH("k_finalize_rows");
+            shot_final_rows(ctx, planP, m.Sacc.as<float2>(), m.blu.as<float2>(), nr, R, nullptr,
+                            m.refl.as<float2>(), nullptr, dV, nullptr, nullptr, dtrk, drows, st);
         });
         PT_.end(st);
     }
