@@ -130,8 +130,16 @@ void release_work(WorkBufs& w) {
     DevBuf* bufs[] = {&w.cnt, &w.off, &w.V, &w.Vd, &w.tcnt, &w.tlist, &w.tcount, &w.rec,
                       &w.bounds, &w.psurf, &w.srow, &w.refl, &w.shotS, &w.blu, &w.tA, &w.tB, &w.tC,
                       &w.pairs, &w.t0trace, &w.dpart, &w.shots, &w.prisms, &w.out, &w.nvalid, &w.oow,
-                      &w.umask, &w.ucnt, &w.uoff, &w.U, &w.ubase, &w.brec, &w.items, &w.bbox};
+                      &w.umask, &w.ucnt, &w.uoff, &w.ubase, &w.brec, &w.items, &w.bbox};
     for (DevBuf* b : bufs) b->release();
+    if (w.pin) hipHostFree(w.pin);
+    w.pin = nullptr;
+}
+
+int* alloc_pin() {
+    void* p = nullptr;
+    ERP_HIP_TRY(hipHostMalloc(&p, sizeof(int) * kPinWords, hipHostMallocDefault));
+    return static_cast<int*>(p);
 }
 
 // Runs one job on a slot: the pipeline on the slot's stream, the copies back
@@ -204,6 +212,13 @@ void start_slots(erp_ctx* ctx, int n) {
         if (e != hipSuccess) {
             delete s;
             throw ErpError{ERP_E_HIP, std::string("hipStreamCreate: ") + hipGetErrorString(e)};
+        }
+        try {
+            s->work.pin = alloc_pin();
+        } catch (...) {
+            hipStreamDestroy(s->stream);
+            delete s;
+            throw;
         }
         s->th = std::thread(slot_main, ctx, s);
         ctx->slots.push_back(s);
@@ -289,11 +304,13 @@ int erp_ctx_create(int device, erp_ctx** out) {
         hipDeviceProp_t prop;
         ERP_HIP_TRY(hipGetDeviceProperties(&prop, device));
         ctx->num_cu = prop.multiProcessorCount;
+        ctx->work.pin = alloc_pin();
         fft_init_twiddles(ctx);
         scratch_init(device);
         ERP_HIP_TRY(hipStreamSynchronize(ctx->stream));
     });
     if (rc != ERP_OK) {
+        release_work(ctx->work);
         if (ctx->stream) hipStreamDestroy(ctx->stream);
         delete ctx;
         return rc;
@@ -597,6 +614,7 @@ int erp_run_dev_noalloc(erp_ctx* ctx, const erp_params* par, const erp_mesh* mes
         a.base = static_cast<char*>(g_scratch[ctx->device].ptr);
         a.cap = (size_t)ERP_SCRATCH_BYTES;
         WorkBufs w;  // every buffer is lent from the arena; nothing to release
+        w.pin = ctx->work.pin;  // this thread holds ctx->mu
         try {
             erp_run_impl(ctx, par, mesh, targets, shots, ns, prisms, nprisms, (float2*)out_dev,
                          (int32_t*)nvalid_dev, flags, ctx->stream, w, nullptr, &a);

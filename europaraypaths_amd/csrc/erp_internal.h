@@ -189,7 +189,15 @@ struct BandTables {
     DevBuf tab;
 };
 
+// Pinned host words of a run: the counts of a batch (up to kPinCounts: V per
+// shot, U per block of two), the target counts, the window check, then
+// target lists of up to kPinList entries.
+constexpr int kPinCounts = 128;
+constexpr size_t kPinList = 16384;
+constexpr size_t kPinWords = 512 + kPinList;
+
 struct WorkBufs {
+    int* pin = nullptr;  // kPinWords pinned words, owned by the context or slot
     DevBuf cnt, off, V, Vd, tcnt, tlist, tcount;  // counts / offsets
     DevBuf rec;        // compacted facet records
     DevBuf bounds;     // per-shot bounds of illuminated facets
@@ -207,9 +215,9 @@ struct WorkBufs {
     DevBuf out;        // S x nr complex (device output staging)
     DevBuf nvalid;     // S int32
     DevBuf oow;        // count of target terms outside their pair's bin window
-    // shot-pair target kernel: union masks, counts, offsets and sizes per
-    // block of two shots; block records; work items
-    DevBuf umask, ucnt, uoff, U, ubase, brec, items;
+    // shot-pair target kernel: union masks, counts and offsets per block of
+    // two shots; block records; work items with their slices and segments
+    DevBuf umask, ucnt, uoff, ubase, brec, items;
     DevBuf bbox;       // per (shot, facet block) box of the lit facets
 };
 

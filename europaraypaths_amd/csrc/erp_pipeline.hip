@@ -406,6 +406,44 @@ __global__ void k_init_bounds(Bounds* b, int S) {
     }
 }
 
+// What a batch needs before its surface kernel, in one launch: the record
+// bases (exclusive sums of V over the shots and of U over the blocks of two
+// shots; S <= 64, one wave), the shots' bounds, and the buffers that are
+// summed into cleared: the surface bins and the spectral sums to zero, the
+// block records' Itd to -1 ("not lit").  Sizes in 8-byte words.
+__global__ void __launch_bounds__(256) k_batch_prep(
+    const int* __restrict__ V, const int* __restrict__ U, int S, int64_t* __restrict__ base,
+    int64_t* __restrict__ ubase, Bounds* __restrict__ b, double* __restrict__ z0, size_t n0,
+    double* __restrict__ z1, size_t n1, double* __restrict__ itd, size_t ni) {
+    if (blockIdx.x == 0 && threadIdx.x < 64) {
+        const int s = threadIdx.x;
+        auto scan = [&](int n, const int* v, int64_t* out) {
+            int64_t x = s < n ? v[s] : 0;
+            const int64_t own = x;
+            for (int o = 1; o < 64; o <<= 1) {
+                const int64_t y = __shfl_up(x, o);
+                if (s >= o) x += y;
+            }
+            if (s < n) out[s] = x - own;
+        };
+        if (base) scan(S, V, base);
+        if (ubase) scan((S + 1) / 2, U, ubase);
+        if (s < S) {
+            b[s].itd_min = ~0ull; b[s].itd_max = 0ull;
+            b[s].xmin = b[s].ymin = b[s].zmin = 0xFFFFFFFFu;
+            b[s].xmax = b[s].ymax = b[s].zmax = 0u;
+            b[s].cx = b[s].cy = b[s].cz = 0.f;
+            b[s].rad = -1.f;
+        }
+    }
+    const size_t n = n0 + n1 + ni;
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
+        if (i < n0) z0[i] = 0.0;
+        else if (i < n0 + n1) z1[i - n0] = 0.0;
+        else itd[i - n0 - n1] = -1.0;
+    }
+}
+
 // Bounding sphere of each shot's lit facets: centre c = the centre of the
 // shot's box, radius = the largest distance from c to a corner of a lit
 // facet block's box (every lit facet lies in its block's box).  Each facet
@@ -546,12 +584,21 @@ __global__ void __launch_bounds__(NT) k_illum_mask(
 // ---------------------------------------------------------------------------
 // 2. per-shot exclusive scan of block counts
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(1024) k_scan_blocks(const int* __restrict__ cnt,
-                                                      int* __restrict__ off,
-                                                      int* __restrict__ V, int nblk,
-                                                      const TrackK* __restrict__ trk,
-                                                      const RowK* __restrict__ rows) {
-    const int s = blockIdx.x;
+// rows [0, S): the shots' counts; rows from S on (in the same launch): those
+// of the blocks of two shots (cnt2, off2, V2, rows2)
+__global__ void __launch_bounds__(1024) k_scan_blocks(
+    const int* __restrict__ cnt, int* __restrict__ off, int* __restrict__ V, int nblk, int S,
+    const int* __restrict__ cnt2, int* __restrict__ off2, int* __restrict__ V2,
+    const TrackK* __restrict__ trk, const RowK* __restrict__ rows,
+    const RowK* __restrict__ rows2) {
+    int s = blockIdx.x;
+    if (s >= S) {
+        s -= S;
+        cnt = cnt2;
+        off = off2;
+        V = V2;
+        rows = rows2;
+    }
     // rows of a multi-track batch: stride nblk, the row's mesh's own count;
     // a padding row (shot -1) illuminates nothing
     if (trk && rows[s].shot < 0) {
@@ -3451,10 +3498,10 @@ void window_conv(erp_ctx* ctx, const FftPlan& plan, float2* data, int rows, cons
 // After a run: the count of target terms that fell outside a bin window
 // their pair's bounds should have covered (k_target_accum_fast); any is a
 // broken bound, whose terms were dropped, so the run fails.
-void check_windows(const int* oow, hipStream_t st) {
-    int n = 0;
-    ERP_HIP_TRY(hipMemcpyAsync(&n, oow, sizeof(int), hipMemcpyDeviceToHost, st));
+void check_windows(const int* oow, int* host, hipStream_t st) {
+    ERP_HIP_TRY(hipMemcpyAsync(host, oow, sizeof(int), hipMemcpyDeviceToHost, st));
     ERP_HIP_TRY(hipStreamSynchronize(st));
+    const int n = *host;
     if (n != 0)
         throw ErpError{ERP_E_INTERNAL,
                        std::to_string(n) + " facet x target terms fell outside the bin window "
@@ -4008,6 +4055,13 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
         if (!spec && any_typed) b += 3 * Arena::round(cap * 16) + Arena::round(cap * 4);
         return b;
     };
+    // upload of one launch of the shot-pair kernel: 16 bytes for its item
+    // counter, the slices and segments, then the items
+    auto item_head = [&](int C_, int S_) -> size_t {
+        const size_t ints = 2 * ((size_t)C_ / GS + S_ + 2) + 3 * (size_t)S_;
+        return 16 + ((ints * sizeof(int) + 15) & ~(size_t)15);
+    };
+    auto item_bytes = [&](int C_, int S_) { return item_head(C_, S_) + sizeof(int4) * (size_t)C_; };
     // Allocation-free run: every batch buffer is lent from the arena before
     // the loop (the loop's ensure calls then find it large enough).  Shots per
     // batch and pairs per launch shrink until the fixed buffers take at most
@@ -4024,7 +4078,7 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
             if (nprisms > 0) buf(W.prisms, sizeof(erp_prism) * (size_t)nprisms, "prism table");
             buf(W.cnt, sizeof(int) * s * nblk, "block counts");
             buf(W.off, sizeof(int) * s * nblk, "block offsets");
-            buf(W.V, sizeof(int) * s, "illuminated counts");
+            buf(W.V, sizeof(int) * (s + (s + 1) / 2), "illuminated counts");
             buf(W.Vd, sizeof(unsigned long long) * s * nblk * MASKW, "aperture mask");
             buf(W.bounds, sizeof(Bounds) * s, "shot bounds");
             buf(W.tcount, sizeof(int64_t) * s, "record bases");
@@ -4060,9 +4114,8 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
                 buf(W.umask, sizeof(unsigned long long) * nb * nblk * MASKW, "union masks");
                 buf(W.ucnt, sizeof(int) * nb * nblk, "union counts");
                 buf(W.uoff, sizeof(int) * nb * nblk, "union offsets");
-                buf(W.U, sizeof(int) * nb, "union sizes");
                 buf(W.ubase, sizeof(int64_t) * nb, "block record bases");
-                buf(W.items, sizeof(int4) * (size_t)C_, "pair items");
+                buf(W.items, item_bytes(C_, S_), "pair items");
             }
             return tot;
         };
@@ -4091,7 +4144,7 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
     }
     W.cnt.ensure(sizeof(int) * (size_t)Smax * nblk);
     W.off.ensure(sizeof(int) * (size_t)Smax * nblk);
-    W.V.ensure(sizeof(int) * (size_t)Smax);
+    W.V.ensure(sizeof(int) * ((size_t)Smax + (Smax + 1) / 2));  // V per shot, U per block of two
     W.Vd.ensure(sizeof(unsigned long long) * (size_t)Smax * nblk * MASKW);  // mask
     W.bounds.ensure(sizeof(Bounds) * (size_t)Smax);
     W.tcount.ensure(sizeof(int64_t) * (size_t)Smax);  // rec_base
@@ -4121,7 +4174,7 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
     const bool check_win = any_typed && (!spec || det);
     if (check_win) {
         W.oow.ensure(256);
-        ERP_HIP_TRY(hipMemsetAsync(W.oow.p, 0, sizeof(int), st));
+        zero(W.oow.as<float2>(), 1, st);
     }
 
     // the shot-pair kernel's buffers: union masks and records per block of
@@ -4131,15 +4184,17 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
         W.umask.ensure(sizeof(unsigned long long) * (size_t)nbk_max * nblk * MASKW);
         W.ucnt.ensure(sizeof(int) * (size_t)nbk_max * nblk);
         W.uoff.ensure(sizeof(int) * (size_t)nbk_max * nblk);
-        W.U.ensure(sizeof(int) * (size_t)nbk_max);
         W.ubase.ensure(sizeof(int64_t) * (size_t)nbk_max);
     }
-    std::vector<int> hU(nbk_max);
-    std::vector<int64_t> hubase(nbk_max + 1);
-
-    std::vector<int> hV(Smax), htc(2 * Smax);
-    std::vector<int64_t> hbase(Smax + 1);
+    // counts come back through pinned memory: one wait per read, whatever
+    // the number of arrays
+    int* const hV = W.pin;                       // V, then U from Smax on
+    int* const hU = hV + Smax;
+    int* const htc = hV + kPinCounts;            // target counts
+    int* const hoow = htc + 2 * kShotsPerBatch;  // the window check's count
+    int* const hlist = hoow + 1;                 // short target lists
     int* dV = W.V.as<int>();
+    int* dU = dV + Smax;
     int64_t* dbase = W.tcount.as<int64_t>();
     unsigned long long* dmask = W.Vd.as<unsigned long long>();
     Bounds* dbounds = W.bounds.as<Bounds>();
@@ -4163,26 +4218,27 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
                            W.cnt.as<int>(), nblk, tile_nx, (const TrackK*)nullptr,
                            (const RowK*)nullptr, S, MASK_SB);
         ERP_CHECK_LAUNCH("k_illum_mask");
-        hipLaunchKernelGGL(k_scan_blocks, dim3(S), dim3(1024), 0, st, W.cnt.as<int>(),
-                           W.off.as<int>(), dV, nblk, (const TrackK*)nullptr,
-                           (const RowK*)nullptr);
-        ERP_CHECK_LAUNCH("k_scan_blocks");
         // blocks of two shots: the union of their masks, its offsets and size
-        int nbk = (S + 1) / 2;
-        if (pairk) {
-            hipLaunchKernelGGL(k_union_mask, dim3(nblk, nbk), dim3(MASKW), 0, st, dmask, nblk, S,
-                               W.umask.as<unsigned long long>(), W.ucnt.as<int>(),
-                               (const TrackK*)nullptr, (const RowK*)nullptr);
-            ERP_CHECK_LAUNCH("k_union_mask");
-            hipLaunchKernelGGL(k_scan_blocks, dim3(nbk), dim3(1024), 0, st, W.ucnt.as<int>(),
-                               W.uoff.as<int>(), W.U.as<int>(), nblk, (const TrackK*)nullptr,
+        int nbk = pairk ? (S + 1) / 2 : 0;
+        auto scan = [&](int shots_, int blocks_) {
+            hipLaunchKernelGGL(k_scan_blocks, dim3(shots_ + blocks_), dim3(1024), 0, st,
+                               W.cnt.as<int>(), W.off.as<int>(), dV, nblk, shots_,
+                               (const int*)W.ucnt.as<int>(), W.uoff.as<int>(), dU,
+                               (const TrackK*)nullptr, (const RowK*)nullptr,
                                (const RowK*)nullptr);
             ERP_CHECK_LAUNCH("k_scan_blocks");
-            ERP_HIP_TRY(hipMemcpyAsync(hU.data(), W.U.p, sizeof(int) * nbk,
-                                       hipMemcpyDeviceToHost, st));
-        }
+        };
+        auto unite = [&](int shots_) {
+            hipLaunchKernelGGL(k_union_mask, dim3(nblk, (shots_ + 1) / 2), dim3(MASKW), 0, st,
+                               dmask, nblk, shots_, W.umask.as<unsigned long long>(),
+                               W.ucnt.as<int>(), (const TrackK*)nullptr, (const RowK*)nullptr);
+            ERP_CHECK_LAUNCH("k_union_mask");
+        };
+        if (pairk) unite(S);
+        scan(S, nbk);
         PT_.end(st);
-        ERP_HIP_TRY(hipMemcpyAsync(hV.data(), dV, sizeof(int) * S, hipMemcpyDeviceToHost, st));
+        ERP_HIP_TRY(hipMemcpyAsync(hV, dV, sizeof(int) * ((size_t)Smax + nbk),
+                                   hipMemcpyDeviceToHost, st));
         ERP_HIP_TRY(hipStreamSynchronize(st));
         auto brec_need = [](size_t cap) {
             return 5 * Arena::round(cap * 16) + Arena::round(cap * 4);
@@ -4198,16 +4254,9 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
             if (fitb == 0 && S > 1) {
                 S = 1;
                 nbk = 1;
-                hipLaunchKernelGGL(k_union_mask, dim3(nblk, 1), dim3(MASKW), 0, st, dmask, nblk, 1,
-                                   W.umask.as<unsigned long long>(), W.ucnt.as<int>(),
-                                   (const TrackK*)nullptr, (const RowK*)nullptr);
-                ERP_CHECK_LAUNCH("k_union_mask");
-                hipLaunchKernelGGL(k_scan_blocks, dim3(1), dim3(1024), 0, st, W.ucnt.as<int>(),
-                                   W.uoff.as<int>(), W.U.as<int>(), nblk, (const TrackK*)nullptr,
-                                   (const RowK*)nullptr);
-                ERP_CHECK_LAUNCH("k_scan_blocks");
-                ERP_HIP_TRY(hipMemcpyAsync(hU.data(), W.U.p, sizeof(int), hipMemcpyDeviceToHost,
-                                           st));
+                unite(1);
+                scan(0, 1);
+                ERP_HIP_TRY(hipMemcpyAsync(hU, dU, sizeof(int), hipMemcpyDeviceToHost, st));
                 ERP_HIP_TRY(hipStreamSynchronize(st));
                 if (brec_need((size_t)hU[0]) <= W.brec.bytes) fitb = 1;
             }
@@ -4235,26 +4284,24 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
                                    std::to_string(W.rec.bytes) + " for records"};
             S = fit;
         }
-        hbase[0] = 0;
-        for (int s = 0; s < S; ++s) hbase[s + 1] = hbase[s] + (need_rec ? hV[s] : 0);
         // the target kernel reads a shot's records at 32-bit byte offsets
-        for (int s = 0; s < S; ++s)
+        int64_t Vtot = 0;
+        for (int s = 0; s < S; ++s) {
             if (need_rec && hV[s] >= (1 << 28))
                 throw ErpError{ERP_E_INVALID, "a shot illuminates 2^28 facets or more"};
-        const int64_t Vtot = hbase[S];
-        ERP_HIP_TRY(hipMemcpyAsync(dbase, hbase.data(), sizeof(int64_t) * S,
-                                   hipMemcpyHostToDevice, st));
+            if (need_rec) Vtot += hV[s];
+        }
+        size_t ucap = 0;  // block records
         Rec rec{};
         BlkRec brk{};
         if (pairk && Vtot > 0) {
             // block records: 84 bytes per facet of a block's union
-            hubase[0] = 0;
             for (int j = 0; j < nbk; ++j) {
                 if (hU[j] >= (1 << 28))
                     throw ErpError{ERP_E_INVALID, "two shots illuminate 2^28 facets or more"};
-                hubase[j + 1] = hubase[j] + hU[j];
+                ucap += (size_t)hU[j];
             }
-            const size_t cap = (size_t)hubase[nbk];
+            const size_t cap = ucap;
             auto rnd = [](size_t n) { return (n + 255) & ~(size_t)255; };
             const size_t bytes = brec_need(cap);
             if (arena) W.brec.ensure(bytes);  // fits: the batch was cut to fit
@@ -4270,15 +4317,8 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
             br.src = (float4*)take(cap * 16);
             brk.umask = W.umask.as<unsigned long long>();
             brk.uoff = W.uoff.as<int>();
-            brk.U = W.U.as<int>();
+            brk.U = dU;
             brk.ubase = W.ubase.as<int64_t>();
-            ERP_HIP_TRY(hipMemcpyAsync(W.ubase.p, hubase.data(), sizeof(int64_t) * nbk,
-                                       hipMemcpyHostToDevice, st));
-            if (cap > 0) {
-                hipLaunchKernelGGL(k_fill_itd, dim3(grid_for(cap)), dim3(256), 0, st, br.itd,
-                                   (int64_t)cap);
-                ERP_CHECK_LAUNCH("k_fill_itd");
-            }
         } else if (need_rec && Vtot > 0) {
             const size_t cap = (size_t)Vtot;
             // at most every facet of every shot of the batch (the bound that
@@ -4308,12 +4348,19 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
         }
 
         // 3: fused surface kernel
-        hipLaunchKernelGGL(k_init_bounds, dim3(1), dim3(64), 0, st, dbounds, S);
-        ERP_CHECK_LAUNCH("k_init_bounds");
+        {
+            const size_t n0 = do_trace ? srow_f2 : 0, n1 = any_typed ? (size_t)S * P : 0,
+                         ni = brk.rec.itd ? 2 * ucap : 0;
+            hipLaunchKernelGGL(k_batch_prep, dim3(grid_for(n0 + n1 + ni, 256, 4096)), dim3(256), 0,
+                               st, (const int*)dV, (const int*)dU, S, need_rec ? dbase : nullptr,
+                               pairk ? W.ubase.as<int64_t>() : nullptr, dbounds,
+                               W.srow.as<double>(), n0, W.shotS.as<double>(), n1,
+                               reinterpret_cast<double*>(brk.rec.itd), ni);
+            ERP_CHECK_LAUNCH("k_batch_prep");
+        }
         double Vsum = 0;
         for (int s = 0; s < S; ++s) Vsum += hV[s];
         PT_.begin(ERP_STAGE_SURFACE, st, Vsum);
-        if (do_trace) zero(W.srow.as<float2>(), srow_f2, st);
         const int write = (need_rec && Vtot > 0) ? 1 : 0;
         if (T == 0 && !spec && !det && ph == PH_F64 && acc == ACC_F64) {
             // no targets: nothing reads records or bounds (shots are the fast
@@ -4406,8 +4453,14 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
                                (const RowK*)nullptr);
             ERP_CHECK_LAUNCH("k_target_select");
             PT_.end(st);
-            ERP_HIP_TRY(hipMemcpyAsync(htc.data(), W.tcnt.p, sizeof(int) * 2 * S,
-                                       hipMemcpyDeviceToHost, st));
+            ERP_HIP_TRY(hipMemcpyAsync(htc, W.tcnt.p, sizeof(int) * 2 * S, hipMemcpyDeviceToHost,
+                                       st));
+            // short lists come with their counts; long ones once the longest
+            // is known
+            const bool short_lists = pairk && (size_t)S * Tcap <= kPinList;
+            if (short_lists)
+                ERP_HIP_TRY(hipMemcpyAsync(hlist, list1, sizeof(int) * (size_t)S * Tcap,
+                                           hipMemcpyDeviceToHost, st));
             ERP_HIP_TRY(hipStreamSynchronize(st));
             const erp_prism* dpr = nprisms > 0 ? W.prisms.as<erp_prism>() : nullptr;
 
@@ -4415,8 +4468,7 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
             int64_t npairs = 0;
             for (int s = 0; s < S; ++s) npairs += htc[2 * s];
             if (npairs > 0) {
-                float2* Sacc = W.shotS.as<float2>();
-                zero(Sacc, (size_t)S * P, st);
+                float2* Sacc = W.shotS.as<float2>();  // cleared by k_batch_prep
                 const size_t gcap = (size_t)C / GS + S + 2;
                 // half: A rows, then one partial row per slice
                 W.tA.ensure(sizeof(float2) * (size_t)P *
@@ -4441,43 +4493,46 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
                     // consecutive shots, from the shots' target lists
                     int maxc = 0;
                     for (int s = 0; s < S; ++s) maxc = std::max(maxc, htc[2 * s]);
-                    std::vector<int> hl((size_t)S * maxc);
-                    if (maxc > 0) {
+                    std::vector<int> hl(short_lists ? 0 : (size_t)S * maxc);
+                    if (maxc > 0 && !short_lists) {
                         ERP_HIP_TRY(hipMemcpy2DAsync(hl.data(), sizeof(int) * maxc, list1,
                                                      sizeof(int) * Tcap, sizeof(int) * maxc, S,
                                                      hipMemcpyDeviceToHost, st));
                         ERP_HIP_TRY(hipStreamSynchronize(st));
                     }
                     std::vector<std::vector<PairIdx>> bl;
-                    merge_pair_lists(hl.data(), (size_t)maxc, htc.data(), S, bl);
-                    W.items.ensure(sizeof(int4) * (size_t)C);
-                    int4* ditems = W.items.as<int4>();
-                    int* dnext = dpw + C;  // item counter, in the spare tail of the list
+                    merge_pair_lists(short_lists ? hlist : hl.data(),
+                                     (size_t)(short_lists ? Tcap : maxc), htc, S, bl);
+                    W.items.ensure(item_bytes(C, Smax));
+                    const size_t head = item_head(C, Smax);
+                    int* dnext = W.items.as<int>();  // item counter
+                    int* dsl = dnext + 4;            // slices, then segments
+                    int4* ditems = reinterpret_cast<int4*>(W.items.as<char>() + head);
+                    std::vector<char> up;
                     PairChunk pc;
                     int jb = 0;
                     size_t ib = 0;
                     PairCursor cur;
                     for (;;) {
                         // deterministic: every shot's slices independent of the launches
-                        if (det) fill_pair_chunk_canon(bl, cur, C, GS, hV.data(), pc);
-                        else fill_pair_chunk(bl, jb, ib, C, GS, hV.data(), pc);
+                        if (det) fill_pair_chunk_canon(bl, cur, C, GS, hV, pc);
+                        else fill_pair_chunk(bl, jb, ib, C, GS, hV, pc);
                         const int n = pc.rows;
                         if (n == 0) break;
                         const int nseg = (int)pc.sg_s.size();
                         const int ngroups = (int)pc.gb.size();
                         const int nit = (int)pc.items.size();
-                        // slices and segments at the offsets the chain reads them
-                        std::vector<int> up(2 * gcap + 3 * (size_t)S, 0);
-                        std::copy(pc.gb.begin(), pc.gb.end(), up.begin());
-                        std::copy(pc.ge.begin(), pc.ge.end(), up.begin() + gcap);
-                        std::copy(pc.sg_s.begin(), pc.sg_s.end(), up.begin() + 2 * gcap);
-                        std::copy(pc.gsb.begin(), pc.gsb.end(), up.begin() + 2 * gcap + S);
-                        std::copy(pc.gse.begin(), pc.gse.end(), up.begin() + 2 * gcap + 2 * S);
-                        ERP_HIP_TRY(hipMemcpyAsync(dgb, up.data(), sizeof(int) * up.size(),
+                        // counter 0, slices and segments, items: one upload
+                        up.assign(head + sizeof(int4) * (size_t)nit, 0);
+                        int* u = reinterpret_cast<int*>(up.data()) + 4;
+                        std::copy(pc.gb.begin(), pc.gb.end(), u);
+                        std::copy(pc.ge.begin(), pc.ge.end(), u + gcap);
+                        std::copy(pc.sg_s.begin(), pc.sg_s.end(), u + 2 * gcap);
+                        std::copy(pc.gsb.begin(), pc.gsb.end(), u + 2 * gcap + S);
+                        std::copy(pc.gse.begin(), pc.gse.end(), u + 2 * gcap + 2 * S);
+                        std::memcpy(up.data() + head, pc.items.data(), sizeof(int4) * nit);
+                        ERP_HIP_TRY(hipMemcpyAsync(W.items.p, up.data(), up.size(),
                                                    hipMemcpyHostToDevice, st));
-                        ERP_HIP_TRY(hipMemcpyAsync(ditems, pc.items.data(), sizeof(int4) * nit,
-                                                   hipMemcpyHostToDevice, st));
-                        ERP_HIP_TRY(hipMemsetAsync(dnext, 0, sizeof(int), st));
                         PT_.begin(ERP_STAGE_TARGET_ACCUM, st, pc.triples);
                         // persistent grid: one workgroup per CU (its two windows
                         // take 128 KB of LDS), each taking items until none is left
@@ -4500,8 +4555,9 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
                         target_pairs_half(ctx, planP, A, dpb, dpw, nr, n, g_targ_nat, Z, st);
                         PT_.end(st);
                         PT_.begin(ERP_STAGE_TARGET_SUM, st, (double)n);
-                        target_sum_half(planP, Z, A + (size_t)C * P, dgb, dge, ngroups, dseg,
-                                        dseg + S, dseg + 2 * S, nseg, Sacc, -1.0f / kp.sqrtP, st,
+                        int* sg = dsl + 2 * gcap;
+                        target_sum_half(planP, Z, A + (size_t)C * P, dsl, dsl + gcap, ngroups, sg,
+                                        sg + S, sg + 2 * S, nseg, Sacc, -1.0f / kp.sqrtP, st,
                                         nullptr, det, wl);
                         PT_.end(st);
                     }
@@ -4725,7 +4781,7 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
             ERP_CHECK_LAUNCH("k_finalize");
         }
     }
-    if (check_win) check_windows(W.oow.as<int>(), st);
+    if (check_win) check_windows(W.oow.as<int>(), hoow, st);
 }
 
 // ---------------------------------------------------------------------------
@@ -5063,20 +5119,18 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
                                m.mask.as<unsigned long long>(), m.cnt.as<int>(), nblk_max, 0,
                                dtrk, drows, R, 1);
             ERP_CHECK_LAUNCH("k_illum_mask");
-            hipLaunchKernelGGL(k_scan_blocks, dim3(R), dim3(1024), 0, st, m.cnt.as<int>(),
-                               m.off.as<int>(), dV, nblk_max, dtrk, drows);
-            ERP_CHECK_LAUNCH("k_scan_blocks");
             if (pairk) {
                 hipLaunchKernelGGL(k_union_mask, dim3(nblk_max, nbk), dim3(MASKW), 0, st,
                                    m.mask.as<unsigned long long>(), nblk_max, R,
                                    m.umask.as<unsigned long long>(), m.ucnt.as<int>(), dtrk,
                                    drows);
                 ERP_CHECK_LAUNCH("k_union_mask");
-                hipLaunchKernelGGL(k_scan_blocks, dim3(nbk), dim3(1024), 0, st, m.ucnt.as<int>(),
-                                   m.uoff.as<int>(), m.U.as<int>(), nblk_max, dtrk,
-                                   m.brows.as<RowK>());
-                ERP_CHECK_LAUNCH("k_scan_blocks");
             }
+            hipLaunchKernelGGL(k_scan_blocks, dim3(R + (pairk ? nbk : 0)), dim3(1024), 0, st,
+                               m.cnt.as<int>(), m.off.as<int>(), dV, nblk_max, R,
+                               (const int*)m.ucnt.as<int>(), m.uoff.as<int>(), m.U.as<int>(), dtrk,
+                               drows, (const RowK*)m.brows.as<RowK>());
+            ERP_CHECK_LAUNCH("k_scan_blocks");
         });
         PT_.end(st);
         ERP_HIP_TRY(hipMemcpyAsync(hV.data(), dV, sizeof(int) * r, hipMemcpyDeviceToHost, st));
@@ -5353,7 +5407,7 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
         });
         PT_.end(st);
     }
-    if (targ) check_windows(d_next + 1, st);
+    if (targ) check_windows(d_next + 1, ctx->work.pin + kPinCounts, st);
 }
 
 }  // namespace
