@@ -331,6 +331,11 @@ void erp_ctx_destroy(erp_ctx* ctx) {
     }
     ctx->chirps.clear();
     ctx->bands.clear();
+    for (auto* t : ctx->narrows) {
+        t->tab.release();
+        delete t;
+    }
+    ctx->narrows.clear();
     release_work(ctx->work);
     mt_state_free(ctx->mt);
     ctx->mt = nullptr;

@@ -688,40 +688,6 @@ __global__ void k_band_scale(float2* __restrict__ tab, int n, float sc) {
     if (i < n) tab[i] = make_float2(tab[i].x * sc, tab[i].y * sc);
 }
 
-// Where a row's samples go (the combine step of combineRadarSignals,
-// radar_kernels.cu:302-311): a run's output, or its track's radargram
-struct FinalOut {
-    const float2* refl;
-    const float2* add;
-    const int* Vs;
-    float2* out;
-    int32_t* nvalid;
-    const TrackK* trk;
-    const RowK* rk;
-};
-// false: a padding row of a multi-track batch
-__device__ __forceinline__ bool final_row(const FinalOut& fo, int r, int nr, float2** o,
-                                          const float2** tab) {
-    if (fo.trk) {
-        const RowK row = fo.rk[r];
-        if (row.shot < 0) return false;
-        const TrackK& t = fo.trk[row.trk];
-        *o = t.out + (size_t)row.shot * nr;
-        *tab = t.band;
-        if (t.nvalid && blockIdx.x == 0 && threadIdx.x == 0) t.nvalid[row.shot] = fo.Vs[r];
-    } else {
-        *o = fo.out + (size_t)r * nr;
-        if (fo.nvalid && blockIdx.x == 0 && threadIdx.x == 0) fo.nvalid[r] = fo.Vs[r];
-    }
-    return true;
-}
-__device__ __forceinline__ float2 final_value(const FinalOut& fo, size_t i, bool live, float2 v) {
-    if (!live) return make_float2(0.f, 0.f);
-    if (fo.refl) v = cadd(fo.refl[i], v);
-    if (fo.add) v = cadd(v, fo.add[i]);
-    return v;
-}
-
 // P <= 4096: the whole stage of one row in one workgroup
 __global__ void __launch_bounds__(NT) k_final_small(const float2* __restrict__ S, int P, int log2P,
                                                     int nr, const float2* tab, FinalOut fo,
@@ -1707,10 +1673,7 @@ void surface_conv_rows(erp_ctx* ctx, const FftPlan& p, const double2* srow, int 
     ERP_CHECK_LAUNCH("k_conv_cols_out");
 }
 
-void build_band(erp_ctx* ctx, const FftPlan& p, float2* tab, int nr, float smpl, float B,
-                hipStream_t st) {
-    // the largest kept frequency index of cropSpectrum (elementary_kernels.cu:
-    // 258-278): freq = k smpl / L, kept unless |freq| > B
+int band_limit(int nr, float smpl, float B) {
     const int L = 2 * nr - 1, kmax = L / 2;
     auto kept = [&](int k) {
         return !(std::fabs(((double)k * (double)smpl) / (double)L) > (double)B);
@@ -1719,6 +1682,12 @@ void build_band(erp_ctx* ctx, const FftPlan& p, float2* tab, int nr, float smpl,
     int K = g >= kmax ? kmax : g >= 0.0 ? (int)g : 0;  // (a NaN starts at 0)
     while (K < kmax && kept(K + 1)) ++K;
     while (K >= 0 && !kept(K)) --K;
+    return K;
+}
+
+void build_band(erp_ctx* ctx, const FftPlan& p, float2* tab, int nr, float smpl, float B,
+                hipStream_t st) {
+    const int K = band_limit(nr, smpl, B);
     const int n = 2 * p.N;
     hipLaunchKernelGGL(k_band_gen, dim3((n + 255) / 256), dim3(256), 0, st, tab, p.N, nr, K);
     ERP_CHECK_LAUNCH("k_band_gen");
@@ -1729,12 +1698,9 @@ void build_band(erp_ctx* ctx, const FftPlan& p, float2* tab, int nr, float smpl,
 }
 
 void shot_final_rows(erp_ctx* ctx, const FftPlan& p, float2* S, float2* work, int nr, int rows,
-                     const float2* tab, const float2* refl, const float2* add, const int* Vs,
-                     float2* out, int32_t* nvalid, const TrackK* trk, const RowK* rk,
-                     hipStream_t st) {
+                     const float2* tab, const FinalOut& fo, hipStream_t st) {
     if (rows <= 0) return;
     const float2* tw = ctx->twiddle.as<float2>();
-    const FinalOut fo{refl, add, Vs, out, nvalid, trk, rk};
     if (!p.two_pass) {
         hipLaunchKernelGGL(k_final_small, dim3(1, rows), dim3(NT), 0, st, S, p.N, p.log2N, nr, tab,
                            fo, tw);

@@ -189,6 +189,29 @@ struct BandTables {
     DevBuf tab;
 };
 
+// Narrow-band chain of typed targets (erp_narrow.hip): band, decimation and
+// tables of one (nr, dr, res, smpl, B)
+struct NarrowPlan {
+    int ok;                  // the chain takes this run
+    int nr, K;               // kept frequencies |k| <= K
+    int q, Tq, T;            // decimation, filter half length T = q Tq
+    int iL0, nL, iR0, nR;    // first column and columns (multiples of 16) per part
+    int Nu, nfb;             // all columns; blocks of 16 bins per filter tile
+    double kappa;            // dr / res
+    const float* tab;        // rows of e_k and M_k (k_narrow_table)
+    const float* fir;        // filter operand of k_narrow_fir
+};
+struct NarrowTables {
+    int nr = 0;
+    float dr = 0, res = 0, smpl = 0, B = 0;
+    NarrowPlan plan{};
+    DevBuf tab;
+};
+constexpr int kNarrowSlice = 32;  // pairs per slice
+// entries from one pair row to the next: 256 bytes past a power of two, so
+// that the rows of a slice, read side by side, fall on different channels
+inline int narrow_stride(int P) { return P / 2 + 32; }
+
 // Pinned host words of a run: the counts of a batch (up to kPinCounts: V per
 // shot, U per block of two), the target counts, the window check, then
 // target lists of up to kPinList entries.
@@ -256,9 +279,10 @@ struct erp_ctx {
     std::vector<std::pair<int, DevBuf*>> inter;  // inter-pass twiddles per size
     std::vector<ChirpSpec*> chirps;
     std::vector<BandTables*> bands;
+    std::vector<NarrowTables*> narrows;
     WorkBufs work;
     std::mutex mu;        // serialises the synchronous entry points
-    // guards inter / chirps / bands (shared by all streams); recursive because
+    // guards inter / chirps / bands / narrows (shared by all streams); recursive because
     // building a chirp or band table runs FFTs that look up inter tables
     std::recursive_mutex cache_mu;
     int num_cu = 0;
@@ -328,6 +352,7 @@ void fft_natural_order(const FftPlan& p, const float2* src, float2* dst, hipStre
 // zeros).  work: rows x P, unused by single-pass sizes.
 struct TrackK;
 struct RowK;
+struct FinalOut;
 void surface_conv_rows(erp_ctx* ctx, const FftPlan& p, const double2* srow, int nr, int rows,
                        bool det, const unsigned* smax, const int* Vs, const float2* G,
                        float2* work, float2* out, const TrackK* trk, const RowK* rk,
@@ -336,14 +361,10 @@ void surface_conv_rows(erp_ctx* ctx, const FftPlan& p, const double2* srow, int 
 void build_band(erp_ctx* ctx, const FftPlan& p, float2* tab, int nr, float smpl, float B,
                 hipStream_t st);
 // Last stage of typed targets: each row's summed spectrum S (P, overwritten)
-// -> c = IFFT(S), cropped to the band and decimated, plus refl and add
-// (either may be null), zero where Vs is 0, into out and nvalid (or, with
-// trk, each row's place in its track's radargram).  work: rows x 2P, unused
-// by single-pass sizes.
+// -> c = IFFT(S), cropped to the band and decimated, written as fo says.
+// work: rows x 2P, unused by single-pass sizes.
 void shot_final_rows(erp_ctx* ctx, const FftPlan& p, float2* S, float2* work, int nr, int rows,
-                     const float2* tab, const float2* refl, const float2* add, const int* Vs,
-                     float2* out, int32_t* nvalid, const TrackK* trk, const RowK* rk,
-                     hipStream_t st);
+                     const float2* tab, const FinalOut& fo, hipStream_t st);
 // Specular typed targets of single-pass sizes: prod[p] = FFT(B_p) FFT(z_p),
 // z_p the range-compressed window of A_p, summed per segment into S
 void target_spectra_small(erp_ctx* ctx, const FftPlan& p, const float2* A, const float2* B, int nr,
@@ -411,7 +432,9 @@ struct KPar {
     double B, smpl;
     int nr, P_fft, rerad;
     int row_live;      // entries of a pair row the spectral chain reads: P_fft / 2
-                       // for the per-pair LDS chain, P_fft otherwise
+                       // for the per-pair LDS chain, nr for the narrow-band one,
+                       // P_fft otherwise
+    int row_stride;    // entries from one pair row to the next
     uint32_t mode;
     uint64_t seed;
     int win_shift;     // 0; > 0 only to test the target kernel's window check
@@ -436,11 +459,76 @@ struct TrackK {
     float2* out;                   // the track's radargram, ns x nr (device)
     int32_t* nvalid;               // its illuminated counts (device) or null
     float tscale;                  // -1 / sqrt(P): outward trace of a target
+    NarrowPlan narrow;             // groups of the narrow-band chain
 };
 struct RowK {
     int trk;   // track of the row
     int shot;  // the row's shot index within its track
 };
+
+// Where a row's samples go (the combine step of combineRadarSignals,
+// radar_kernels.cu:302-311): plus refl and add (either may be null), zero
+// where Vs is 0, into a run's out and nvalid or its track's radargram (trk)
+struct FinalOut {
+    const float2* refl;
+    const float2* add;
+    const int* Vs;
+    float2* out;
+    int32_t* nvalid;
+    const TrackK* trk;
+    const RowK* rk;
+};
+// false: a padding row of a multi-track batch
+__device__ __forceinline__ bool final_row(const FinalOut& fo, int r, int nr, float2** o,
+                                          const float2** tab) {
+    if (fo.trk) {
+        const RowK row = fo.rk[r];
+        if (row.shot < 0) return false;
+        const TrackK& t = fo.trk[row.trk];
+        *o = t.out + (size_t)row.shot * nr;
+        *tab = t.band;
+        if (t.nvalid && blockIdx.x == 0 && threadIdx.x == 0) t.nvalid[row.shot] = fo.Vs[r];
+    } else {
+        *o = fo.out + (size_t)r * nr;
+        if (fo.nvalid && blockIdx.x == 0 && threadIdx.x == 0) fo.nvalid[r] = fo.Vs[r];
+    }
+    return true;
+}
+__device__ __forceinline__ float2 final_value(const FinalOut& fo, size_t i, bool live, float2 v) {
+    if (!live) return make_float2(0.f, 0.f);
+    if (fo.refl) v = make_float2(fo.refl[i].x + v.x, fo.refl[i].y + v.y);
+    if (fo.add) v = make_float2(v.x + fo.add[i].x, v.y + fo.add[i].y);
+    return v;
+}
+
+
+// rows of a multi-track batch (trk null: one run)
+struct NarrowMt {
+    const TrackK* trk;
+    const RowK* rk;
+    const int* pshot;  // row of each pair
+};
+// the largest kept frequency index of cropSpectrum (elementary_kernels.cu:
+// 258-278): freq = k smpl / L, kept unless |freq| > B; -1: none
+int band_limit(int nr, float smpl, float B);
+void zero_words(float2* p, size_t n, hipStream_t st);
+// plan of a run (p.ok: the narrow-band chain takes it), its table size, its
+// tables (synchronous on st)
+NarrowPlan narrow_plan(int nr, float dr, float res, float smpl, float B);
+size_t narrow_table_floats(const NarrowPlan& p);
+void narrow_build(NarrowPlan& p, float* tab, hipStream_t st);
+// X_k Z_k summed per slice: part (nslices rows of K + 1 float4) from the
+// pairs' rows of A; Ad: nslices x Nu x 64 floats
+void narrow_pairs(const NarrowPlan& p, const NarrowMt& mt, const float2* A, int P,
+                  const int* pbase, const int* pwin, const int* gb, const int* ge, int nslices,
+                  float* Ad, float4* part, hipStream_t st);
+// each segment's slices into its shot's row of S (rows of K + 1 float4)
+void narrow_sum(const NarrowPlan& p, const NarrowMt& mt, const float4* part, const int* seg_shot,
+                const int* seg_beg, const int* seg_end, int nseg, const float* seg_scale,
+                float scale, float4* S, hipStream_t st);
+// shot_final_rows for these sums
+void narrow_final_rows(const NarrowPlan& p, const float4* S, int rows, const FinalOut& fo,
+                       hipStream_t st);
 
 // Deterministic accumulation: every term is rounded once to a signed 64-bit
 // fixed-point value v * 2^E and summed with integer atomics, which are exact

@@ -38,6 +38,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <tuple>
 
 namespace {
 
@@ -52,9 +53,11 @@ constexpr int TWIN = 4096;     // target LDS window (bins)
 constexpr int NTT = 512;       // threads per workgroup of the target kernels
 // (shot, target) pairs per target launch: their P-point rows take at most
 // kPairRowBytes per buffer set.  Large launches keep the last round of
-// workgroups a small part of each launch and need fewer host round trips.
+// workgroups a small part of each launch and need fewer host round trips:
+// 32768 pairs rather than 16384 give the narrow-band chain's short workgroups
+// 10 % (4096 bins, 16.1 to 14.5 ms per 7e5 pairs).
 constexpr int64_t kPairRowBytes = (int64_t)6144 << 20;
-constexpr int kMaxPairsPerLaunch = 16384;
+constexpr int kMaxPairsPerLaunch = 32768;
 // Shots per batch (default and maximum).  Each batch waits on the host a
 // few times (illuminated counts, target counts and lists), so a 50-shot
 // step runs as one batch rather than two.
@@ -2389,7 +2392,7 @@ k_target_accum_fast(const float* __restrict__ tg0, int64_t Tpad0, const int* __r
         const float tnx = tg[3 * Tpad + t], tny = tg[4 * Tpad + t], tnz = tg[5 * Tpad + t];
         const double tx = txf, ty = tyf, tz = tzf;
         const double rst = (double)sh.rst;
-        const int nr = kp.nr, P = kp.P_fft;
+        const int nr = kp.nr;
         const bool lossless = kp.mode & ERP_MODE_LOSSLESS;
 
         // second medium: a uniform flag per pair
@@ -2407,7 +2410,7 @@ k_target_accum_fast(const float* __restrict__ tg0, int64_t Tpad0, const int* __r
             pbase[pi] = fits ? base : -1;
             pwin[pi] = len;
         }
-        float2* rowA = outA + (size_t)pi * P;
+        float2* rowA = outA + (size_t)pi * kp.row_stride;
         // out-of-window terms: counted as broken bounds where the window
         // covers every bin the bounds allow (deterministic: always, so no
         // float atomic can reach the row)
@@ -2807,7 +2810,7 @@ k_target_accum_pair(const float* __restrict__ tg0, int64_t Tpad0, const int4* __
             len[k] = pw.len;
             top[k] = pw.top;
             fits[k] = pw.fits;
-            rowp[k] = outA + (size_t)row[k] * kp.P_fft;
+            rowp[k] = outA + (size_t)row[k] * kp.row_stride;
             // out-of-window terms of a pair whose window covers its bounds
             // (deterministic: of every pair) are broken bounds (counted);
             // the others go to the row
@@ -3380,7 +3383,7 @@ KPar make_kpar(const erp_params& p, int P_fft) {
     k.smpl = p.smpl;
     k.nr = p.nr;
     k.P_fft = P_fft;
-    k.row_live = P_fft;
+    k.row_live = k.row_stride = P_fft;
     k.rerad = p.rerad_funct;
     k.mode = p.mode;
     k.seed = p.seed;
@@ -3462,15 +3465,51 @@ const float2* get_band(erp_ctx* ctx, int nr, float smpl, float B, const FftPlan&
     b->B = B;
     b->tab.ensure(sizeof(float2) * 2 * (size_t)plan.N);
     build_band(ctx, plan, b->tab.as<float2>(), nr, smpl, B, st);
-    if (ctx->bands.size() > 8 && ctx->active.load() == 0) {
-        ERP_HIP_TRY(hipStreamSynchronize(st));
-        ctx->bands.front()->tab.release();
-        delete ctx->bands.front();
-        ctx->bands.erase(ctx->bands.begin());
-    }
     ctx->bands.push_back(b);
     ERP_HIP_TRY(hipStreamSynchronize(st));
     return b->tab.as<float2>();
+}
+
+// plan and tables of the narrow-band chain, cached per context
+NarrowPlan get_narrow(erp_ctx* ctx, const NarrowPlan& plan, float dr, float res, float smpl,
+                      float B, hipStream_t st) {
+    std::lock_guard<std::recursive_mutex> lk(ctx->cache_mu);
+    for (NarrowTables* t : ctx->narrows)
+        if (t->nr == plan.nr && t->dr == dr && t->res == res && t->smpl == smpl && t->B == B)
+            return t->plan;
+    NarrowTables* t = new NarrowTables();
+    t->nr = plan.nr;
+    t->dr = dr;
+    t->res = res;
+    t->smpl = smpl;
+    t->B = B;
+    t->plan = plan;
+    try {
+        t->tab.ensure(sizeof(float) * narrow_table_floats(plan));
+        narrow_build(t->plan, t->tab.as<float>(), st);
+    } catch (...) {
+        t->tab.release();
+        delete t;
+        throw;
+    }
+    ctx->narrows.push_back(t);
+    return t->plan;
+}
+
+// Drops the oldest tables past 8 of each kind.  Called where a synchronous
+// run begins: it holds no pointer yet, and no asynchronous job is active.
+void trim_tables(erp_ctx* ctx) {
+    std::lock_guard<std::recursive_mutex> lk(ctx->cache_mu);
+    if (ctx->active.load() != 0) return;
+    auto trim = [](auto& v) {
+        while (v.size() > 8) {
+            v.front()->tab.release();  // hipFree waits for the device
+            delete v.front();
+            v.erase(v.begin());
+        }
+    };
+    trim(ctx->bands);
+    trim(ctx->narrows);
 }
 
 void zero(float2* p, size_t n, hipStream_t st) {
@@ -3878,6 +3917,8 @@ TargetAccumFn pick_target_accum(bool det, int ph, int acc, bool s3) {
     }
 }
 
+void zero_words(float2* p, size_t n, hipStream_t st) { zero(p, n, st); }
+
 // Device bytes of one run, following the allocations of erp_run_impl: the
 // work buffers of one batch of up to kShotsPerBatch shots (facet records counted for
 // every facet illuminated by every shot of the batch, an upper bound) plus
@@ -3903,6 +3944,8 @@ int64_t erp_footprint_impl(const erp_params* par, int64_t F, int64_t T, int64_t 
         b += S * T * 8 + S * 8;               // target lists and counts
         b += S * nblk * 32;                   // facet block boxes (bounding spheres)
         b += P * 8 * (C * nbuf + gcap);       // per-target chunk rows and partial sums
+        const NarrowPlan nar = narrow_plan((int)nr, par->dr, 2.f * par->rng_res, par->smpl, par->B);
+        if (!spec && nar.ok) b += 4 * (int64_t)narrow_table_floats(nar);
         b += 4 * (C * 4 + 2 * gcap + 3 * S + 16);
     }
     b += ns * nr * 8 + ns * 4;                // the radargram and the counts
@@ -3941,6 +3984,7 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
         throw ErpError{ERP_E_UNSUPPORTED,
                        "non-specular runs need convolution and convolution_linear "
                        "(sim.cu:431-439,778 otherwise write past the chirp buffer)"};
+    if (!arena) trim_tables(ctx);
     const int64_t F = mesh->F;
     const int64_t T = targets ? targets->T : 0;
     const bool any_t0 = T > 0 && targets->n0 > 0, any_typed = T > 0 && targets->n0 < T;
@@ -3997,7 +4041,6 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
     const float2* g_surf = nullptr;
     if (!spec || (conv && lin)) g_surf = chirp(p.rng_res, 0);
     const float2* g_targ = nullptr;
-    if (T > 0 && conv && lin) g_targ = chirp(res_t, 0);
     // plain mode: per-pair spectral chain in one workgroup when P / 2 fits
     // LDS (nr below P / 2: its cropped variant, whose range kernel has the
     // kept window at P / 2 and whose rows are read up to P / 2)
@@ -4005,14 +4048,35 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
     kp.row_live = half ? P / 2 : P;
     // the per-pair chain's spectrum: natural, or in the wave-local layout
     const bool wl = half && target_wl(planP);
-    const float2* g_targ_nat = half ? chirp(res_t, wl ? 2 : 1, nr < P / 2 ? 2 : 0) : nullptr;
+    // a narrow band: the decimated chain instead.  Deterministic runs keep the
+    // transforms, so that their bits do not depend on the room for its tables
+    // (an allocation-free run gives them at most a sixteenth of its region).
+    NarrowPlan nar{};
+    if (half && any_typed && !det) nar = narrow_plan(nr, p.dr, res_t, p.smpl, p.B);
+    if (nar.ok && arena && sizeof(float) * narrow_table_floats(nar) > arena->left() / 16)
+        nar.ok = 0;
+    if (nar.ok && arena)
+        narrow_build(nar, arena->take_n<float>(narrow_table_floats(nar), "narrow-band tables"), st);
+    else if (nar.ok)
+        nar = get_narrow(ctx, nar, p.dr, res_t, p.smpl, p.B, st);
+    const bool nb = nar.ok;
+    if (nb) {
+        kp.row_live = nr;
+        kp.row_stride = narrow_stride(P);
+    }
+    const NarrowMt nomt{nullptr, nullptr, nullptr};
+    // complex64 per shot of the summed spectrum
+    const size_t sumP = nb ? 2 * ((size_t)nar.K + 1) : (size_t)P;
+    const float2* g_targ_nat =
+        half && !nb ? chirp(res_t, wl ? 2 : 1, nr < P / 2 ? 2 : 0) : nullptr;
+    if (T > 0 && conv && lin && (!half || any_t0)) g_targ = chirp(res_t, 0);
     // circular convolution of type-0 targets: one genChirp table per rx window
     // start; with an arena one table is rebuilt for each shot
     float2* g_circ = (arena && any_t0 && conv && !lin)
                          ? arena->take_n<float2>((size_t)P, "circular chirp spectrum")
                          : nullptr;
     const float2* band = nullptr;
-    if (any_typed) {
+    if (any_typed && !nb) {
         if (arena) {
             float2* tab = arena->take_n<float2>(2 * (size_t)P, "band tables");
             build_band(ctx, planP, tab, nr, p.smpl, p.B, st);
@@ -4031,7 +4095,7 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
     // (shot, target) pairs per target launch and the per-pair buffer layout
     const bool fused = !spec && !half && (!planP.two_pass || nr % planP.N1 == 0);
     // pairs per multiply-accumulate group (fused) or per summed slice (half)
-    const int GS = half ? target_half_slice() : 16;
+    const int GS = nb ? kNarrowSlice : half ? target_half_slice() : 16;
     const int nbuf = half ? 2 : (fused ? 3 : (spec ? 4 : 3));
     int C = (int)std::max<int64_t>(1, kPairRowBytes / ((int64_t)P * 8 * nbuf));
     C = std::min<int>(C, kMaxPairsPerLaunch);
@@ -4054,6 +4118,17 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
             b += Arena::round(cap * 48) + 2 * Arena::round(cap * 4) + Arena::round(cap * 12);
         if (!spec && any_typed) b += 3 * Arena::round(cap * 16) + Arena::round(cap * 4);
         return b;
+    };
+    // pair rows and slice sums; per-pair products (the narrow-band chain:
+    // decimated rows per slice) of launches of C pairs in at most gc slices
+    auto pair_bytes = [&](int C_, size_t gc) -> size_t {
+        const size_t rows = sizeof(float2) * (size_t)kp.row_stride * (size_t)C_ * (nbuf - 1);
+        return rows + gc * (nb ? sizeof(float4) * ((size_t)nar.K + 1)
+                               : half ? sizeof(float2) * (size_t)P : 0);
+    };
+    auto prod_bytes = [&](int C_, size_t gc) -> size_t {
+        return nb ? sizeof(float) * gc * nar.Nu * 2 * kNarrowSlice
+                  : sizeof(float2) * (size_t)C_ * P;
     };
     // upload of one launch of the shot-pair kernel: 16 bytes for its item
     // counter, the slices and segments, then the items
@@ -4087,8 +4162,8 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
             buf(W.refl, sizeof(float2) * s * nr, "reflected traces");
             if (any_t0) buf(W.out, sizeof(float2) * s * nr, "refracted traces");
             if (any_typed) {
-                buf(W.shotS, sizeof(float2) * s * P, "spectral sums");
-                buf(W.blu, sizeof(float2) * s * 2 * P, "band crop rows");
+                buf(W.shotS, sizeof(float2) * s * sumP, "spectral sums");
+                if (!nb) buf(W.blu, sizeof(float2) * s * 2 * P, "band crop rows");
             }
             if (any_t0) buf(W.t0trace, sizeof(float2) * s * P, "type-0 traces");
             if (spec && !conv)
@@ -4101,9 +4176,8 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
             size_t pb = 0;
             if (any_typed) {
                 const size_t gc = (size_t)C_ / GS + s + 2;
-                buf(W.tA, sizeof(float2) * (size_t)P * ((size_t)C_ * (nbuf - 1) + (half ? gc : 0)),
-                    "pair rows");
-                buf(W.tC, sizeof(float2) * (size_t)C_ * P, "pair products");
+                buf(W.tA, pair_bytes(C_, gc), "pair rows");
+                buf(W.tC, prod_bytes(C_, gc), "pair products");
                 pb = sizeof(int) * ((size_t)C_ * 4 + 2 * gc + 3 * s + 16);
             }
             if (any_t0) pb = std::max(pb, sizeof(int) * 2 * s * (size_t)T + 64);
@@ -4156,8 +4230,8 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
     W.refl.ensure(sizeof(float2) * (size_t)Smax * nr);
     if (any_t0) W.out.ensure(sizeof(float2) * (size_t)Smax * nr);  // type-0 targets
     if (any_typed) {
-        W.shotS.ensure(sizeof(float2) * (size_t)Smax * P);
-        W.blu.ensure(sizeof(float2) * (size_t)Smax * 2 * P);
+        W.shotS.ensure(sizeof(float2) * (size_t)Smax * sumP);
+        if (!nb) W.blu.ensure(sizeof(float2) * (size_t)Smax * 2 * P);
     }
     if (any_t0) W.t0trace.ensure(sizeof(float2) * (size_t)Smax * P);
     if (spec && !conv)
@@ -4349,7 +4423,7 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
 
         // 3: fused surface kernel
         {
-            const size_t n0 = do_trace ? srow_f2 : 0, n1 = any_typed ? (size_t)S * P : 0,
+            const size_t n0 = do_trace ? srow_f2 : 0, n1 = any_typed ? (size_t)S * sumP : 0,
                          ni = brk.rec.itd ? 2 * ucap : 0;
             hipLaunchKernelGGL(k_batch_prep, dim3(grid_for(n0 + n1 + ni, 256, 4096)), dim3(256), 0,
                                st, (const int*)dV, (const int*)dU, S, need_rec ? dbase : nullptr,
@@ -4471,9 +4545,8 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
                 float2* Sacc = W.shotS.as<float2>();  // cleared by k_batch_prep
                 const size_t gcap = (size_t)C / GS + S + 2;
                 // half: A rows, then one partial row per slice
-                W.tA.ensure(sizeof(float2) * (size_t)P *
-                            ((size_t)C * (nbuf - 1) + (half ? gcap : 0)));
-                W.tC.ensure(sizeof(float2) * (size_t)C * P);
+                W.tA.ensure(pair_bytes(C, gcap));
+                W.tC.ensure(prod_bytes(C, gcap));
                 float2* A = W.tA.as<float2>();
                 float2* Bq = A + (size_t)C * P;                 // y / Y' (and MODE 1: B)
                 float2* Bs = spec ? Bq + (size_t)C * P : nullptr;
@@ -4488,6 +4561,26 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
                 int* dge = dgb + gcap;
                 int* dseg = dge + gcap;              // segment shot / begin / end
                 int* dpw = dseg + 3 * S;             // per-pair window length (fused)
+                // the pairs' chain and their sums (in the stage PT_ has begun)
+                auto chain = [&](const int* gb_, const int* ge_, int ngroups, const int* ss,
+                                 const int* sb, const int* se, int nseg, int n) {
+                    float2* sums = A + (size_t)C * kp.row_stride;
+                    const float sc = -1.0f / kp.sqrtP;  // outward trace = -A / sqrt(P)
+                    if (nb)
+                        narrow_pairs(nar, nomt, A, kp.row_stride, dpb, dpw, gb_, ge_, ngroups, W.tC.as<float>(),
+                                     reinterpret_cast<float4*>(sums), st);
+                    else
+                        target_pairs_half(ctx, planP, A, dpb, dpw, nr, n, g_targ_nat, Z, st);
+                    PT_.end(st);
+                    PT_.begin(ERP_STAGE_TARGET_SUM, st, (double)n);
+                    if (nb)
+                        narrow_sum(nar, nomt, reinterpret_cast<float4*>(sums), ss, sb, se, nseg,
+                                   nullptr, sc, reinterpret_cast<float4*>(Sacc), st);
+                    else
+                        target_sum_half(planP, Z, sums, gb_, ge_, ngroups, ss, sb, se, nseg, Sacc,
+                                        sc, st, nullptr, det, wl);
+                    PT_.end(st);
+                };
                 if (pairk) {
                     // the shot-pair kernel: items of a target and two
                     // consecutive shots, from the shots' target lists
@@ -4552,14 +4645,8 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
                         ERP_CHECK_LAUNCH("k_target_accum_pair");
                         PT_.end(st);
                         PT_.begin(ERP_STAGE_TARGET_FFT, st, (double)n);
-                        target_pairs_half(ctx, planP, A, dpb, dpw, nr, n, g_targ_nat, Z, st);
-                        PT_.end(st);
-                        PT_.begin(ERP_STAGE_TARGET_SUM, st, (double)n);
                         int* sg = dsl + 2 * gcap;
-                        target_sum_half(planP, Z, A + (size_t)C * P, dsl, dsl + gcap, ngroups, sg,
-                                        sg + S, sg + 2 * S, nseg, Sacc, -1.0f / kp.sqrtP, st,
-                                        nullptr, det, wl);
-                        PT_.end(st);
+                        chain(dsl, dsl + gcap, ngroups, sg, sg + S, sg + 2 * S, nseg, n);
                     }
                 }
                 // iterate pairs in (shot, target) order
@@ -4625,14 +4712,7 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
                     PT_.end(st);
                     PT_.begin(ERP_STAGE_TARGET_FFT, st, (double)n);
                     if (half) {
-                        // outward trace = -A/sqrt(P): scale -1/sqrt(P)
-                        target_pairs_half(ctx, planP, A, dpb, dpw, nr, n, g_targ_nat, Z, st);
-                        PT_.end(st);
-                        PT_.begin(ERP_STAGE_TARGET_SUM, st, (double)n);
-                        target_sum_half(planP, Z, A + (size_t)C * P, dgb, dge, ngroups, dseg,
-                                        dseg + S, dseg + 2 * S, nseg, Sacc, -1.0f / kp.sqrtP, st,
-                                        nullptr, det, wl);
-                        PT_.end(st);
+                        chain(dgb, dge, ngroups, dseg, dseg + S, dseg + 2 * S, nseg, n);
                         continue;
                     }
                     if (fused) {
@@ -4770,9 +4850,11 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
         const float2* r0 = have_refr0 ? refr0 : nullptr;
         if (have_refr) {
             PT_.begin(ERP_STAGE_SHOT_FINAL, st, (double)S);
-            shot_final_rows(ctx, planP, W.shotS.as<float2>(), W.blu.as<float2>(), nr, S, band,
-                            have_refl ? refl : nullptr, r0, dV, out_dev + (size_t)s0 * nr, nv,
-                            nullptr, nullptr, st);
+            const FinalOut fo{have_refl ? refl : nullptr, r0, dV, out_dev + (size_t)s0 * nr, nv,
+                              nullptr, nullptr};
+            if (nb) narrow_final_rows(nar, W.shotS.as<float4>(), S, fo, st);
+            else shot_final_rows(ctx, planP, W.shotS.as<float2>(), W.blu.as<float2>(), nr, S, band,
+                                 fo, st);
             PT_.end(st);
         } else {
             hipLaunchKernelGGL(k_finalize, dim3(grid_for((size_t)nr * S)), dim3(256), 0, st,
@@ -4809,11 +4891,12 @@ namespace {
 struct MtKey {
     int R = 0, nblk = 0, nr = 0, Tcap = 0, C = 0, ntrk = 0;
     size_t reccap = 0;
+    int nu = 0, nk = 0;  // columns and frequencies of the narrow-band chain
     bool det = false, s3 = false, targ = false, pair = false;
     bool operator==(const MtKey& o) const {
         return R == o.R && nblk == o.nblk && nr == o.nr && Tcap == o.Tcap && C == o.C &&
                ntrk == o.ntrk && reccap == o.reccap && det == o.det && s3 == o.s3 &&
-               targ == o.targ && pair == o.pair;
+               targ == o.targ && pair == o.pair && nu == o.nu && nk == o.nk;
     }
 };
 
@@ -4908,10 +4991,16 @@ bool mt_eligible(const erp_track& t, uint32_t flags) {
     return true;
 }
 
+// the narrow-band chain's plan of a track, as a run of its own would take it
+NarrowPlan mt_narrow(const erp_track& t, bool det) {
+    const erp_params& p = *t.par;
+    return det ? NarrowPlan{} : narrow_plan(p.nr, p.dr, 2.f * p.rng_res, p.smpl, p.B);
+}
+
 // one group: tracks trk_idx of range length nr, all with (s3) or all
-// without the second subsurface medium
+// without the second subsurface medium, all or none of the narrow-band chain
 void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64_t>& trk_idx,
-                  int nr, bool s3, bool det, hipStream_t st) {
+                  int nr, bool s3, bool narrow, bool det, hipStream_t st) {
     const int P = next_pow2(2 * (int64_t)nr - 1);
     const FftPlan planP = fft_plan(P);
     if (!target_half_supported(planP, nr))
@@ -4933,7 +5022,8 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
         d.kp = make_kpar(p, P);
         d.kp.ortho = mesh->frame_ok ? 1 : 0;
         d.kp.win_shift = (int)ctx->tune_shift;
-        d.kp.row_live = P / 2;
+        d.kp.row_live = narrow ? nr : P / 2;
+        d.kp.row_stride = narrow ? narrow_stride(P) : P;
         d.mesh = mesh->soa.as<float>();
         d.Fpad = mesh->Fpad;
         d.F = mesh->F;
@@ -4947,8 +5037,9 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
             d.Tpad = t.targets->Tpad;
             d.ttype = t.targets->type.as<unsigned char>();
             // sim.cu:853-858: the target range kernel has twice the surface's
-            d.g_targ_nat = get_chirp(ctx, nr, p.dr, 2.f * p.rng_res, tkind, 0.f, P, planP, st,
-                                     target_wl(planP) ? 2 : 1);
+            if (!narrow)
+                d.g_targ_nat = get_chirp(ctx, nr, p.dr, 2.f * p.rng_res, tkind, 0.f, P, planP, st,
+                                         target_wl(planP) ? 2 : 1);
             targ = true;
         }
         // a disabled surface echo: no spectrum, so the row's echo is zero
@@ -4963,18 +5054,31 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
         nrows += t.ns;
     }
 
-    // band tables of every track once any has targets: the tail runs over all
-    // rows of a batch (a row without targets crops a zero sum)
+    // band tables (or the narrow-band chain's) of every track once any has
+    // targets: the tail runs over all rows of a batch (a row without targets
+    // crops a zero sum).  nar: the launches' bounds; rows read their own plan.
+    NarrowPlan nar{};
     if (targ)
         for (int k = 0; k < ntr; ++k) {
-            const erp_params& p = *tracks[trk_idx[k]].par;
-            tk[k].band = get_band(ctx, nr, p.smpl, p.B, planP, st);
+            const erp_track& t = tracks[trk_idx[k]];
+            const erp_params& p = *t.par;
+            if (!narrow) {
+                tk[k].band = get_band(ctx, nr, p.smpl, p.B, planP, st);
+                continue;
+            }
+            tk[k].narrow = get_narrow(ctx, mt_narrow(t, det), p.dr, 2.f * p.rng_res, p.smpl, p.B,
+                                      st);
+            nar.nr = nr;
+            nar.Nu = std::max(nar.Nu, tk[k].narrow.Nu);
+            nar.K = std::max(nar.K, tk[k].narrow.K);
         }
+    const size_t sumP = narrow ? 2 * ((size_t)nar.K + 1) : (size_t)P;
+    const int rowP = narrow ? narrow_stride(P) : P;
 
     // shapes
     int R = kMtRowsDefault;
     if (ctx->tune_rows > 0) R = (int)std::min<int64_t>(ctx->tune_rows, kMtRowsMax);
-    const int GS = target_half_slice();
+    const int GS = narrow ? kNarrowSlice : target_half_slice();
     int C = (int)std::max<int64_t>(1, kPairRowBytes / ((int64_t)P * 8 * 2));
     C = std::min<int>(C, kMaxPairsPerLaunch);
     if (ctx->tune_pairs > 0) C = (int)std::min<int64_t>(C, ctx->tune_pairs);
@@ -4996,6 +5100,7 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
     MtKey key;
     key.R = R; key.nblk = nblk_max; key.nr = nr; key.Tcap = Tcap; key.C = C; key.ntrk = ntr;
     key.reccap = m.key.reccap; key.det = det; key.s3 = s3; key.targ = targ; key.pair = pairk;
+    key.nu = nar.Nu; key.nk = nar.K;
     if (!(key == m.key)) {
         m.reset_graphs();
         m.key = key;
@@ -5015,13 +5120,15 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
     m.srow.ensure(sizeof(float2) * srow_f2);
     m.refl.ensure(sizeof(float2) * r * nr);
     if (targ) {
-        m.Sacc.ensure(sizeof(float2) * r * P);
-        m.blu.ensure(sizeof(float2) * r * 2 * P);
+        m.Sacc.ensure(sizeof(float2) * r * sumP);
+        if (!narrow) m.blu.ensure(sizeof(float2) * r * 2 * P);
         m.list.ensure(sizeof(int) * r * (size_t)Tcap * 2);
         m.tcnt.ensure(sizeof(int) * r * 2);
         m.bbox.ensure(sizeof(float4) * 2 * r * nblk_max);
-        m.A.ensure(sizeof(float2) * (size_t)P * ((size_t)C + gcap));  // pair rows, slice sums
-        m.Z.ensure(sizeof(float2) * (size_t)P * C);                   // per-pair products
+        // pair rows, slice sums; per-pair products (narrow: decimated slices)
+        m.A.ensure(sizeof(float2) * ((size_t)rowP * C + (size_t)gcap * sumP));
+        m.Z.ensure(narrow ? sizeof(float) * (size_t)gcap * nar.Nu * 2 * kNarrowSlice
+                          : sizeof(float2) * (size_t)P * C);
     }
     // host-written tables of a launch: pair rows and list indices, slices,
     // segments, the pair count, segment scales
@@ -5250,7 +5357,7 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
                                    (const unsigned char*)nullptr, dshots, dV, 0.0, list1, list0,
                                    m.tcnt.as<int>(), Tcap, dtrk, drows);
                 ERP_CHECK_LAUNCH("k_target_select");
-                zero(m.Sacc.as<float2>(), r * P, st);
+                zero(m.Sacc.as<float2>(), r * sumP, st);
             } else {
                 hipLaunchKernelGGL(k_finalize_rows, dim3(grid_for(r * nr)), dim3(256), 0, st,
                                    m.refl.as<float2>(), dV, nr, R, dtrk, drows);
@@ -5267,6 +5374,21 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
 
         float2* A = m.A.as<float2>();
         float2* Z = m.Z.as<float2>();
+        // the pairs' chain and their sums
+        auto chain = [&] {
+            float2* sums = A + (size_t)C * rowP;
+            if (narrow) {
+                const NarrowMt mt{dtrk, drows, t_pshot};
+                narrow_pairs(nar, mt, A, rowP, d_pbase, d_pwin, t_slb, t_sle, gcap, m.Z.as<float>(),
+                             reinterpret_cast<float4*>(sums), st);
+                narrow_sum(nar, mt, reinterpret_cast<float4*>(sums), t_sgs, t_sgb, t_sge, segcap,
+                           t_scale, 1.0f, m.Sacc.as<float4>(), st);
+                return;
+            }
+            target_pairs_half(ctx, planP, A, d_pbase, d_pwin, nr, C, nullptr, Z, st, d_G, t_n);
+            target_sum_half(planP, Z, sums, t_slb, t_sle, gcap, t_sgs, t_sgb, t_sge, segcap,
+                            m.Sacc.as<float2>(), 1.0f, st, t_scale, det, target_wl(planP));
+        };
         if (pairk) {
             // shot-pair kernel: items of a target and a block's two rows, from
             // the rows' target lists; launches of whole items of at most C rows
@@ -5337,11 +5459,7 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
                                        d_next + 1, dtrk, drows, (const int*)d_nitems,
                                        (const int*)dV);
                     ERP_CHECK_LAUNCH("k_target_accum_pair");
-                    target_pairs_half(ctx, planP, A, d_pbase, d_pwin, nr, C, nullptr, Z, st, d_G,
-                                      t_n);
-                    target_sum_half(planP, Z, A + (size_t)C * P, t_slb, t_sle, gcap, t_sgs, t_sgb,
-                                    t_sge, segcap, m.Sacc.as<float2>(), 1.0f, st, t_scale, det,
-                                    target_wl(planP));
+                    chain();
                 });
                 PT_.end(st);
             }
@@ -5390,11 +5508,7 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
                                    (const erp_prism*)nullptr, 0, kp0, A, d_pbase, d_pwin, 0, 0,
                                    d_next, dtrk, drows, (const int*)t_n, d_next + 1);
                 ERP_CHECK_LAUNCH("k_target_accum_fast");
-                target_pairs_half(ctx, planP, A, d_pbase, d_pwin, nr, C, nullptr, Z, st, d_G,
-                                  t_n);
-                target_sum_half(planP, Z, A + (size_t)C * P, t_slb, t_sle, gcap, t_sgs, t_sgb,
-                                t_sge, segcap, m.Sacc.as<float2>(), 1.0f, st, t_scale, det,
-                                target_wl(planP));
+                chain();
             });
             PT_.end(st);
         }
@@ -5402,8 +5516,10 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
         // tail: each row's band crop, plus its echo, into the track's radargram
         PT_.begin(ERP_STAGE_SHOT_FINAL, st, (double)nb);
         mt_launch(m.gTail, direct, st, [&] {
-            shot_final_rows(ctx, planP, m.Sacc.as<float2>(), m.blu.as<float2>(), nr, R, nullptr,
-                            m.refl.as<float2>(), nullptr, dV, nullptr, nullptr, dtrk, drows, st);
+            const FinalOut fo{m.refl.as<float2>(), nullptr, dV, nullptr, nullptr, dtrk, drows};
+            if (narrow) narrow_final_rows(nar, m.Sacc.as<float4>(), R, fo, st);
+            else shot_final_rows(ctx, planP, m.Sacc.as<float2>(), m.blu.as<float2>(), nr, R,
+                                 nullptr, fo, st);
         });
         PT_.end(st);
     }
@@ -5418,8 +5534,10 @@ void erp_run_tracks_impl(erp_ctx* ctx, const erp_track* tracks, int64_t ntracks,
                            ERP_RUN_PHASE_DF | ERP_RUN_ACC_F32 | ERP_RUN_ACC_COMP;
     if (flags & ~known) throw ErpError{ERP_E_INVALID, "unknown run flags"};
     const bool det = flags & ERP_RUN_DETERMINISTIC;
-    // groups of one range length and second-medium setting, in track order
-    std::vector<std::pair<std::pair<int, bool>, std::vector<int64_t>>> groups;
+    trim_tables(ctx);
+    // groups of one range length, second-medium setting and spectral chain,
+    // in track order
+    std::vector<std::pair<std::tuple<int, bool, bool>, std::vector<int64_t>>> groups;
     std::vector<int64_t> solo;
     for (int64_t i = 0; i < ntracks; ++i) {
         const erp_track& t = tracks[i];
@@ -5427,7 +5545,8 @@ void erp_run_tracks_impl(erp_ctx* ctx, const erp_track* tracks, int64_t ntracks,
             solo.push_back(i);
             continue;
         }
-        const std::pair<int, bool> gk{t.par->nr, t.par->eps_3 > 0.f};
+        const std::tuple<int, bool, bool> gk{t.par->nr, t.par->eps_3 > 0.f,
+                                             mt_narrow(t, det).ok != 0};
         auto it = std::find_if(groups.begin(), groups.end(),
                                [&](const auto& g) { return g.first == gk; });
         if (it == groups.end()) groups.push_back({gk, {i}});
@@ -5439,6 +5558,7 @@ void erp_run_tracks_impl(erp_ctx* ctx, const erp_track* tracks, int64_t ntracks,
                      static_cast<float2*>(t.out_dev), static_cast<int32_t*>(t.nvalid_dev), flags,
                      st, ctx->work, &ctx->prof);
     }
-    for (const auto& g : groups) mt_run_group(ctx, tracks, g.second, g.first.first, g.first.second,
-                                              det, st);
+    for (const auto& g : groups)
+        mt_run_group(ctx, tracks, g.second, std::get<0>(g.first), std::get<1>(g.first),
+                     std::get<2>(g.first), det, st);
 }
