@@ -2078,7 +2078,7 @@ __device__ __forceinline__ RecV load_rec(const RecShot& rs, unsigned k) {
 // the interface z = zi, so part of each facet's forced ray runs in eps_3
 // (a uniform flag per pair).
 struct Strat {
-    bool deep;
+    int deep;
     double zi, tz, dn;
     float tsq;
 };
@@ -2606,9 +2606,9 @@ __device__ __forceinline__ BRecV load_brec(const BRecBlk& rb, unsigned u) {
 }
 
 template <bool S3>
-__device__ __forceinline__ TLeg tri_leg(const BRecV& rv, bool frame_ok, double tx, double ty,
-                                        double tz, float tnx, float tny, float tnz, bool tn_up,
-                                        bool lossless, const erp_prism* __restrict__ prisms,
+__device__ __forceinline__ TLeg tri_leg(const BRecV& rv, int frame_ok, double tx, double ty,
+                                        double tz, float tnx, float tny, float tnz, int tn_up,
+                                        int lossless, const erp_prism* __restrict__ prisms,
                                         int np, const KPar& kp, const Strat& st) {
     TLeg o;
     const float fx = rv.qa.x, fy = rv.qa.y, fz = rv.qa.z;
@@ -2629,24 +2629,6 @@ __device__ __forceinline__ TLeg tri_leg(const BRecV& rv, bool frame_ok, double t
     const double invd = rd * fma(-y0, hr, 1.5);
     const double ix = dx * invd, iy = dy * invd, iz = dz * invd;
     const float Ix = (float)ix, Iy = (float)iy, Iz = (float)iz;
-    const float2 csT = cos_sin_hw(ix, iy, iz, nx, ny, nz);
-    const float cT = csT.x, sT = csT.y;
-    float Iu = Ix * ux + Iy * uy + Iz * uz;
-    float Iv = Ix * vx + Iy * vy + Iz * vz;
-    if (!frame_ok) {
-        const float2 e = uv_dots_exact(ix, iy, iz, ux, uy, uz, vx, vy, vz);
-        Iu = e.x;
-        Iv = e.y;
-    }
-    const float sTT = tn_up ? __builtin_amdgcn_sqrtf(fmaxf(0.f, (float)((1.0 + iz) * (1.0 - iz))))
-                            : cos_sin_hw(ix, iy, iz, tnx, tny, tnz).y;
-    // azimuth (cos Tph, sin Tph) = (Iv, Iu) / |(Iu, Iv)|, (1, 0) below 1e-30
-    // (where every sinc argument is < 1e-6 whatever the azimuth)
-    const float q2 = Iu * Iu + Iv * Iv;
-    const bool az = q2 > 1e-30f;
-    const float rinv = az ? __builtin_amdgcn_rsqf(q2) : 0.f;
-    const float cph = az ? Iv * rinv : 1.f;
-    const float sph = Iu * rinv;
     // pi-sincs from half their arguments h = x / 2 in revolutions, where the
     // hardware sine's own reduction is as accurate as an explicit one
     // (1.2e-7 absolute up to |h| = 260, checked against double on gfx950;
@@ -2660,10 +2642,34 @@ __device__ __forceinline__ TLeg tri_leg(const BRecV& rv, bool frame_ok, double t
         *num = __builtin_amdgcn_sinf(ha);
         *den = ha;
     };
-    pisinc_h(a * (sT * cph), &n1, &d1);
-    pisinc_h(a * (sT * sph), &n2, &d2);
-    pisinc_h(a * sTT * cph, &n3, &d3);
-    pisinc_h(a * sTT * sph, &n4, &d4);
+    // cosine and sine of the facet's angle (cos_sin_hw with its clamp on the
+    // rounded product, one instruction for two)
+    const double cn = -(ix * nx + iy * ny + iz * nz);
+    const float cT = (float)cn;
+    const float sT = __builtin_amdgcn_sqrtf(fmaxf(0.f, (float)((1.0 - cn) * (1.0 + cn))));
+    float Iu = Ix * ux + Iy * uy + Iz * uz;
+    float Iv = Ix * vx + Iy * vy + Iz * vz;
+    if (!frame_ok) {
+        const float2 e = uv_dots_exact(ix, iy, iz, ux, uy, uz, vx, vy, vz);
+        Iu = e.x;
+        Iv = e.y;
+    }
+    // (sin from (Iu, Iv) themselves would save its root, but the reference's
+    // sine is that of the rounded normal, which near the facet's axis differs
+    // by up to 3e-6: 1e-5 of the strongest terms)
+    const float sTT = tn_up ? __builtin_amdgcn_sqrtf(Ix * Ix + Iy * Iy)
+                            : cos_sin_hw(ix, iy, iz, tnx, tny, tnz).y;
+    // azimuth (cos Tph, sin Tph) = (Iv, Iu) / |(Iu, Iv)|, (1, 0) below 1e-30
+    // (where every sinc argument is < 1e-6 whatever the azimuth)
+    const float q2 = Iu * Iu + Iv * Iv;
+    const bool az = q2 > 1e-30f;
+    const float rinv = az ? __builtin_amdgcn_rsqf(q2) : 0.f;
+    const float cph = a * (az ? Iv * rinv : 1.f);
+    const float sph = a * (Iu * rinv);
+    pisinc_h(sT * cph, &n1, &d1);
+    pisinc_h(sT * sph, &n2, &d2);
+    pisinc_h(sTT * cph, &n3, &d3);
+    pisinc_h(sTT * sph, &n4, &d4);
     const float den = fabsf((d1 * d2) * (d3 * d4));
     float g = fabsf((n1 * n2) * (n3 * n4)) * __builtin_amdgcn_rcpf(den) * (0.0625f * rs);
     if (S3 && !lossless && st.deep && (double)fz > st.zi) g *= st.tsq;
@@ -2698,7 +2704,7 @@ __device__ __forceinline__ Tri tri_shot(const TLeg& g, double itd, float2 src, d
     const double xq = fma(rngt, kp.inv_dr, -rst * kp.inv_dr);
     o.b = (int)xq;
     o.w = xq - (double)o.b;
-    if (o.w < 1e-7 || o.w > 1.0 - 1e-7) {
+    if (!(o.w >= 1e-7 && o.w <= 1.0 - 1e-7)) {  // (a NaN too)
         // the facet's coordinates pass through an empty asm statement, so
         // that the exact root below stays on this rare path (the two shots'
         // copies of it would otherwise be merged and hoisted out of it)
@@ -2714,7 +2720,7 @@ __device__ __forceinline__ Tri tri_shot(const TLeg& g, double itd, float2 src, d
         }
         o.valid = bin_of(rngt, rst, kp.drd, nr, &o.b, &o.w);
     } else {
-        o.valid = (xq > -1.0) && (xq < (double)nr);
+        o.valid = (unsigned)o.b < (unsigned)nr;  // here w > 0, so xq >= 0
     }
     o.c = cmul(src, g.Gc);
     return o;
@@ -2727,6 +2733,41 @@ constexpr int NTB = 1024;  // threads of k_target_accum_pair (one workgroup per 
 // On the 2048^2 fBm workload every pair's bounds (the nearer of the shot's
 // box and bounding-sphere bounds) fit 5056 bins.
 constexpr int TWB = 5056;
+
+// Windows of the pairs of one launch of k_target_accum_pair, one thread per
+// (item, shot): wtab[row] = (base, top), pbase (-1: does not fit), pwin.  In
+// that kernel they cost every one of its 16 waves about 250 instructions at
+// the start of each item, a sixth of its work where a shot lights 6e3 facets
+// (883 against 728 us per 32768 pairs of 4096 bins), and a chain of FP64 roots
+// that nothing else on the CU hid.  Multi-track batches (trk): also the rows' range kernel
+// spectra, and the item counter cleared.
+__global__ void __launch_bounds__(256) k_pair_windows(
+    const int4* __restrict__ items, int nitems0, const float* __restrict__ tg0, int64_t Tpad0,
+    const erp_shot* __restrict__ shots, const Bounds* __restrict__ bounds, KPar kp0,
+    int* __restrict__ pbase, int* __restrict__ pwin, int2* __restrict__ wtab,
+    const TrackK* __restrict__ trk, const RowK* __restrict__ rows,
+    const int* __restrict__ nitems_dev, int* __restrict__ next_item,
+    const float4** __restrict__ Gpair) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x, it = i >> 1, k = i & 1;
+    if (trk && i == 0) *next_item = 0;
+    if (it >= (nitems_dev ? *nitems_dev : nitems0)) return;
+    const int4 item = items[it];
+    const int t = item.x, row = k ? item.z : item.y, s = 2 * item.w + k;
+    if (row < 0) return;
+    const TrackK* tk = trk ? &trk[rows[2 * item.w].trk] : nullptr;
+    const KPar& kp = tk ? tk->kp : kp0;
+    const float* tg = tk ? tk->tg : tg0;
+    const int64_t Tpad = tk ? tk->Tpad : Tpad0;
+    const float tz = tg[2 * Tpad + t];
+    const bool deep = kp.has3 && (double)tz < kp.zi;
+    const PairWin pw = pair_window(bounds[s], tg[t], tg[Tpad + t], tz, deep ? kp.n_lo : kp.n_d,
+                                   deep ? kp.n_hi : kp.n_d, (double)shots[s].rst, kp, kp.nr, TWB,
+                                   true);
+    pbase[row] = pw.fits ? pw.base : -1;
+    pwin[row] = pw.len;
+    wtab[row] = make_int2(pw.base, pw.top);
+    if (tk) Gpair[row] = reinterpret_cast<const float4*>(tk->g_targ_nat);
+}
 
 // MT: a multi-track batch: an item's block is two rows of one track, whose
 // targets, parameters and facet frames it uses; the item count is read from
@@ -2742,9 +2783,10 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(1, NTB)))
 k_target_accum_pair(const float* __restrict__ tg0, int64_t Tpad0, const int4* __restrict__ items,
                     int nitems0, int* __restrict__ next_item, const erp_shot* __restrict__ shots,
                     const int64_t* __restrict__ ubase, const int* __restrict__ Ucnt, BRec rec,
-                    const Bounds* __restrict__ bounds, const erp_prism* __restrict__ prisms,
-                    int np, KPar kp0, float2* __restrict__ outA, int* __restrict__ pbase,
-                    int* __restrict__ pwin, int frame_ok0, int* __restrict__ oow,
+                    const erp_prism* __restrict__ prisms, int np, KPar kp0,
+                    float2* __restrict__ outA, const int* __restrict__ pbase,
+                    const int* __restrict__ pwin, const int2* __restrict__ wtab, int frame_ok0,
+                    int* __restrict__ oow,
                     const TrackK* __restrict__ trk, const RowK* __restrict__ rows,
                     const int* __restrict__ nitems_dev, const int* __restrict__ Vs) {
     __shared__ double winS[4 * TWB];
@@ -2772,15 +2814,17 @@ k_target_accum_pair(const float* __restrict__ tg0, int64_t Tpad0, const int4* __
         const KPar& kp = MT ? tkp->kp : kp0;
         const float* __restrict__ tg = MT ? tkp->tg : tg0;
         const int64_t Tpad = MT ? tkp->Tpad : Tpad0;
-        const int frame_ok = MT ? tkp->frame_ok : frame_ok0;
+        // flags as scalar integers: a comparison's result would be kept as a
+        // lane mask and tested with vector instructions in the loop
+        auto flag_of = [](bool f) { return __builtin_amdgcn_readfirstlane(f ? 1 : 0); };
+        const int frame_ok = flag_of(MT ? tkp->frame_ok : frame_ok0);
         const int nr = kp.nr;
-        const bool lossless = kp.mode & ERP_MODE_LOSSLESS;
+        const int lossless = flag_of(kp.mode & ERP_MODE_LOSSLESS);
         const float txf = tg[t], tyf = tg[Tpad + t], tzf = tg[2 * Tpad + t];
         const float tnx = tg[3 * Tpad + t], tny = tg[4 * Tpad + t], tnz = tg[5 * Tpad + t];
         const double tx = txf, ty = tyf, tz = tzf;
-        const bool tn_up = tnx == 0.f && tny == 0.f && tnz == 1.f;
-        const Strat st{S3 && (double)tzf < kp.zi, kp.zi, (double)tzf, kp.dn, kp.tsq};
-        const double n_lo = st.deep ? kp.n_lo : kp.n_d, n_hi = st.deep ? kp.n_hi : kp.n_d;
+        const int tn_up = flag_of(tnx == 0.f && tny == 0.f && tnz == 1.f);
+        const Strat st{flag_of(S3 && (double)tzf < kp.zi), kp.zi, (double)tzf, kp.dn, kp.tsq};
 
         // each shot's window (as k_target_accum_fast's); a shot without the
         // target has an empty one
@@ -2802,29 +2846,23 @@ k_target_accum_pair(const float* __restrict__ tg0, int64_t Tpad0, const int4* __
             rowp[k] = nullptr;
             flag[k] = nullptr;
             if (row[k] < 0) continue;
-            const int s = 2 * blk + k;
-            rst[k] = (double)shots[s].rst;
-            const PairWin pw = pair_window(bounds[s], txf, tyf, tzf, n_lo, n_hi, rst[k], kp, nr,
-                                           TWB, true);
-            base[k] = pw.base;
-            len[k] = pw.len;
-            top[k] = pw.top;
-            fits[k] = pw.fits;
+            rst[k] = (double)shots[2 * blk + k].rst;
+            const int2 w = wtab[row[k]];  // k_pair_windows
+            base[k] = w.x;
+            top[k] = w.y;
+            len[k] = pwin[row[k]];
+            fits[k] = pbase[row[k]] >= 0;
             rowp[k] = outA + (size_t)row[k] * kp.row_stride;
             // out-of-window terms of a pair whose window covers its bounds
             // (deterministic: of every pair) are broken bounds (counted);
             // the others go to the row
-            flag[k] = (DET || pw.fits) ? oow : nullptr;
-            if (threadIdx.x == 0) {
-                pbase[row[k]] = pw.fits ? pw.base : -1;
-                pwin[row[k]] = pw.len;
-            }
-            if (!pw.fits) {
+            flag[k] = (DET || fits[k]) ? oow : nullptr;
+            if (!fits[k]) {
                 spill = true;
                 // bins outside what the window passes write: zero
-                const int hi = DET ? max(pw.top, pw.base) : pw.base + TWB;
+                const int hi = DET ? max(top[k], base[k]) : base[k] + TWB;
                 for (int i = threadIdx.x; i < kp.row_live; i += NTB)
-                    if (i < pw.base || i >= hi || i >= nr) rowp[k][i] = make_float2(0.f, 0.f);
+                    if (i < base[k] || i >= hi || i >= nr) rowp[k][i] = make_float2(0.f, 0.f);
             }
         }
         // the row's zeros land before any thread's out-of-window atomics
@@ -2843,6 +2881,9 @@ k_target_accum_pair(const float* __restrict__ tg0, int64_t Tpad0, const int4* __
                          reinterpret_cast<const char*>(rec.itd + r0),
                          reinterpret_cast<const char*>(rec.src + r0)};
         const unsigned ul = (unsigned)max(U - 1, 0);
+        unsigned lim[2];  // bins b of the window whose b + 1 is in it and the row
+#pragma unroll
+        for (int k = 0; k < 2; ++k) lim[k] = max(min(len[k], nr - base[k]) - 1, 0);
         // every union facet through add(k, term): one facet per thread and
         // step, the next step's record loaded before this step's arithmetic
         // into the other of two register sets (clamped, in-bounds indices:
@@ -2863,6 +2904,13 @@ k_target_accum_pair(const float* __restrict__ tg0, int64_t Tpad0, const int4* __
                     if (o.valid) add(k, o);
                 }
             };
+            if (DET) {
+                // the next record's registers would spill; the other waves
+                // cover the loads
+#pragma unroll 1
+                for (int u = threadIdx.x; u < U; u += NTB) step(load_brec(rb, (unsigned)u));
+                return;
+            }
             BRecV a0 = load_brec(rb, min((unsigned)threadIdx.x, ul));
             for (int u = threadIdx.x; u < U; u += 2 * NTB) {
                 const BRecV a1 = load_brec(rb, min((unsigned)(u + NTB), ul));
@@ -2875,7 +2923,20 @@ k_target_accum_pair(const float* __restrict__ tg0, int64_t Tpad0, const int4* __
 
         if constexpr (!DET) {
             for_terms([&](int k, const Tri& o) {
-                tri_add<ACC_F64>(o, base[k], len[k], nr, win[k], rowp[k], flag[k]);
+                // nearly every term: both bins inside the window and the row
+                const int k0 = o.b - base[k];
+                if ((unsigned)k0 < lim[k]) {
+                    const double cx = o.c.x, cy = o.c.y, c1x = cx * o.w, c1y = cy * o.w;
+                    // (through the array itself: a pointer kept in win makes
+                    // these generic accesses)
+                    double* x = winS + 2 * k * TWB + k0;
+                    atomicAdd(x, cx - c1x);
+                    atomicAdd(x + TWB, cy - c1y);
+                    atomicAdd(x + 1, c1x);
+                    atomicAdd(x + TWB + 1, c1y);
+                } else {
+                    tri_add<ACC_F64>(o, base[k], len[k], nr, win[k], rowp[k], flag[k]);
+                }
             });
             __syncthreads();
             // flush each window into its row and clear what was read
@@ -2893,6 +2954,7 @@ k_target_accum_pair(const float* __restrict__ tg0, int64_t Tpad0, const int4* __
             // the split weights, each <= 1) / Ttd; max(|re|, |im|) x 1.4143
             // bounds the phasor's modulus
             float m[2] = {0.f, 0.f};
+#pragma unroll 4
             for (int u = threadIdx.x; u < U; u += NTB) {
                 const unsigned o16 = (unsigned)u << 4;
                 const float4 qa = *reinterpret_cast<const float4*>(rb.qa + o16);
@@ -2911,10 +2973,10 @@ k_target_accum_pair(const float* __restrict__ tg0, int64_t Tpad0, const int4* __
                 if ((threadIdx.x & 63) == 0) s_m[threadIdx.x >> 6][k] = m[k];
             }
             __syncthreads();
-            double scale[2], inv[2];
+            double scale[2];
             // a shot of at least 1024 lit facets bounds every term below
             // 2^61 / 2048 = 2^50 in fixed point: det_fix51 applies
-            bool fast[2];
+            int fast[2];
             int npass = 1;
 #pragma unroll
             for (int k = 0; k < 2; ++k) {
@@ -2924,8 +2986,7 @@ k_target_accum_pair(const float* __restrict__ tg0, int64_t Tpad0, const int4* __
                 // 97.409...
                 const int V = row[k] >= 0 ? Vs[2 * blk + k] : 0;
                 scale[k] = det_scale((double)V, 2.0 * 1.4143 * (double)mk * 97.40909103400244);
-                inv[k] = scale[k] > 0.0 ? 1.0 / scale[k] : 0.0;
-                fast[k] = V >= 1024;
+                fast[k] = flag_of(V >= 1024);
                 if (row[k] >= 0 && !fits[k])
                     npass = max(npass, (top[k] - base[k] + TWB - 1) / TWB);
             }
@@ -2937,19 +2998,18 @@ k_target_accum_pair(const float* __restrict__ tg0, int64_t Tpad0, const int4* __
             // one window per shot and pass: [base + p TWB, ...) below top
             for (int p = 0; p < npass; ++p) {
                 int wb[2], wl[2];
-                bool first[2], last[2];
+                int first[2], last[2];
+                unsigned dl[2];  // fast: bins whose next bin is in the window and the row
 #pragma unroll
                 for (int k = 0; k < 2; ++k) {
                     wb[k] = base[k] + p * TWB;
                     wl[k] = row[k] < 0 ? 0 : fits[k] ? (p == 0 ? len[k] : 0)
                                                      : min(TWB, max(0, top[k] - wb[k]));
-                    first[k] = p == 0;
-                    last[k] = fits[k] || wb[k] + TWB >= top[k];
+                    first[k] = flag_of(p == 0);
+                    last[k] = flag_of(fits[k] || wb[k] + TWB >= top[k]);
+                    dl[k] = fast[k] ? max(min(wl[k], nr - wb[k]) - 1, 0) : 0;
                 }
-                for_terms([&](int k, const Tri& o) {
-                    const float wf = (float)o.w;
-                    const float2 c0 = make_float2(o.c.x * (1.f - wf), o.c.y * (1.f - wf));
-                    const float2 c1 = make_float2(o.c.x * wf, o.c.y * wf);
+                auto general = [&](int k, const Tri& o, float2 c0, float2 c1) {
                     const int k0 = o.b - wb[k];
                     auto put = [&](int i, float2 c) {
                         if (fast[k]) lds_add2_fix51(wux(k), wuy(k), i, c, scale[k]);
@@ -2964,18 +3024,32 @@ k_target_accum_pair(const float* __restrict__ tg0, int64_t Tpad0, const int4* __
                         else if ((o.b + 1 < base[k] && first[k]) || (o.b + 1 >= top[k] && last[k]))
                             atomicAdd(flag[k], 1);
                     }
+                };
+                for_terms([&](int k, const Tri& o) {
+                    const float wf = (float)o.w;
+                    const float2 c0 = make_float2(o.c.x * (1.f - wf), o.c.y * (1.f - wf));
+                    const float2 c1 = make_float2(o.c.x * wf, o.c.y * wf);
+                    const int k0 = o.b - wb[k];
+                    if ((unsigned)k0 < dl[k]) {  // nearly every term
+                        lds_add2_fix51(wux(k), wuy(k), k0, c0, scale[k]);
+                        lds_add2_fix51(wux(k), wuy(k), k0 + 1, c1, scale[k]);
+                    } else {
+                        general(k, o, c0, c1);
+                    }
                 });
                 __syncthreads();
 #pragma unroll
-                for (int k = 0; k < 2; ++k)
+                for (int k = 0; k < 2; ++k) {
+                    const double inv = scale[k] > 0.0 ? 1.0 / scale[k] : 0.0;
                     for (int i = threadIdx.x; i < wl[k]; i += NTB) {
                         const int b = wb[k] + i;
                         if (b < nr)
-                            rowp[k][b] = make_float2((float)det_unfix(wux(k)[i], inv[k]),
-                                                     (float)det_unfix(wuy(k)[i], inv[k]));
+                            rowp[k][b] = make_float2((float)det_unfix(wux(k)[i], inv),
+                                                     (float)det_unfix(wuy(k)[i], inv));
                         wux(k)[i] = 0ull;
                         wuy(k)[i] = 0ull;
                     }
+                }
                 if (p + 1 < npass) __syncthreads();
             }
         }
@@ -4556,6 +4630,7 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
                 W.pairs.ensure(sizeof(int) * ((size_t)C * 4 + 2 * gcap + 3 * (size_t)S + 16));
                 int* dps = W.pairs.as<int>();
                 int* dpt = dps + C;
+                int2* dpt2 = reinterpret_cast<int2*>(dps);  // shot-pair kernel: (base, top)
                 int* dpb = dpt + C;                  // per-pair window base (fused)
                 int* dgb = dpb + C;                  // group begin / end
                 int* dge = dgb + gcap;
@@ -4630,6 +4705,13 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
                         // persistent grid: one workgroup per CU (its two windows
                         // take 128 KB of LDS), each taking items until none is left
                         const int grid = std::max(1, std::min(nit, ctx->num_cu));
+                        hipLaunchKernelGGL(k_pair_windows, dim3((2 * nit + 255) / 256), dim3(256),
+                                           0, st, (const int4*)ditems, nit,
+                                           targets->xyzn.as<float>(), Tpad, dshots, dbounds, kp,
+                                           dpb, dpw, dpt2, (const TrackK*)nullptr,
+                                           (const RowK*)nullptr, (const int*)nullptr,
+                                           (int*)nullptr, (const float4**)nullptr);
+                        ERP_CHECK_LAUNCH("k_pair_windows");
                         auto kern = det ? (kp.has3 ? k_target_accum_pair<true, false, true>
                                                    : k_target_accum_pair<false, false, true>)
                                         : (kp.has3 ? k_target_accum_pair<true>
@@ -4637,8 +4719,8 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
                         hipLaunchKernelGGL(kern, dim3(grid), dim3(NTB), 0, st,
                                            targets->xyzn.as<float>(), Tpad,
                                            (const int4*)ditems, nit, dnext, dshots,
-                                           brk.ubase, brk.U, brk.rec, dbounds, dpr, (int)nprisms,
-                                           kp, A, dpb, dpw, mesh->frame_ok ? 1 : 0,
+                                           brk.ubase, brk.U, brk.rec, dpr, (int)nprisms, kp, A,
+                                           dpb, dpw, dpt2, mesh->frame_ok ? 1 : 0,
                                            W.oow.as<int>(), (const TrackK*)nullptr,
                                            (const RowK*)nullptr, (const int*)nullptr,
                                            (const int*)dV);
@@ -5135,8 +5217,8 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
     const size_t tab_ints = 2 * (size_t)C + 2 * (size_t)gcap + 3 * (size_t)segcap + 1 + segcap;
     m.tabs.ensure(sizeof(int) * tab_ints);
     // device-written: pair window bases and lengths, the pair counter, the
-    // per-pair range kernel spectra
-    m.dtabs.ensure(sizeof(int) * (2 * (size_t)C + 64) + sizeof(void*) * (size_t)C);
+    // per-pair range kernel spectra and windows
+    m.dtabs.ensure(sizeof(int) * (2 * (size_t)C + 64) + 2 * sizeof(void*) * (size_t)C);
     if (pairk) {
         m.umask.ensure(sizeof(unsigned long long) * (size_t)nbk * nblk_max * MASKW);
         m.ucnt.ensure(sizeof(int) * (size_t)nbk * nblk_max);
@@ -5161,6 +5243,7 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
     int* d_pwin = d_pbase + C;
     int* d_next = d_pwin + C;  // 64 ints: the pair counter, then padding
     const float4** d_G = reinterpret_cast<const float4**>(d_next + 64);
+    int2* d_wtab = reinterpret_cast<int2*>(d_G + C);  // shot-pair kernel: (base, top) per row
 
     ERP_HIP_TRY(hipMemcpyAsync(m.trk.p, tk.data(), sizeof(TrackK) * (size_t)ntr,
                                hipMemcpyHostToDevice, st));
@@ -5440,11 +5523,12 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
                                            hipMemcpyHostToDevice, st));
                 PT_.begin(ERP_STAGE_TARGET_ACCUM, st, pc.triples);
                 mt_launch(m.gChunk, direct, st, [&] {
-                    // range kernel spectra per row, the item counter cleared
-                    hipLaunchKernelGGL(k_pair_targets_rows, dim3((C + 255) / 256), dim3(256), 0,
-                                       st, t_ptgt, t_pshot, list1, Tcap, t_n, d_next, d_G, dtrk,
-                                       drows);
-                    ERP_CHECK_LAUNCH("k_pair_targets_rows");
+                    // windows, range kernel spectra per row, the item counter cleared
+                    hipLaunchKernelGGL(k_pair_windows, dim3((2 * C + 255) / 256), dim3(256), 0, st,
+                                       (const int4*)d_items, 0, (const float*)nullptr, (int64_t)0,
+                                       dshots, dbounds, kp0, d_pbase, d_pwin, d_wtab, dtrk, drows,
+                                       (const int*)d_nitems, d_next, d_G);
+                    ERP_CHECK_LAUNCH("k_pair_windows");
                     auto kern = det ? (s3 ? k_target_accum_pair<true, true, true>
                                           : k_target_accum_pair<false, true, true>)
                                     : (s3 ? k_target_accum_pair<true, true>
@@ -5454,9 +5538,9 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
                                        dim3(NTB), 0, st, (const float*)nullptr, (int64_t)0,
                                        (const int4*)d_items, 0, d_next, dshots,
                                        (const int64_t*)m.ubase.as<int64_t>(),
-                                       (const int*)m.U.as<int>(), brk.rec, dbounds,
-                                       (const erp_prism*)nullptr, 0, kp0, A, d_pbase, d_pwin, 0,
-                                       d_next + 1, dtrk, drows, (const int*)d_nitems,
+                                       (const int*)m.U.as<int>(), brk.rec,
+                                       (const erp_prism*)nullptr, 0, kp0, A, d_pbase, d_pwin,
+                                       d_wtab, 0, d_next + 1, dtrk, drows, (const int*)d_nitems,
                                        (const int*)dV);
                     ERP_CHECK_LAUNCH("k_target_accum_pair");
                     chain();
