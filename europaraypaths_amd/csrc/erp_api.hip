@@ -806,6 +806,10 @@ int erp_focus(erp_ctx* ctx, const float* rdr, int64_t Nr, int64_t Na, int64_t ro
         std::lock_guard<std::mutex> lk(ctx->mu);
         set_device(ctx);
         DevBuf d_rdr, d_hs, d_nsx, d_off, d_rows, d_filt, d_out;
+        struct Free {
+            DevBuf* b[7];
+            ~Free() { for (DevBuf* d : b) d->release(); }
+        } free_at_end{{&d_rdr, &d_hs, &d_nsx, &d_off, &d_rows, &d_filt, &d_out}};
         d_rdr.ensure(sizeof(float2) * (size_t)(Nr * Na));
         d_hs.ensure(sizeof(int) * (size_t)nrows);
         d_nsx.ensure(sizeof(int) * (size_t)nrows);
