@@ -49,7 +49,6 @@ constexpr int WPB = NT / 64;   // waves per block
 constexpr int MASKW = FB / 64; // mask words per block (32)
 constexpr int SWIN = 2048;     // surface LDS window (bins)
 constexpr int LWIN = 1024;     // that of the surface kernel without records
-constexpr int TWIN = 4096;     // target LDS window (bins)
 constexpr int NTT = 512;       // threads per workgroup of the target kernels
 // (shot, target) pairs per target launch: their P-point rows take at most
 // kPairRowBytes per buffer set.  Large launches keep the last round of
@@ -187,6 +186,15 @@ __device__ __forceinline__ float2 sc_angles(float Iu, float Iv, float s) {
 __device__ __forceinline__ float sinc_f(float x) {
     if (fabsf(x) < 1e-6f) return 1.0f;
     return sinpif(x) / (3.14159265358979f * x);
+}
+
+// sin(pi |x|) and |x| / 2, at least 5e-7 (where the sinc is 1 to 1e-12): the
+// sinc sin(pi x) / (pi x) is num / (2 pi den).  Hardware sine on the exactly
+// reduced argument in revolutions, 1.2e-7 absolute.
+__device__ __forceinline__ void pisinc(float x, float* num, float* den) {
+    const float h = fmaxf(fabsf(0.5f * x), 5e-7f);
+    *num = __builtin_amdgcn_sinf(__builtin_amdgcn_fractf(h));
+    *den = h;
 }
 
 // sin(pi r) and cos(pi r) for |r| <= 0.5 from their Taylor series (degree 13
@@ -995,9 +1003,12 @@ __global__ void __launch_bounds__(NT) k_surface(
                 for (int a = 0; a < 12; ++a) rec.geo[(size_t)a * rec.cap + r] = g[a];
                 rec.F[r] = Fr;
                 rec.fRfrC[r] = fRfrC;
-                rec.ang[r] = atan2f(sI, cI);                 // Ith
-                rec.ang[rec.cap + r] = atan2f(Iu, Iv);       // Iph
-                rec.ang[2 * rec.cap + r] = tir ? 1e4f : asinf(sR);  // Rth
+                // cos Iph, sin Iph (Iph = atan2(Iu, Iv): 0 where both vanish)
+                // and sin Rth (2: past the critical angle)
+                const float rI = sqrtf(Iu * Iu + Iv * Iv);
+                rec.ang[r] = rI > 0.f ? Iv / rI : 1.f;
+                rec.ang[rec.cap + r] = rI > 0.f ? Iu / rI : 0.f;
+                rec.ang[2 * rec.cap + r] = tir ? 2.f : sR;
             }
             if (rec.qa) {
                 // F Dmax / pi^4: the gain factor of the target kernel's
@@ -1647,8 +1658,60 @@ __device__ __forceinline__ float rerad_f(int fn, float th) {
     }
 }
 
-// MODE 0: type != 0, non-specular: one trace A (the inward trace PTtarg);
-//         the outward trace is -A/sqrt(P) exactly.
+// Specular reradiation factors of a facet towards a target and back
+// (geometry_kernels.cu:530-539, 565-572): fs^2 / lam times
+//     sinc(fs / lam sin(Rth - Tth) cos dph) sinc(... sin dph),  dph = Iph - Tph,
+// and the same with sin(RrTh) for the way back (sinc is even, so its dph may
+// take either sign).  The angles enter through sines and cosines only: those
+// of Iph and Rth are the facet record's, (sT, cT) and (Iu, Iv) the target
+// leg's, so no angle is formed; past a critical angle the reference takes
+// 1e4 for the angle.
+__device__ __forceinline__ void spec_factors(float sT, float cT, float cph, float sph, float cI,
+                                             float sI, float sRec, const KPar& kp, float* vi,
+                                             float* vo) {
+    const float s1e4 = -0.30561438888825215f, c1e4 = -0.95215536825901485f;
+    const bool tir = sRec > 1.f;
+    const float sR = tir ? s1e4 : sRec;
+    const float cR = tir ? c1e4 : __builtin_amdgcn_sqrtf((1.f - sRec) * (1.f + sRec));
+    const float si = sR * cT - cR * sT;
+    const float back = kp.sqrt_e2e1 * sT;
+    const float so = back > 1.f ? s1e4 : back;
+    const float cd = cI * cph + sI * sph, sd = sI * cph - cI * sph;
+    float n1, d1, n2, d2;
+    pisinc(kp.fs_lam * si * cd, &n1, &d1);
+    pisinc(kp.fs_lam * si * sd, &n2, &d2);
+    *vi = kp.fs2_lam * 0.25f * (n1 * n2) * __builtin_amdgcn_rcpf(d1 * d2) * 0.101321184f;
+    pisinc(kp.fs_lam * so * cd, &n1, &d1);
+    pisinc(kp.fs_lam * so * sd, &n2, &d2);
+    *vo = kp.fs2_lam * 0.25f * (n1 * n2) * __builtin_amdgcn_rcpf(d1 * d2) * 0.101321184f;
+}
+
+// The same in the reference's steps, for the type-0 targets: their terms take
+// the factors squared, and the hardware functions' errors with them (the sinc
+// sums' error against 64 bits would be 1.8e-6 instead of 1.2e-6).
+__device__ __forceinline__ void spec_factors_angles(float sT, float cT, float Iu, float Iv,
+                                                    const Rec& rec, int64_t r, const KPar& kp,
+                                                    float* vi, float* vo) {
+    const float Iph = atan2f(rec.ang[rec.cap + r], rec.ang[r]), sRec = rec.ang[2 * rec.cap + r];
+    const float Rth = sRec > 1.f ? 1e4f : asinf(sRec);
+    const float Tth = atan2f(sT, cT), Tph = atan2f(Iu, Iv);
+    const float si = sinf(Rth - Tth), dph = Iph - Tph;
+    *vi = kp.fs2_lam * sinc_f(kp.fs_lam * si * cosf(dph)) * sinc_f(kp.fs_lam * si * sinf(dph));
+    const float sR = kp.sqrt_e2e1 * sinf(ERP_PI_F - Tth);
+    const float so = sinf((sR > 1.f) ? 1e4f : asinf(sR)), dpo = Tph - Iph;
+    *vo = kp.fs2_lam * sinc_f(kp.fs_lam * so * cosf(dpo)) * sinc_f(kp.fs_lam * so * sinf(dpo));
+}
+
+// Bins of k_target_accum's LDS window(s): 64 KB, less for short ranges (none
+// holds more than nr bins), which lets more workgroups share a CU.
+constexpr int TWIN_MAX = 4096;
+inline int accum_window(int mode, int nr) {
+    return std::min(mode == 1 ? TWIN_MAX / 2 : TWIN_MAX, (nr + 63) & ~63);
+}
+inline size_t accum_lds(int mode, int nr) {
+    return sizeof(double2) * (mode == 1 ? 2 : 1) * (size_t)accum_window(mode, nr);
+}
+
 // MODE 1: type != 0, specular: inward (A) and outward (B) traces separately.
 // MODE 2: type == 0 (genRefrPhasor): single bin, summed into one per-shot
 //         trace (out row = per shot, global atomics after the LDS window).
@@ -1661,16 +1724,18 @@ __device__ __forceinline__ float rerad_f(int fn, float th) {
 // targets of a shot add to the shot's row): pass 1 only takes the largest
 // component of each pair into tmax[shot]; pass 2 adds the terms, scaled by
 // the shot's bound, into the shot's row as fixed-point (int64) pairs.
+// MODE 1 is bound by its instructions (80 % busy): hardware sines, roots and
+// reciprocals and no angles, 359 to 219 us per 600 pairs, and no fence where the
+// window holds the pair, to 97.
 template <int MODE, bool DET = false>
 __global__ void __launch_bounds__(NTT) k_target_accum(
     const float* __restrict__ tg, int64_t Tpad, const int* __restrict__ pshot,
     const int* __restrict__ ptgt, const erp_shot* __restrict__ shots,
     const int* __restrict__ Vs, const int64_t* __restrict__ rec_base, Rec rec,
     const Bounds* __restrict__ bounds, const erp_prism* __restrict__ prisms, int np, KPar kp,
-    float2* __restrict__ outA, float2* __restrict__ outB, int* __restrict__ pbase,
-    unsigned* __restrict__ tmax, const int* __restrict__ tcnt, int pass, int* __restrict__ oow) {
-    extern __shared__ double2 lds[];
-    constexpr int WIN = (MODE == 1) ? TWIN / 2 : TWIN;  // MODE 1 holds two windows
+    float2* __restrict__ outA, float2* __restrict__ outB, unsigned* __restrict__ tmax,
+    const int* __restrict__ tcnt, int pass, int* __restrict__ oow, int WIN) {
+    extern __shared__ double2 lds[];  // MODE 1 holds two windows of WIN bins
     double2* winA = lds;
     double2* winB = lds + WIN;  // MODE 1 only
     const int pi = blockIdx.x;
@@ -1698,9 +1763,8 @@ __global__ void __launch_bounds__(NTT) k_target_accum(
     int base = (int)floor((rlo - rst) / kp.drd) - 2;
     base = max(base, 0);
     // upper bound: Itd_max + n * (distance to the farthest AABB corner)
-    bool fits = false;
     int top = nr;
-    if (DET && MODE == 1) {
+    if (MODE == 1) {
         const float fx = fmaxf(fabsf(o2f(bd.xmin) - txf), fabsf(o2f(bd.xmax) - txf));
         const float fy = fmaxf(fabsf(o2f(bd.ymin) - tyf), fabsf(o2f(bd.ymax) - tyf));
         const float fz = fmaxf(fabsf(o2f(bd.zmin) - tzf), fabsf(o2f(bd.zmax) - tzf));
@@ -1709,20 +1773,10 @@ __global__ void __launch_bounds__(NTT) k_target_accum(
         const double rhi = ithmax + kp.n_d * tmax_d * (1.0 + 1e-6) + 1.0;
         top = min((int)ceil((rhi - rst) / kp.drd) + 2, nr);
     }
-    if (MODE == 0 && pbase) {
-        const float fx = fmaxf(fabsf(o2f(bd.xmin) - txf), fabsf(o2f(bd.xmax) - txf));
-        const float fy = fmaxf(fabsf(o2f(bd.ymin) - tyf), fabsf(o2f(bd.ymax) - tyf));
-        const float fz = fmaxf(fabsf(o2f(bd.zmin) - tzf), fabsf(o2f(bd.zmax) - tzf));
-        const double tmax = sqrt((double)fx * fx + (double)fy * fy + (double)fz * fz);
-        const double ithmax = __longlong_as_double((long long)bd.itd_max);
-        const double rhi = ithmax + kp.n_d * tmax * (1.0 + 1e-6) + 1.0;
-        const int top = (int)ceil((rhi - rst) / kp.drd) + 2;
-        fits = (top < base + WIN - 1) || (base + WIN >= nr);
-        if (threadIdx.x == 0) pbase[pi] = fits ? base : -1;
-    }
-
     float2* rowA = (MODE == 2) ? outA + (size_t)s * P : outA + (size_t)pi * P;
     float2* rowB = (MODE == 1) ? outB + (size_t)pi * P : nullptr;
+    // radiateTarget's phase against accumulateTarget's: half a wavelength
+    const float2 half_lam = phasor_cycles(-0.5 * (double)kp.lam * kp.inv_cyc);
 
     // one facet x target term of facet k: add(b, w, c, d) with the bin, the
     // split weight, the inward term and (MODE 1) the outward term, unless
@@ -1737,17 +1791,84 @@ __global__ void __launch_bounds__(NTT) k_target_accum(
         const float vx = rec.geo[9 * rec.cap + r], vy = rec.geo[10 * rec.cap + r],
                     vz = rec.geo[11 * rec.cap + r];
         const double Itd = rec.itd[r];
+        if constexpr (MODE == 1) {
+            // the arithmetic of tri_leg and tri_shot: bins from the range to
+            // 1e-14, repeated exactly within 1e-7 of a bin edge
+            const double dx = tx - (double)fx, dy = ty - (double)fy, dz = tz - (double)fz;
+            const double t2 = fma(dx, dx, fma(dy, dy, dz * dz));
+            const float rs = __builtin_amdgcn_rsqf((float)t2);
+            const double rd = (double)rs, hr = 0.5 * rd, y0 = t2 * rd;
+            const double Ttd = fma(fma(-y0, y0, t2), hr, y0);
+            double rngt = fma(Ttd, kp.n_d, Itd);
+            const double xq = fma(rngt, kp.inv_dr, -rst * kp.inv_dr);
+            int b = (int)xq;
+            float w;
+            {
+                const double wd = xq - (double)b;
+                w = (float)wd;
+                if (!(wd >= 1e-7 && wd <= 1.0 - 1e-7)) {
+                    rngt = madd_nc(Itd, dist3(dx, dy, dz), kp.n_d);
+                    if (!bin_of(rngt, rst, kp.drd, nr, &b, &w)) return;
+                } else if ((unsigned)b >= (unsigned)nr) {
+                    return;
+                }
+            }
+            const double invd = rd * fma(-y0, hr, 1.5);
+            const double ix = dx * invd, iy = dy * invd, iz = dz * invd;
+            const float Ix = (float)ix, Iy = (float)iy, Iz = (float)iz;
+            const float2 csT = cos_sin_hw(ix, iy, iz, nx, ny, nz);
+            const float cT = csT.x, sT = csT.y, sTT = cos_sin_hw(ix, iy, iz, tnx, tny, tnz).y;
+            float Iu = Ix * ux + Iy * uy + Iz * uz;
+            float Iv = Ix * vx + Iy * vy + Iz * vz;
+            if (!kp.ortho) {
+                const float2 e = uv_dots_exact(ix, iy, iz, ux, uy, uz, vx, vy, vz);
+                Iu = e.x;
+                Iv = e.y;
+            }
+            const float q2 = Iu * Iu + Iv * Iv;
+            const bool az = q2 > 1e-30f;
+            const float ri = az ? __builtin_amdgcn_rsqf(q2) : 0.f;
+            const float cph = az ? Iv * ri : 1.f, sph = Iu * ri;
+            float n1, d1, n2, d2, n3, d3, n4, d4;
+            pisinc(kp.piLlam * (sT * cph), &n1, &d1);
+            pisinc(kp.piLlam * (sT * sph), &n2, &d2);
+            pisinc(kp.piLlam * (sTT * cph), &n3, &d3);
+            pisinc(kp.piLlam * (sTT * sph), &n4, &d4);
+            // 1 / (2 pi)^4
+            float amp = rec.F[r] * (kp.Dmax * 6.41623909e-4f) *
+                        (fabsf((n1 * n2) * (n3 * n4)) *
+                         __builtin_amdgcn_rcpf((d1 * d2) * (d3 * d4))) * rs;
+            float ampB = amp / kp.sqrtP;
+            if (!lossless) {
+                const float Ttdf = (float)Ttd;
+                float expo = 0.f, tot = 0.f;
+                for (int p = 0; p < np; ++p) {
+                    const float d = prism_len(fx, fy, fz, Ix, Iy, Iz, prisms[p], Ttdf);
+                    tot += d;
+                    expo += prisms[p].alpha * d;
+                }
+                expo += kp.alpha2 * (Ttdf - tot);
+                const float kc = kp.ks * cT;
+                const float e = __builtin_amdgcn_exp2f(-2.885390082f * fmaf(kc, kc, expo));
+                // specular EI / EO facet reradiation factors
+                float vi, vo;
+                spec_factors(sT, cT, cph, sph, rec.ang[r], rec.ang[rec.cap + r],
+                             rec.ang[2 * rec.cap + r], kp, &vi, &vo);
+                ampB *= e * fabsf(vo);
+                amp *= e * fabsf(vi);
+            }
+            const float2 ph = phasor_rc_hw(rngt, kp.inv_cyc);
+            // radiateTarget: phasor(rngt - lam / 2), P = 1 W
+            const float2 pb = cmul(ph, half_lam);
+            add(b, w, make_float2(ph.x * amp, ph.y * amp), make_float2(pb.x * ampB, pb.y * ampB));
+            return;
+        }
         // compTargetRays: forced ray facet -> target
         const double dx = tx - (double)fx, dy = ty - (double)fy, dz = tz - (double)fz;
         const double Ttd = dist3(dx, dy, dz);
-        double rngt;
-        if (MODE == 2) {
-            // genRefrPhasor: sltrng = Itd + Ttd; rngt = (sltrng - Ttd) + Ttd*(c1/c2)
-            const double sl = Itd + Ttd;
-            rngt = madd_nc(sl - Ttd, Ttd, kp.c1c2);
-        } else {
-            rngt = madd_nc(Itd, Ttd, kp.n_d);
-        }
+        // genRefrPhasor: sltrng = Itd + Ttd; rngt = (sltrng - Ttd) + Ttd*(c1/c2)
+        const double sl = Itd + Ttd;
+        const double rngt = madd_nc(sl - Ttd, Ttd, kp.c1c2);
         int b;
         float w;
         if (!bin_of(rngt, rst, kp.drd, nr, &b, &w)) return;
@@ -1777,94 +1898,30 @@ __global__ void __launch_bounds__(NTT) k_target_accum(
             expo += kp.alpha2 * (Ttdf - tot);
         }
         const float kc = kp.ks * cT;
-        if (MODE == 2) {
-            // EI = atten*fRfrC*rough (*rerad_spec), EO likewise; rerad(TargetTh)
-            const float fRfrC = rec.fRfrC[r];
-            float EI = expf(-4.f * expo) * fRfrC * expf(-4.f * kc * kc);
-            float EO = EI;
-            if (kp.mode & ERP_MODE_SPECULAR) {
-                const float Ith = rec.ang[r], Iph = rec.ang[rec.cap + r],
-                            Rth = rec.ang[2 * rec.cap + r];
-                const float Tth = atan2f(sT, cT);
-                const float Tph = atan2f(Iu, Iv);
-                const float dth = Rth - Tth, dph = Iph - Tph;
-                const float si = sinf(dth);
-                const float a1 = sinc_f(kp.fs_lam * si * cosf(dph)),
-                            a2 = sinc_f(kp.fs_lam * si * sinf(dph));
-                const float vi = kp.fs2_lam * a1 * a2;
-                EI *= vi * vi;
-                float sR = kp.sqrt_e2e1 * sinf(ERP_PI_F - Tth);
-                const float RrTh = (sR > 1.f) ? 1e4f : asinf(sR);
-                const float so = sinf(RrTh), dpo = Tph - Iph;
-                const float b1 = sinc_f(kp.fs_lam * so * cosf(dpo)),
-                            b2 = sinc_f(kp.fs_lam * so * sinf(dpo));
-                const float vo = kp.fs2_lam * b1 * b2;
-                EO *= vo * vo;
-                (void)Ith;
-            }
-            const float TTh = atan2f(sTT, cTT);
-            const double sl = Itd + Ttd;
-            const double sl2 = sl * sl;
-            const float req = (float)((double)V * ((double)(kp.P * sh.grefr * sh.grefr * kp.fs *
-                                                           kp.fs * kp.fs * kp.fs) /
-                                                   (ERP_FOURPI5_SQ * sl2 * sl2)));
-            const float rc = rerad_f(kp.rerad, TTh) * EI * EO * req;
-            const float2 ph = phasor_cycles(-2.0 * rngt * kp.inv_cyc);
-            const float2 c = make_float2(ph.x * rc, ph.y * rc);
-            add(b, 0.f, c, make_float2(0.f, 0.f));
-            return;
+        // EI = atten*fRfrC*rough (*rerad_spec), EO likewise; rerad(TargetTh)
+        const float fRfrC = rec.fRfrC[r];
+        float EI = expf(-4.f * expo) * fRfrC * expf(-4.f * kc * kc);
+        float EO = EI;
+        if (kp.mode & ERP_MODE_SPECULAR) {
+            float vi, vo;
+            spec_factors_angles(sT, cT, Iu, Iv, rec, r, kp, &vi, &vo);
+            EI *= vi * vi;
+            EO *= vo * vo;
         }
-        // accumulateTarget / radiateTarget amplitude:
-        // sqrt(Pray n) = F_f * sqrt(G(Tth,Tph) G(TargetTh,Tph)) / Ttd * sqrt(EI-part)
-        // (cos Tph, sin Tph) = (I.v, I.u) / |(I.u, I.v)|
-        const float rp = sqrtf(Iu * Iu + Iv * Iv);
-        const float cph = (rp > 0.f) ? Iv / rp : 1.f;
-        const float sph = (rp > 0.f) ? Iu / rp : 0.f;
-        const float2 scT = make_float2(sT * cph, sT * sph);
-        const float s1 = sinc_f(kp.piLlam * scT.x), s2 = sinc_f(kp.piLlam * scT.y);
-        const float s3 = sinc_f(kp.piLlam * sTT * cph), s4 = sinc_f(kp.piLlam * sTT * sph);
-        const float gg = fabsf(s1 * s2) * fabsf(s3 * s4) * kp.Dmax;
-        float amp = rec.F[r] * gg / Ttdf;
-        float ampB = 0.f;
-        if (!lossless) {
-            const float e = expf(-2.f * (expo + kc * kc));
-            amp *= e;
-            if (MODE == 1) {
-                // specular EI/EO facet reradiation factors (geometry_kernels.cu:530-539,565-572)
-                const float Iph = rec.ang[rec.cap + r], Rth = rec.ang[2 * rec.cap + r];
-                const float Tth = atan2f(sT, cT);
-                const float Tph = atan2f(Iu, Iv);
-                const float si = sinf(Rth - Tth), dph = Iph - Tph;
-                const float a1 = sinc_f(kp.fs_lam * si * cosf(dph)),
-                            a2 = sinc_f(kp.fs_lam * si * sinf(dph));
-                const float vi = kp.fs2_lam * a1 * a2;
-                const float sR = kp.sqrt_e2e1 * sinf(ERP_PI_F - Tth);
-                const float RrTh = (sR > 1.f) ? 1e4f : asinf(sR);
-                const float so = sinf(RrTh), dpo = Tph - Iph;
-                const float b1 = sinc_f(kp.fs_lam * so * cosf(dpo)),
-                            b2 = sinc_f(kp.fs_lam * so * sinf(dpo));
-                const float vo = kp.fs2_lam * b1 * b2;
-                ampB = amp * fabsf(vo) / kp.sqrtP;
-                amp *= fabsf(vi);
-            }
-        } else if (MODE == 1) {
-            ampB = amp / kp.sqrtP;
-        }
-        const float2 ph = phasor_cycles(rngt * kp.inv_cyc);
-        const float2 c = make_float2(ph.x * amp, ph.y * amp);
-        float2 d = make_float2(0.f, 0.f);
-        if (MODE == 1) {
-            // radiateTarget: phasor(rngt - lam/2), P = 1 W
-            const float2 pb = phasor_cycles(rngt * kp.inv_cyc - 0.5 * (double)kp.lam * kp.inv_cyc);
-            d = make_float2(pb.x * ampB, pb.y * ampB);
-        }
-        add(b, w, c, d);
+        const float TTh = atan2f(sTT, cTT);
+        const double sl2 = sl * sl;
+        const float req = (float)((double)V * ((double)(kp.P * sh.grefr * sh.grefr * kp.fs *
+                                                       kp.fs * kp.fs * kp.fs) /
+                                               (ERP_FOURPI5_SQ * sl2 * sl2)));
+        const float rc = rerad_f(kp.rerad, TTh) * EI * EO * req;
+        const float2 ph = phasor_cycles(-2.0 * rngt * kp.inv_cyc);
+        const float2 c = make_float2(ph.x * rc, ph.y * rc);
+        add(b, 0.f, c, make_float2(0.f, 0.f));
     };
 
     if constexpr (!DET) {
-        // zero the output rows outside the window (MODE 2 rows are pre-zeroed);
-        // unnecessary when every contribution provably lands inside the window
-        if (MODE != 2 && !fits) {
+        // zero the output rows outside the window (MODE 2 rows are pre-zeroed)
+        if (MODE != 2) {
             for (int k = threadIdx.x; k < P; k += NTT) {
                 if (k < base || k >= base + WIN || k >= nr) {
                     rowA[k] = make_float2(0.f, 0.f);
@@ -1876,8 +1933,10 @@ __global__ void __launch_bounds__(NTT) k_target_accum(
             winA[k] = make_double2(0.0, 0.0);
             if (MODE == 1) winB[k] = make_double2(0.0, 0.0);
         }
-        // only the row zeros above must land before other threads' atomics
-        if (MODE != 2 && !fits) __threadfence();
+        // the row zeros above land before other threads' atomics, where the
+        // bounds leave room for any (the fence writes the L2 back: 219 us with
+        // it, 97 without for 600 pairs of 1500 bins and 1.3e4 facets)
+        if (MODE != 2 && top - base > WIN) __threadfence();
         __syncthreads();
 
         for (int k = threadIdx.x; k < V; k += NTT) {
@@ -1918,7 +1977,6 @@ __global__ void __launch_bounds__(NTT) k_target_accum(
             }
         }
     } else {
-        static_assert(MODE != 0, "the deterministic mode of MODE 0 is k_target_accum_fast");
         // the largest component of this pair's terms (not needed by the
         // second pass of MODE 2, which reads its shot's bound)
         __shared__ float red[NTT / 64];
@@ -3247,18 +3305,9 @@ __device__ __forceinline__ void refr0_term(const Rec& rec, int64_t rr, double tx
         Iu = e.x;
         Iv = e.y;
     }
-    const float Iph = rec.ang[rec.cap + rr], Rth = rec.ang[2 * rec.cap + rr];
-    const float Tth = atan2f(sT, cT);
-    const float Tph = atan2f(Iu, Iv);
-    const float si = sinf(Rth - Tth), dph = Iph - Tph;
-    const float a1 = sinc_f(kp.fs_lam * si * cosf(dph)), a2 = sinc_f(kp.fs_lam * si * sinf(dph));
-    const float vi = kp.fs2_lam * a1 * a2;
+    float vi, vo;
+    spec_factors_angles(sT, cT, Iu, Iv, rec, rr, kp, &vi, &vo);
     EI *= vi * vi;
-    const float sR = kp.sqrt_e2e1 * sinf(ERP_PI_F - Tth);
-    const float RrTh = (sR > 1.f) ? 1e4f : asinf(sR);
-    const float so = sinf(RrTh), dpo = Tph - Iph;
-    const float b1 = sinc_f(kp.fs_lam * so * cosf(dpo)), b2 = sinc_f(kp.fs_lam * so * sinf(dpo));
-    const float vo = kp.fs2_lam * b1 * b2;
     EO *= vo * vo;
     const double sl = Itd + Ttd;
     const double sl2 = sl * sl;
@@ -3266,7 +3315,7 @@ __device__ __forceinline__ void refr0_term(const Rec& rec, int64_t rr, double tx
                                                    kp.fs * kp.fs) /
                                            (ERP_FOURPI5_SQ * sl2 * sl2)));
     // refrRadarSignal passes d_Tth to rerad_funct (sim.cu:930-934)
-    const float amp = rerad_f(kp.rerad, Tth) * EI * EO * req;
+    const float amp = rerad_f(kp.rerad, atan2f(sT, cT)) * EI * EO * req;
     const double rngt = madd_nc(sl - Ttd, Ttd, kp.cc2);
     const float2 ph = phasor_cycles(-2.0 * rngt * kp.inv_cyc);
     *R = rngt;
@@ -4784,11 +4833,12 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
                         ERP_CHECK_LAUNCH("k_target_accum_fast");
                     } else {
                         auto kern1 = det ? k_target_accum<1, true> : k_target_accum<1, false>;
-                        hipLaunchKernelGGL(kern1, dim3(n), dim3(NTT), sizeof(double2) * TWIN, st,
+                        hipLaunchKernelGGL(kern1, dim3(n), dim3(NTT), accum_lds(1, nr), st,
                                            targets->xyzn.as<float>(), Tpad, dps, dpt, dshots, dV,
                                            dbase, rec, dbounds, dpr, (int)nprisms, kp, A, Bs,
-                                           nullptr, (unsigned*)nullptr, (const int*)nullptr, 0,
-                                           det ? W.oow.as<int>() : nullptr);
+                                           (unsigned*)nullptr, (const int*)nullptr, 0,
+                                           det ? W.oow.as<int>() : nullptr,
+                                           accum_window(1, nr));
                         ERP_CHECK_LAUNCH("k_target_accum<1>");
                     }
                     PT_.end(st);
@@ -4876,11 +4926,11 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
                                                hipMemcpyHostToDevice, st));
                     if (!det) {
                         hipLaunchKernelGGL(k_target_accum<2>, dim3(n), dim3(NTT),
-                                           sizeof(double2) * TWIN, st, targets->xyzn.as<float>(),
+                                           accum_lds(2, nr), st, targets->xyzn.as<float>(),
                                            Tpad, dps, dps + n, dshots, dV, dbase, rec, dbounds,
-                                           dpr, (int)nprisms, kp, t0, nullptr, nullptr,
+                                           dpr, (int)nprisms, kp, t0, nullptr,
                                            (unsigned*)nullptr, (const int*)nullptr, 0,
-                                           (int*)nullptr);
+                                           (int*)nullptr, accum_window(2, nr));
                         ERP_CHECK_LAUNCH("k_target_accum<2>");
                     } else {
                         // per-shot bounds (the surface's maxima are consumed), then
@@ -4890,11 +4940,12 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
                         auto kern2 = k_target_accum<2, true>;
                         for (int pass = 1; pass <= 2; ++pass) {
                             hipLaunchKernelGGL(kern2, dim3(n), dim3(NTT),
-                                               sizeof(double2) * TWIN, st,
+                                               accum_lds(2, nr), st,
                                                targets->xyzn.as<float>(), Tpad, dps, dps + n,
                                                dshots, dV, dbase, rec, dbounds, dpr, (int)nprisms,
-                                               kp, t0, nullptr, nullptr, smax,
-                                               (const int*)W.tcnt.as<int>(), pass, (int*)nullptr);
+                                               kp, t0, nullptr, smax,
+                                               (const int*)W.tcnt.as<int>(), pass, (int*)nullptr,
+                                               accum_window(2, nr));
                             ERP_CHECK_LAUNCH("k_target_accum<2>");
                         }
                         hipLaunchKernelGGL(k_fix_rows, dim3(grid_for((size_t)P * S)), dim3(256), 0,
