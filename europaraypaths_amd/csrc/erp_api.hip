@@ -138,7 +138,8 @@ void release_work(WorkBufs& w) {
 
 int* alloc_pin() {
     void* p = nullptr;
-    ERP_HIP_TRY(hipHostMalloc(&p, sizeof(int) * kPinWords, hipHostMallocDefault));
+    ERP_HIP_TRY(hipHostMalloc(&p, sizeof(int) * kPinWords,
+                              hipHostMallocMapped | hipHostMallocCoherent));
     return static_cast<int*>(p);
 }
 

@@ -212,12 +212,14 @@ constexpr int kNarrowSlice = 32;  // pairs per slice
 // that the rows of a slice, read side by side, fall on different channels
 inline int narrow_stride(int P) { return P / 2 + 32; }
 
-// Pinned host words of a run: the counts of a batch (up to kPinCounts: V per
-// shot, U per block of two), the target counts, the window check, then
-// target lists of up to kPinList entries.
-constexpr int kPinCounts = 128;
+// Pinned host words of a run, which the kernels write directly (a copy back
+// is a launch of its own, 4.7 us): the counts of a batch (V per row, then U per
+// block of two), the target counts, the window check, then target lists of up
+// to kPinList entries.  Sizes for the rows of a multi-track batch.
+constexpr int kPinCounts = 384;
+constexpr int kPinTargets = 512;
 constexpr size_t kPinList = 16384;
-constexpr size_t kPinWords = 512 + kPinList;
+constexpr size_t kPinWords = kPinCounts + kPinTargets + 8 + kPinList;
 
 struct WorkBufs {
     int* pin = nullptr;  // kPinWords pinned words, owned by the context or slot

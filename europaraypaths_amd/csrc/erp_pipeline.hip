@@ -406,39 +406,35 @@ __global__ void k_pair_targets(int* __restrict__ ptgt, const int* __restrict__ p
     if (i == 0) *next_pair = 0;  // the target kernel's pair counter
 }
 
-__global__ void k_init_bounds(Bounds* b, int S) {
-    int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s < S) {
-        b[s].itd_min = ~0ull; b[s].itd_max = 0ull;
-        b[s].xmin = b[s].ymin = b[s].zmin = 0xFFFFFFFFu;
-        b[s].xmax = b[s].ymax = b[s].zmax = 0u;
-        b[s].cx = b[s].cy = b[s].cz = 0.f;
-        b[s].rad = -1.f;
-    }
-}
-
 // What a batch needs before its surface kernel, in one launch: the record
-// bases (exclusive sums of V over the shots and of U over the blocks of two
-// shots; S <= 64, one wave), the shots' bounds, and the buffers that are
-// summed into cleared: the surface bins and the spectral sums to zero, the
-// block records' Itd to -1 ("not lit").  Sizes in 8-byte words.
+// bases (exclusive sums of V over the rows and of U over the blocks of two
+// rows; S <= 256; rows of a multi-track batch without targets keep none), the
+// rows' bounds, and the buffers that are summed into cleared: the surface bins
+// and the spectral sums to zero, the block records' Itd to -1 ("not lit").
+// Sizes in 8-byte words.
 __global__ void __launch_bounds__(256) k_batch_prep(
     const int* __restrict__ V, const int* __restrict__ U, int S, int64_t* __restrict__ base,
     int64_t* __restrict__ ubase, Bounds* __restrict__ b, double* __restrict__ z0, size_t n0,
-    double* __restrict__ z1, size_t n1, double* __restrict__ itd, size_t ni) {
-    if (blockIdx.x == 0 && threadIdx.x < 64) {
+    double* __restrict__ z1, size_t n1, double* __restrict__ itd, size_t ni,
+    const TrackK* __restrict__ trk, const RowK* __restrict__ rows) {
+    __shared__ int64_t sum[256];
+    if (blockIdx.x == 0) {
         const int s = threadIdx.x;
-        auto scan = [&](int n, const int* v, int64_t* out) {
-            int64_t x = s < n ? v[s] : 0;
-            const int64_t own = x;
-            for (int o = 1; o < 64; o <<= 1) {
-                const int64_t y = __shfl_up(x, o);
-                if (s >= o) x += y;
+        auto scan = [&](int n, int per, const int* v, int64_t* out) {
+            int64_t own = 0;
+            if (s < n && (!trk || (rows[per * s].shot >= 0 && trk[rows[per * s].trk].T > 0)))
+                own = v[s];
+            int64_t x = own;
+            for (int o = 1; o < 256; o <<= 1) {
+                sum[s] = x;
+                __syncthreads();
+                if (s >= o) x += sum[s - o];
+                __syncthreads();
             }
             if (s < n) out[s] = x - own;
         };
-        if (base) scan(S, V, base);
-        if (ubase) scan((S + 1) / 2, U, ubase);
+        if (base) scan(S, 1, V, base);
+        if (ubase) scan((S + 1) / 2, 2, U, ubase);
         if (s < S) {
             b[s].itd_min = ~0ull; b[s].itd_max = 0ull;
             b[s].xmin = b[s].ymin = b[s].zmin = 0xFFFFFFFFu;
@@ -601,19 +597,21 @@ __global__ void __launch_bounds__(1024) k_scan_blocks(
     const int* __restrict__ cnt, int* __restrict__ off, int* __restrict__ V, int nblk, int S,
     const int* __restrict__ cnt2, int* __restrict__ off2, int* __restrict__ V2,
     const TrackK* __restrict__ trk, const RowK* __restrict__ rows,
-    const RowK* __restrict__ rows2) {
+    const RowK* __restrict__ rows2, int* __restrict__ hV, int* __restrict__ hU) {
+    // hV, hU: the host's copies of V and V2 (pinned memory)
     int s = blockIdx.x;
     if (s >= S) {
         s -= S;
         cnt = cnt2;
         off = off2;
         V = V2;
+        hV = hU;
         rows = rows2;
     }
     // rows of a multi-track batch: stride nblk, the row's mesh's own count;
     // a padding row (shot -1) illuminates nothing
     if (trk && rows[s].shot < 0) {
-        if (threadIdx.x == 0) V[s] = 0;
+        if (threadIdx.x == 0) V[s] = hV[s] = 0;
         return;
     }
     const int n = trk ? trk[rows[s].trk].nblk : nblk;
@@ -637,7 +635,7 @@ __global__ void __launch_bounds__(1024) k_scan_blocks(
         if (threadIdx.x == 1023) carry += buf[1023];
         __syncthreads();
     }
-    if (threadIdx.x == 0) V[s] = carry;
+    if (threadIdx.x == 0) V[s] = hV[s] = carry;
 }
 
 // ---------------------------------------------------------------------------
@@ -1539,7 +1537,9 @@ __global__ void __launch_bounds__(1024) k_target_select(
     const float* __restrict__ tg, int64_t Tpad, int T, const unsigned char* __restrict__ ttype,
     const erp_shot* __restrict__ shots, const int* __restrict__ Vs, double cos_ap,
     int* __restrict__ list1, int* __restrict__ list0, int* __restrict__ tcnt, int Tcap,
-    const TrackK* __restrict__ trk, const RowK* __restrict__ rows) {
+    const TrackK* __restrict__ trk, const RowK* __restrict__ rows, int* __restrict__ hcnt,
+    int* __restrict__ hlist) {
+    // hcnt, hlist: the host's copies of tcnt and (short lists) of list1
 #pragma clang fp contract(off)
     const int s = blockIdx.x;
     if (trk) {
@@ -1593,12 +1593,15 @@ __global__ void __launch_bounds__(1024) k_target_select(
             run1 += a;
             run0 += b;
         }
-        if (in1) list1[(size_t)s * Tcap + o1] = t;
+        if (in1) {
+            list1[(size_t)s * Tcap + o1] = t;
+            if (hlist) hlist[(size_t)s * Tcap + o1] = t;
+        }
         if (in0) list0[(size_t)s * Tcap + o0] = t;
     }
     if (threadIdx.x == 0) {
-        tcnt[2 * s] = run1;
-        tcnt[2 * s + 1] = run0;
+        tcnt[2 * s] = hcnt[2 * s] = run1;
+        tcnt[2 * s + 1] = hcnt[2 * s + 1] = run0;
     }
 }
 
@@ -3143,14 +3146,6 @@ __global__ void k_union_mask(const unsigned long long* __restrict__ mask, int nb
     if (w == 0) ucnt[(size_t)j * nblk + blk] = c_s;
 }
 
-// block records not written by a shot read as "not lit": Itd -1
-__global__ void k_fill_itd(double2* __restrict__ p, int64_t n) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x)
-        p[i] = make_double2(-1.0, -1.0);
-}
-
-
 // S[s][k] += scale * sum over the shot's pairs of X[p][k] * Z[p][k]
 __global__ void k_accum_spectra(float2* __restrict__ S, const float2* __restrict__ X,
                                 const float2* __restrict__ Z, const int* __restrict__ seg_shot,
@@ -4383,12 +4378,11 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
         W.uoff.ensure(sizeof(int) * (size_t)nbk_max * nblk);
         W.ubase.ensure(sizeof(int64_t) * (size_t)nbk_max);
     }
-    // counts come back through pinned memory: one wait per read, whatever
-    // the number of arrays
+    // counts come back through pinned memory
     int* const hV = W.pin;                       // V, then U from Smax on
     int* const hU = hV + Smax;
     int* const htc = hV + kPinCounts;            // target counts
-    int* const hoow = htc + 2 * kShotsPerBatch;  // the window check's count
+    int* const hoow = htc + kPinTargets;         // the window check's count
     int* const hlist = hoow + 1;                 // short target lists
     int* dV = W.V.as<int>();
     int* dU = dV + Smax;
@@ -4422,7 +4416,7 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
                                W.cnt.as<int>(), W.off.as<int>(), dV, nblk, shots_,
                                (const int*)W.ucnt.as<int>(), W.uoff.as<int>(), dU,
                                (const TrackK*)nullptr, (const RowK*)nullptr,
-                               (const RowK*)nullptr);
+                               (const RowK*)nullptr, hV, hU);
             ERP_CHECK_LAUNCH("k_scan_blocks");
         };
         auto unite = [&](int shots_) {
@@ -4434,9 +4428,7 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
         if (pairk) unite(S);
         scan(S, nbk);
         PT_.end(st);
-        ERP_HIP_TRY(hipMemcpyAsync(hV, dV, sizeof(int) * ((size_t)Smax + nbk),
-                                   hipMemcpyDeviceToHost, st));
-        ERP_HIP_TRY(hipStreamSynchronize(st));
+        ERP_HIP_TRY(hipStreamSynchronize(st));  // hV, hU
         auto brec_need = [](size_t cap) {
             return 5 * Arena::round(cap * 16) + Arena::round(cap * 4);
         };
@@ -4453,7 +4445,6 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
                 nbk = 1;
                 unite(1);
                 scan(0, 1);
-                ERP_HIP_TRY(hipMemcpyAsync(hU, dU, sizeof(int), hipMemcpyDeviceToHost, st));
                 ERP_HIP_TRY(hipStreamSynchronize(st));
                 if (brec_need((size_t)hU[0]) <= W.brec.bytes) fitb = 1;
             }
@@ -4552,7 +4543,8 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
                                st, (const int*)dV, (const int*)dU, S, need_rec ? dbase : nullptr,
                                pairk ? W.ubase.as<int64_t>() : nullptr, dbounds,
                                W.srow.as<double>(), n0, W.shotS.as<double>(), n1,
-                               reinterpret_cast<double*>(brk.rec.itd), ni);
+                               reinterpret_cast<double*>(brk.rec.itd), ni,
+                               (const TrackK*)nullptr, (const RowK*)nullptr);
             ERP_CHECK_LAUNCH("k_batch_prep");
         }
         double Vsum = 0;
@@ -4642,22 +4634,17 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
             const int Tcap = (int)T;
             int* list1 = W.tlist.as<int>();
             int* list0 = list1 + (size_t)S * Tcap;
+            // short lists come with their counts; long ones once the longest
+            // is known
+            const bool short_lists = pairk && (size_t)S * Tcap <= kPinList;
             PT_.begin(ERP_STAGE_TARGET_SELECT, st, (double)T * S);
             hipLaunchKernelGGL(k_target_select, dim3(S), dim3(1024), 0, st,
                                targets->xyzn.as<float>(), Tpad, (int)T,
                                targets->type.as<unsigned char>(), dshots, dV, p.cos_ap, list1,
                                list0, W.tcnt.as<int>(), Tcap, (const TrackK*)nullptr,
-                               (const RowK*)nullptr);
+                               (const RowK*)nullptr, htc, short_lists ? hlist : nullptr);
             ERP_CHECK_LAUNCH("k_target_select");
             PT_.end(st);
-            ERP_HIP_TRY(hipMemcpyAsync(htc, W.tcnt.p, sizeof(int) * 2 * S, hipMemcpyDeviceToHost,
-                                       st));
-            // short lists come with their counts; long ones once the longest
-            // is known
-            const bool short_lists = pairk && (size_t)S * Tcap <= kPinList;
-            if (short_lists)
-                ERP_HIP_TRY(hipMemcpyAsync(hlist, list1, sizeof(int) * (size_t)S * Tcap,
-                                           hipMemcpyDeviceToHost, st));
             ERP_HIP_TRY(hipStreamSynchronize(st));
             const erp_prism* dpr = nprisms > 0 ? W.prisms.as<erp_prism>() : nullptr;
 
@@ -5048,11 +5035,13 @@ constexpr int kMtRowsMax = 256;
 
 struct MtState {
     MtKey key;
-    DevBuf trk, rows, shots, cnt, off, V, mask, bounds, base, psurf, srow, refl, Sacc, blu,
+    // rows: shots, rows, first rows of the blocks (one upload per batch);
+    // tabs: item count, tables, items (one per launch)
+    DevBuf trk, rows, cnt, off, V, mask, bounds, base, psurf, srow, refl, Sacc, blu,
         list, tcnt, A, Z, tabs, dtabs, rec;
     // shot-pair kernel: union masks, counts, offsets, sizes, first records
-    // and first rows per block of two rows; work items and their count
-    DevBuf umask, ucnt, uoff, U, ubase, brows, items;
+    // per block of two rows
+    DevBuf umask, ucnt, uoff, U, ubase;
     DevBuf bbox;  // facet block boxes of the rows (bounding spheres)
     MtGraph gA1, gA2, gChunk, gTail;
     void reset_graphs() {
@@ -5063,9 +5052,9 @@ struct MtState {
     }
     void release() {
         reset_graphs();
-        DevBuf* b[] = {&trk, &rows, &shots, &cnt, &off, &V, &mask, &bounds, &base, &psurf, &srow,
+        DevBuf* b[] = {&trk, &rows, &cnt, &off, &V, &mask, &bounds, &base, &psurf, &srow,
                        &refl, &Sacc, &blu, &list, &tcnt, &A, &Z, &tabs, &dtabs, &rec,
-                       &umask, &ucnt, &uoff, &U, &ubase, &brows, &items, &bbox};
+                       &umask, &ucnt, &uoff, &U, &ubase, &bbox};
         for (DevBuf* d : b) d->release();
         key = MtKey{};
     }
@@ -5240,8 +5229,7 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
     }
     const size_t r = (size_t)R;
     m.trk.ensure(sizeof(TrackK) * (size_t)ntr);
-    m.rows.ensure(sizeof(RowK) * r);
-    m.shots.ensure(sizeof(erp_shot) * r);
+    m.rows.ensure((sizeof(erp_shot) + sizeof(RowK)) * r + sizeof(RowK) * (size_t)nbk);
     m.cnt.ensure(sizeof(int) * r * nblk_max);
     m.off.ensure(sizeof(int) * r * nblk_max);
     m.V.ensure(sizeof(int) * r);
@@ -5266,7 +5254,8 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
     // host-written tables of a launch: pair rows and list indices, slices,
     // segments, the pair count, segment scales
     const size_t tab_ints = 2 * (size_t)C + 2 * (size_t)gcap + 3 * (size_t)segcap + 1 + segcap;
-    m.tabs.ensure(sizeof(int) * tab_ints);
+    const size_t tab_head = (16 + sizeof(int) * tab_ints + 15) & ~(size_t)15;
+    m.tabs.ensure(tab_head + (pairk ? sizeof(int4) * (size_t)C : 0));
     // device-written: pair window bases and lengths, the pair counter, the
     // per-pair range kernel spectra and windows
     m.dtabs.ensure(sizeof(int) * (2 * (size_t)C + 64) + 2 * sizeof(void*) * (size_t)C);
@@ -5276,12 +5265,10 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
         m.uoff.ensure(sizeof(int) * (size_t)nbk * nblk_max);
         m.U.ensure(sizeof(int) * (size_t)nbk);
         m.ubase.ensure(sizeof(int64_t) * (size_t)nbk);
-        m.brows.ensure(sizeof(RowK) * (size_t)nbk);
-        m.items.ensure(sizeof(int4) * (size_t)C + 64);  // items, then their count
     }
-    int4* d_items = m.items.as<int4>();
-    int* d_nitems = reinterpret_cast<int*>(d_items + C);
-    int* t_pshot = m.tabs.as<int>();
+    int* d_nitems = m.tabs.as<int>();
+    int4* d_items = reinterpret_cast<int4*>(m.tabs.as<char>() + tab_head);
+    int* t_pshot = d_nitems + 4;
     int* t_ptgt = t_pshot + C;
     int* t_slb = t_ptgt + C;
     int* t_sle = t_slb + gcap;
@@ -5299,8 +5286,9 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
     ERP_HIP_TRY(hipMemcpyAsync(m.trk.p, tk.data(), sizeof(TrackK) * (size_t)ntr,
                                hipMemcpyHostToDevice, st));
     const TrackK* dtrk = m.trk.as<TrackK>();
-    const RowK* drows = m.rows.as<RowK>();
-    const erp_shot* dshots = m.shots.as<erp_shot>();
+    const erp_shot* dshots = m.rows.as<erp_shot>();
+    const RowK* drows = reinterpret_cast<const RowK*>(dshots + r);
+    const RowK* dbrows = drows + r;
     int* dV = m.V.as<int>();
     Bounds* dbounds = m.bounds.as<Bounds>();
     int64_t* dbase = m.base.as<int64_t>();
@@ -5320,15 +5308,21 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
     }
 
     if (targ) ERP_HIP_TRY(hipMemsetAsync(d_next + 1, 0, sizeof(int), st));  // window check
-    std::vector<RowK> hrows(r);
-    std::vector<erp_shot> hshots(r);
-    std::vector<int> hV(r), htc(2 * r), tc1(r), hU(nbk);
-    std::vector<int64_t> hbase(r), hubase(nbk);
-    std::vector<RowK> hbrows(nbk);
+    std::vector<char> hrow_buf((sizeof(erp_shot) + sizeof(RowK)) * r + sizeof(RowK) * nbk);
+    erp_shot* hshots = reinterpret_cast<erp_shot*>(hrow_buf.data());
+    RowK* hrows = reinterpret_cast<RowK*>(hshots + r);
+    RowK* hbrows = hrows + r;
+    // written by the kernels (pinned): counts, target counts, short lists
+    int* const hV = ctx->work.pin;
+    int* const hU = hV + R;
+    int* const htc = hV + kPinCounts;
+    int* const hlist = htc + kPinTargets + 1;
+    const bool short_lists = pairk && r * (size_t)Tcap <= kPinList;
+    std::vector<int> tc1(r);
     std::vector<std::vector<PairIdx>> bl;
     PairChunk pc;
-    std::vector<int4> hitems;
-    std::vector<int> htab(tab_ints);
+    std::vector<char> htab_buf(tab_head + (pairk ? sizeof(int4) * (size_t)C : 0));
+    int* const htab = reinterpret_cast<int*>(htab_buf.data()) + 4;
     StageTimer none_;
     StageTimer& PT_ = ctx->prof.on ? ctx->prof : none_;
     ChunkFill cf;
@@ -5341,16 +5335,10 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
             const erp_track& t = tracks[trk_idx[row.trk]];
             hshots[i] = t.shots[row.shot < 0 ? 0 : row.shot];
         }
-        ERP_HIP_TRY(hipMemcpyAsync(m.rows.p, hrows.data(), sizeof(RowK) * r,
+        // a block's rows share a track: its first row names it
+        for (int j = 0; j < nbk; ++j) hbrows[j] = hrows[2 * j];
+        ERP_HIP_TRY(hipMemcpyAsync(m.rows.p, hrow_buf.data(), hrow_buf.size(),
                                    hipMemcpyHostToDevice, st));
-        ERP_HIP_TRY(hipMemcpyAsync(m.shots.p, hshots.data(), sizeof(erp_shot) * r,
-                                   hipMemcpyHostToDevice, st));
-        if (pairk) {
-            // a block's rows share a track: its first row names it
-            for (int j = 0; j < nbk; ++j) hbrows[j] = hrows[2 * j];
-            ERP_HIP_TRY(hipMemcpyAsync(m.brows.p, hbrows.data(), sizeof(RowK) * nbk,
-                                       hipMemcpyHostToDevice, st));
-        }
 
         // A1: aperture masks, counts
         PT_.begin(ERP_STAGE_MASK, st, 0.0);
@@ -5370,20 +5358,15 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
             hipLaunchKernelGGL(k_scan_blocks, dim3(R + (pairk ? nbk : 0)), dim3(1024), 0, st,
                                m.cnt.as<int>(), m.off.as<int>(), dV, nblk_max, R,
                                (const int*)m.ucnt.as<int>(), m.uoff.as<int>(), m.U.as<int>(), dtrk,
-                               drows, (const RowK*)m.brows.as<RowK>());
+                               drows, dbrows, hV, hU);
             ERP_CHECK_LAUNCH("k_scan_blocks");
         });
         PT_.end(st);
-        ERP_HIP_TRY(hipMemcpyAsync(hV.data(), dV, sizeof(int) * r, hipMemcpyDeviceToHost, st));
-        if (pairk)
-            ERP_HIP_TRY(hipMemcpyAsync(hU.data(), m.U.p, sizeof(int) * nbk, hipMemcpyDeviceToHost,
-                                       st));
         ERP_HIP_TRY(hipStreamSynchronize(st));
 
         // facet records of the rows whose track has targets
         int64_t Vtot = 0;
         for (size_t i = 0; i < r; ++i) {
-            hbase[i] = Vtot;
             const bool keep = hrows[i].shot >= 0 && tk[hrows[i].trk].T > 0;
             if (keep && hV[i] >= (1 << 28))
                 throw ErpError{ERP_E_INVALID, "a shot illuminates 2^28 facets or more"};
@@ -5392,14 +5375,11 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
         if (pairk) {
             // block records: the union of each block's two rows
             for (int j = 0; j < nbk; ++j) {
-                hubase[j] = Vtot;
                 const bool keep = hrows[2 * j].shot >= 0 && tk[hrows[2 * j].trk].T > 0;
                 if (keep && hU[j] >= (1 << 28))
                     throw ErpError{ERP_E_INVALID, "two shots illuminate 2^28 facets or more"};
                 if (keep) Vtot += hU[j];
             }
-            ERP_HIP_TRY(hipMemcpyAsync(m.ubase.p, hubase.data(), sizeof(int64_t) * nbk,
-                                       hipMemcpyHostToDevice, st));
         }
         auto rnd = [](size_t n) { return (n + 255) & ~(size_t)255; };
         // bytes of cap records in this group's layout: block records (84 B)
@@ -5445,22 +5425,19 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
             rec.qd = (float*)take(cap * 4);
             rec.cap = (int64_t)cap;
         }
-        ERP_HIP_TRY(hipMemcpyAsync(dbase, hbase.data(), sizeof(int64_t) * r,
-                                   hipMemcpyHostToDevice, st));
 
         // A2: surface kernel, surface range compression, target selection
         double Vsum = 0;
         for (size_t i = 0; i < r; ++i) Vsum += hV[i];
         PT_.begin(ERP_STAGE_SURFACE, st, Vsum);
         mt_launch(m.gA2, direct, st, [&] {
-            if (pairk) {
-                hipLaunchKernelGGL(k_fill_itd, dim3(grid_for(m.key.reccap)), dim3(256), 0, st,
-                                   brk.rec.itd, (int64_t)m.key.reccap);
-                ERP_CHECK_LAUNCH("k_fill_itd");
-            }
-            hipLaunchKernelGGL(k_init_bounds, dim3((R + 63) / 64), dim3(64), 0, st, dbounds, R);
-            ERP_CHECK_LAUNCH("k_init_bounds");
-            zero(m.srow.as<float2>(), srow_f2, st);
+            const size_t n1 = targ ? r * sumP : 0, ni = pairk ? 2 * m.key.reccap : 0;
+            hipLaunchKernelGGL(k_batch_prep, dim3(grid_for(srow_f2 + n1 + ni, 256, 4096)),
+                               dim3(256), 0, st, (const int*)dV, (const int*)m.U.as<int>(), R,
+                               dbase, pairk ? m.ubase.as<int64_t>() : nullptr, dbounds,
+                               m.srow.as<double>(), srow_f2, m.Sacc.as<double>(), n1,
+                               reinterpret_cast<double*>(brk.rec.itd), ni, dtrk, drows);
+            ERP_CHECK_LAUNCH("k_batch_prep");
             hipLaunchKernelGGL(k_surface, dim3(nblk_max, R), dim3(NT), 0, st,
                                (const float*)nullptr, (int64_t)0, (int64_t)0, dshots,
                                m.mask.as<unsigned long long>(), m.off.as<int>(), dV, dbase,
@@ -5489,9 +5466,9 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
                 hipLaunchKernelGGL(k_target_select, dim3(R), dim3(1024), 0, st,
                                    (const float*)nullptr, (int64_t)0, 0,
                                    (const unsigned char*)nullptr, dshots, dV, 0.0, list1, list0,
-                                   m.tcnt.as<int>(), Tcap, dtrk, drows);
+                                   m.tcnt.as<int>(), Tcap, dtrk, drows, htc,
+                                   short_lists ? hlist : nullptr);
                 ERP_CHECK_LAUNCH("k_target_select");
-                zero(m.Sacc.as<float2>(), r * sumP, st);
             } else {
                 hipLaunchKernelGGL(k_finalize_rows, dim3(grid_for(r * nr)), dim3(256), 0, st,
                                    m.refl.as<float2>(), dV, nr, R, dtrk, drows);
@@ -5501,8 +5478,6 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
         PT_.end(st);
         if (!targ) continue;
 
-        ERP_HIP_TRY(hipMemcpyAsync(htc.data(), m.tcnt.p, sizeof(int) * 2 * r,
-                                   hipMemcpyDeviceToHost, st));
         ERP_HIP_TRY(hipStreamSynchronize(st));
         for (size_t i = 0; i < r; ++i) tc1[i] = htc[2 * i];
 
@@ -5528,32 +5503,33 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
             // the rows' target lists; launches of whole items of at most C rows
             int maxc = 0;
             for (size_t i = 0; i < r; ++i) maxc = std::max(maxc, htc[2 * i]);
-            std::vector<int> hl(r * (size_t)maxc);
-            if (maxc > 0) {
+            std::vector<int> hl(short_lists ? 0 : r * (size_t)maxc);
+            if (maxc > 0 && !short_lists) {
                 ERP_HIP_TRY(hipMemcpy2DAsync(hl.data(), sizeof(int) * maxc, list1,
                                              sizeof(int) * Tcap, sizeof(int) * maxc, r,
                                              hipMemcpyDeviceToHost, st));
                 ERP_HIP_TRY(hipStreamSynchronize(st));
             }
-            merge_pair_lists(hl.data(), (size_t)maxc, htc.data(), R, bl);
+            merge_pair_lists(short_lists ? hlist : hl.data(), (size_t)(short_lists ? Tcap : maxc),
+                             htc, R, bl);
             int jb = 0;
             size_t ib = 0;
             PairCursor cur;
             for (;;) {
                 // deterministic: every row's slices independent of the launches
-                if (det) fill_pair_chunk_canon(bl, cur, C, GS, hV.data(), pc);
-                else fill_pair_chunk(bl, jb, ib, C, GS, hV.data(), pc);
+                if (det) fill_pair_chunk_canon(bl, cur, C, GS, hV, pc);
+                else fill_pair_chunk(bl, jb, ib, C, GS, hV, pc);
                 const int n = pc.rows;
                 if (n == 0) break;
                 const int nsl = (int)pc.gb.size(), nseg = (int)pc.sg_s.size();
                 const int nit = (int)pc.items.size();
                 if (nsl > gcap || nseg > segcap)
                     throw ErpError{ERP_E_INVALID, "multi-track launch tables overflow"};
-                std::fill(htab.begin(), htab.end(), 0);
-                std::copy(pc.rshot.begin(), pc.rshot.end(), htab.begin());
-                std::copy(pc.ridx.begin(), pc.ridx.end(), htab.begin() + C);
-                std::copy(pc.gb.begin(), pc.gb.end(), htab.begin() + 2 * C);
-                std::copy(pc.ge.begin(), pc.ge.end(), htab.begin() + 2 * C + gcap);
+                std::fill(htab, htab + tab_ints, 0);
+                std::copy(pc.rshot.begin(), pc.rshot.end(), htab);
+                std::copy(pc.ridx.begin(), pc.ridx.end(), htab + C);
+                std::copy(pc.gb.begin(), pc.gb.end(), htab + 2 * C);
+                std::copy(pc.ge.begin(), pc.ge.end(), htab + 2 * C + gcap);
                 const size_t so = 2 * (size_t)C + 2 * gcap;
                 for (int k = 0; k < nseg; ++k) {
                     htab[so + k] = pc.sg_s[k];
@@ -5563,15 +5539,11 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
                     std::memcpy(&htab[so + 3 * segcap + 1 + k], &sc, sizeof(float));
                 }
                 htab[so + 3 * segcap] = n;
-                ERP_HIP_TRY(hipMemcpyAsync(m.tabs.p, htab.data(), sizeof(int) * tab_ints,
-                                           hipMemcpyHostToDevice, st));
-                hitems.resize((size_t)C + 1);
-                std::copy(pc.items.begin(), pc.items.end(), hitems.begin());
-                hitems[C] = make_int4(nit, 0, 0, 0);
-                ERP_HIP_TRY(hipMemcpyAsync(d_items, hitems.data(), sizeof(int4) * nit,
-                                           hipMemcpyHostToDevice, st));
-                ERP_HIP_TRY(hipMemcpyAsync(d_items + C, hitems.data() + C, sizeof(int4),
-                                           hipMemcpyHostToDevice, st));
+                htab[-4] = nit;
+                std::memcpy(htab_buf.data() + tab_head, pc.items.data(), sizeof(int4) * nit);
+                ERP_HIP_TRY(hipMemcpyAsync(m.tabs.p, htab_buf.data(),
+                                           tab_head + sizeof(int4) * nit, hipMemcpyHostToDevice,
+                                           st));
                 PT_.begin(ERP_STAGE_TARGET_ACCUM, st, pc.triples);
                 mt_launch(m.gChunk, direct, st, [&] {
                     // windows, range kernel spectra per row, the item counter cleared
@@ -5609,11 +5581,11 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
             const int nsl = (int)cf.gb.size(), nseg = (int)cf.sg_s.size();
             if (nsl > gcap || nseg > segcap)
                 throw ErpError{ERP_E_INVALID, "multi-track launch tables overflow"};
-            std::fill(htab.begin(), htab.end(), 0);
-            std::copy(cf.pshot.begin(), cf.pshot.end(), htab.begin());
-            std::copy(cf.ptgt.begin(), cf.ptgt.end(), htab.begin() + C);
-            std::copy(cf.gb.begin(), cf.gb.end(), htab.begin() + 2 * C);
-            std::copy(cf.ge.begin(), cf.ge.end(), htab.begin() + 2 * C + gcap);
+            std::fill(htab, htab + tab_ints, 0);
+            std::copy(cf.pshot.begin(), cf.pshot.end(), htab);
+            std::copy(cf.ptgt.begin(), cf.ptgt.end(), htab + C);
+            std::copy(cf.gb.begin(), cf.gb.end(), htab + 2 * C);
+            std::copy(cf.ge.begin(), cf.ge.end(), htab + 2 * C + gcap);
             const size_t so = 2 * (size_t)C + 2 * gcap;
             for (int k = 0; k < nseg; ++k) {
                 htab[so + k] = cf.sg_s[k];
@@ -5623,7 +5595,7 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
                 std::memcpy(&htab[so + 3 * segcap + 1 + k], &sc, sizeof(float));
             }
             htab[so + 3 * segcap] = n;
-            ERP_HIP_TRY(hipMemcpyAsync(m.tabs.p, htab.data(), sizeof(int) * tab_ints,
+            ERP_HIP_TRY(hipMemcpyAsync(m.tabs.p, htab_buf.data(), tab_head,
                                        hipMemcpyHostToDevice, st));
             double triples = 0;
             for (int i = 0; i < n; ++i) triples += hV[cf.pshot[i]];
@@ -5658,7 +5630,7 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
         });
         PT_.end(st);
     }
-    if (targ) check_windows(d_next + 1, ctx->work.pin + kPinCounts, st);
+    if (targ) check_windows(d_next + 1, htc + kPinTargets, st);
 }
 
 }  // namespace
