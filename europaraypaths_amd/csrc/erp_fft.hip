@@ -235,6 +235,75 @@ __device__ __forceinline__ void lds_fft(float2* s, int n, int log2n, int nb, boo
     }
 }
 
+// One transform of n <= 4096 points for latency: 1024 threads, radix 4 (one
+// radix 2 stage first for odd log2 n), a butterfly per thread and stage, the
+// twiddles of every stage in registers, loaded once for all transforms of the
+// kernel.  The 256-thread radix-16 stages do the same work in a quarter of the
+// barriers, but with few rows each is a chain of some 400 instructions and 4
+// loads on a wave that has its SIMD to itself: k_final_small (four transforms a
+// row) takes 24 us for 24 rows of 4096 points instead of 43, k_conv_small (two)
+// 16 instead of 22.
+constexpr int NTW = 1024;
+struct WideTw {
+    float2 w[6][3];
+};
+__device__ __forceinline__ void wide_twiddles(WideTw& t, const float2* __restrict__ lad, int n,
+                                              int log2n) {
+#pragma unroll
+    for (int st = 0; st < 6; ++st) {
+        const int Ls = ((log2n & 1) ? 2 : 1) << (2 * st);
+        if (Ls > 1 && 4 * Ls <= n) {
+            const int k = threadIdx.x & (Ls - 1);
+#pragma unroll
+            for (int e = 1; e < 4; ++e) t.w[st][e - 1] = lad[4 * Ls + e * k];
+        }
+    }
+}
+// s in LDS, synchronised before and after
+__device__ __forceinline__ void wide_fft(float2* s, int n, int log2n, bool inv, const WideTw& t) {
+    const int j = threadIdx.x;
+    if (log2n & 1) {  // n <= 2048
+        float2 a, b;
+        if (j < n / 2) {
+            a = s[sw(j)];
+            b = s[sw(j + n / 2)];
+        }
+        __syncthreads();
+        if (j < n / 2) {
+            s[sw(2 * j)] = cadd(a, b);
+            s[sw(2 * j + 1)] = csub(a, b);
+        }
+        __syncthreads();
+    }
+    const int n4 = n / 4;
+#pragma unroll
+    for (int st = 0; st < 6; ++st) {
+        const int Ls = ((log2n & 1) ? 2 : 1) << (2 * st);
+        if (4 * Ls > n) break;
+        float2 v[4];
+        if (j < n4) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = s[sw(j + i * n4)];
+        }
+        __syncthreads();
+        if (j < n4) {
+            const int k = j & (Ls - 1);
+            if (Ls > 1) {
+#pragma unroll
+                for (int e = 1; e < 4; ++e) {
+                    const float2 w = t.w[st][e - 1];
+                    v[e] = cmul(v[e], make_float2(w.x, inv ? -w.y : w.y));
+                }
+            }
+            dft4(v[0], v[1], v[2], v[3], inv);
+            const int dst = (j - k) * 4 + k;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s[sw(dst + i * Ls)] = v[i];
+        }
+        __syncthreads();
+    }
+}
+
 // Copy ladder entries [0, 2n) (the twiddles of every stage of a length-n
 // transform) into LDS; callers sync before the first stage.
 __device__ __forceinline__ const float2* stage_ladder(float2* twl, const float2* __restrict__ tw,
@@ -587,7 +656,7 @@ __device__ __forceinline__ double surf_inv(int det, const unsigned* __restrict__
 }
 
 // P <= 4096: one workgroup per row
-__global__ void __launch_bounds__(NT) k_conv_small(float2* __restrict__ out,
+__global__ void __launch_bounds__(NTW) k_conv_small(float2* __restrict__ out,
                                                    const double2* __restrict__ srow, int nr,
                                                    int det, const unsigned* __restrict__ smax,
                                                    const int* __restrict__ Vs, int P, int log2P,
@@ -601,21 +670,23 @@ __global__ void __launch_bounds__(NT) k_conv_small(float2* __restrict__ out,
         if (rk[r].shot < 0) return;
         G = trk[rk[r].trk].g_surf;
         if (!G) {
-            for (int n = threadIdx.x; n < nr; n += NT)
+            for (int n = threadIdx.x; n < nr; n += NTW)
                 out[(size_t)r * nr + n] = make_float2(0.f, 0.f);
             return;
         }
     }
+    WideTw t;
+    wide_twiddles(t, tw, P, log2P);
     const double inv = surf_inv(det, smax, Vs, r);
     const double2* row = srow + (size_t)r * nr;
-    for (int n = threadIdx.x; n < P; n += NT)
+    for (int n = threadIdx.x; n < P; n += NTW)
         s[sw(n)] = n < nr ? surf_bin(row, n, det, inv) : make_float2(0.f, 0.f);
     __syncthreads();
-    lds_fft(s, P, log2P, 1, false, tw);
-    for (int n = threadIdx.x; n < P; n += NT) s[sw(n)] = cmul(s[sw(n)], G[n]);
+    wide_fft(s, P, log2P, false, t);
+    for (int n = threadIdx.x; n < P; n += NTW) s[sw(n)] = cmul(s[sw(n)], G[n]);
     __syncthreads();
-    lds_fft(s, P, log2P, 1, true, tw);
-    for (int n = threadIdx.x; n < nr; n += NT) out[(size_t)r * nr + n] = s[sw(n + nr)];
+    wide_fft(s, P, log2P, true, t);
+    for (int n = threadIdx.x; n < nr; n += NTW) out[(size_t)r * nr + n] = s[sw(n + nr)];
 }
 
 // two-pass, first column pass from the surface bins
@@ -689,7 +760,7 @@ __global__ void k_band_scale(float2* __restrict__ tab, int n, float sc) {
 }
 
 // P <= 4096: the whole stage of one row in one workgroup
-__global__ void __launch_bounds__(NT) k_final_small(const float2* __restrict__ S, int P, int log2P,
+__global__ void __launch_bounds__(NTW) k_final_small(const float2* __restrict__ S, int P, int log2P,
                                                     int nr, const float2* tab, FinalOut fo,
                                                     const float2* __restrict__ tw) {
     __shared__ float2 s[NPTS];
@@ -697,15 +768,17 @@ __global__ void __launch_bounds__(NT) k_final_small(const float2* __restrict__ S
     float2* o;
     if (!final_row(fo, r, nr, &o, &tab)) return;
     const float2* x = S + (size_t)r * P;
-    for (int n = threadIdx.x; n < P; n += NT) s[sw(n)] = x[n];
+    WideTw t;
+    wide_twiddles(t, tw, P, log2P);
+    for (int n = threadIdx.x; n < P; n += NTW) s[sw(n)] = x[n];
     __syncthreads();
-    lds_fft(s, P, log2P, 1, true, tw);
+    wide_fft(s, P, log2P, true, t);
     // even and odd samples of c (2 nr - 1 of them), P / 2 each
-    constexpr int H = PPT / 2;
-    float2 ce[H], co[H], acc[PPT];
+    constexpr int H = NPTS / NTW / 2;
+    float2 ce[H], co[H], acc[2 * H];
 #pragma unroll
     for (int q = 0; q < H; ++q) {
-        const int l = threadIdx.x + q * NT;
+        const int l = threadIdx.x + q * NTW;
         ce[q] = l < nr ? s[sw(2 * l)] : make_float2(0.f, 0.f);
         co[q] = l < nr - 1 ? s[sw(2 * l + 1)] : make_float2(0.f, 0.f);
     }
@@ -714,17 +787,17 @@ __global__ void __launch_bounds__(NT) k_final_small(const float2* __restrict__ S
         __syncthreads();
 #pragma unroll
         for (int q = 0; q < H; ++q) {
-            const int l = threadIdx.x + q * NT;
+            const int l = threadIdx.x + q * NTW;
             if (l < P / 2) {
                 s[sw(l)] = h ? co[q] : ce[q];
                 s[sw(l + P / 2)] = make_float2(0.f, 0.f);
             }
         }
         __syncthreads();
-        lds_fft(s, P, log2P, 1, false, tw);
+        wide_fft(s, P, log2P, false, t);
 #pragma unroll
-        for (int q = 0; q < PPT; ++q) {
-            const int n = threadIdx.x + q * NT;
+        for (int q = 0; q < 2 * H; ++q) {
+            const int n = threadIdx.x + q * NTW;
             if (n < P) {
                 const float2 v = cmul(s[sw(n)], tab[(size_t)h * P + n]);
                 acc[q] = h ? cadd(acc[q], v) : v;
@@ -733,14 +806,14 @@ __global__ void __launch_bounds__(NT) k_final_small(const float2* __restrict__ S
     }
     __syncthreads();
 #pragma unroll
-    for (int q = 0; q < PPT; ++q) {
-        const int n = threadIdx.x + q * NT;
+    for (int q = 0; q < 2 * H; ++q) {
+        const int n = threadIdx.x + q * NTW;
         if (n < P) s[sw(n)] = acc[q];
     }
     __syncthreads();
-    lds_fft(s, P, log2P, 1, true, tw);
+    wide_fft(s, P, log2P, true, t);
     const bool live = fo.Vs[r] > 0;
-    for (int n = threadIdx.x; n < nr; n += NT)
+    for (int n = threadIdx.x; n < nr; n += NTW)
         o[n] = final_value(fo, (size_t)r * nr + n, live, s[sw(P / 2 + n)]);
 }
 
@@ -1655,7 +1728,7 @@ void surface_conv_rows(erp_ctx* ctx, const FftPlan& p, const double2* srow, int 
     const float2* tw = ctx->twiddle.as<float2>();
     const int d = det ? 1 : 0;
     if (!p.two_pass) {
-        hipLaunchKernelGGL(k_conv_small, dim3(rows), dim3(NT), 0, st, out, srow, nr, d, smax, Vs,
+        hipLaunchKernelGGL(k_conv_small, dim3(rows), dim3(NTW), 0, st, out, srow, nr, d, smax, Vs,
                            p.N, p.log2N, G, trk, rk, tw);
         ERP_CHECK_LAUNCH("k_conv_small");
         return;
@@ -1702,7 +1775,7 @@ void shot_final_rows(erp_ctx* ctx, const FftPlan& p, float2* S, float2* work, in
     if (rows <= 0) return;
     const float2* tw = ctx->twiddle.as<float2>();
     if (!p.two_pass) {
-        hipLaunchKernelGGL(k_final_small, dim3(1, rows), dim3(NT), 0, st, S, p.N, p.log2N, nr, tab,
+        hipLaunchKernelGGL(k_final_small, dim3(1, rows), dim3(NTW), 0, st, S, p.N, p.log2N, nr, tab,
                            fo, tw);
         ERP_CHECK_LAUNCH("k_final_small");
         return;
