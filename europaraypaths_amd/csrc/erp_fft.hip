@@ -964,10 +964,7 @@ __global__ void k_sum_rows(float2* __restrict__ S, const float2* __restrict__ sr
 //     Ze = DFT(z)   = nr E G_e - T1,   T1 = DFT(conj(m) v)
 //     Zo = DFT(z m) = T2 - nr O G_o,   T2 = DFT(m u)
 //     out[2k] = E Ze,  out[2k+1] = O Zo.
-// Six nr-point transforms per pair: E is parked in the even half of the
-// pair's output row (which only the last step writes) instead of being
-// transformed again, and at most one register array is held across a
-// transform.
+// Six nr-point transforms per pair, three for each half of the frequencies.
 // Gn holds the chirp spectrum in natural order as (G[2k], G[2k+1]) pairs.
 // Each output row (P complex) holds two planes: out[k] = product at
 // frequency 2k, out[n + k] = product at frequency 2k + 1.
@@ -1063,30 +1060,40 @@ __device__ __forceinline__ void load_window(float2 (&x)[PPT], const float2* __re
     }
 }
 
+// One workgroup per pair and one group of NTB threads per half plane: group
+// c = 0 (threadIdx.y) runs the transforms of the even frequencies, group 1
+// those of the odd ones, so that a pair is a chain of three transforms
+// instead of six.  x m^c below: times the half-bin modulation m for c = 1.
+//   0: a m^c      -> E (O)    -> e = E (O) kept in registers; x = conj(E G_e)
+//   1: x          -> conj(u)  (conj(v))
+// nr = n: x = m u (conj(m) v);
+//   2: x          -> T2 (T1)  -> swapped between the groups through LDS;
+//                                plane c = E (n E G_e - T1), O (T2 - n O G_o)
 // CROP: nr < n bins (P = 2n, n the next power of two): the kept window
 // z[j] = y[n + j] holds only j < nr, so z is no longer u - conj(m) v over
 // the whole half and the shortcut DFT(IDFT(x)) = n x does not apply; z is
-// formed in the time domain and transformed twice (still six transforms):
-//   0: a          -> E        -> even plane = E; x = conj(E G_e)
-//   1: x          -> conj(u)  -> h = u
-//   2: a m        -> O        -> odd plane = O; x = conj(O G_o)
-//   3: x          -> conj(v)  -> z = u - conj(m) v for j < nr, 0 above;
-//                                x = z, h = z m
-//   4: x          -> Z_e      -> even plane = E Z_e (E read back)
-//   5: h          -> Z_o      -> odd plane = O Z_o (O read back)
+// formed in the time domain, conj(u) and m conj(v) swapped through LDS:
+//   2: z m^c      -> Z_e (Z_o) -> plane c = E Z_e, O Z_o
 // The range kernel spectrum G is placed for the window at n (kind 2 of
-// k_gen_kernel).  Every thread reads back only what it wrote.
+// k_gen_kernel).  A swapped value goes to the slots that only its own thread
+// read last in fft_regs (element tid + q NTB), so one barrier orders the
+// swap, and fft_regs' first barrier the next transform's writes.
+// Bound by the chain of LDS round trips and barriers for few pairs, by the
+// VALU for many.  Against one group running all six (seven) phases, whole
+// runs of vhf chirps (us): 9 pairs per shot, 100 shots, n = 1024 624 to 570
+// (nr = n 736 to 684); 1 681 targets, 24 shots, n = 1024 4 041 to 3 932,
+// 2048 5 227 to 4 996, 4096 6 559 to 6 231, cropped 4096 6 827 to 6 392.
 template <int NTB, bool MT = false, bool CROP = false>
-__global__ void __launch_bounds__(NTB) k_tpair_half(const float2* __restrict__ A, int P,
-                                                    const int* __restrict__ pbase,
-                                                    const int* __restrict__ pwin,
-                                                    const float4* __restrict__ Gn,
-                                                    float2* __restrict__ out,
-                                                    const float2* __restrict__ lad,
-                                                    const float4* const* __restrict__ Gpair,
-                                                    const int* __restrict__ npairs, int nr) {
+__global__ void __launch_bounds__(2 * NTB) k_tpair_half(const float2* __restrict__ A, int P,
+                                                        const int* __restrict__ pbase,
+                                                        const int* __restrict__ pwin,
+                                                        const float4* __restrict__ Gn,
+                                                        float2* __restrict__ out,
+                                                        const float2* __restrict__ lad,
+                                                        const float4* const* __restrict__ Gpair,
+                                                        const int* __restrict__ npairs, int nr) {
     constexpr int n = NTB * PPT;
-    __shared__ float2 s[n + n / 16];
+    __shared__ float2 sm[2][n + n / 16];
     const int p = blockIdx.x;
     // a multi-track launch: a grid of the pair bound, the count on the
     // device, and each pair's own range kernel spectrum
@@ -1094,91 +1101,66 @@ __global__ void __launch_bounds__(NTB) k_tpair_half(const float2* __restrict__ A
         if (p >= *npairs) return;
         Gn = Gpair[p];
     }
+    // uniform over a wave (NTB is a multiple of 64)
+    const int c = __builtin_amdgcn_readfirstlane(threadIdx.y);
+    float2* s = sm[c];
     const int base = pbase[p], win = pwin[p];
     const float2* a = A + (size_t)p * P;
     const float2* mod = lad + 2 * n;  // m(j) = lad[2n + j]
-    float2* o2 = out + (size_t)p * P;  // even plane [0, n), odd plane [n, 2n)
+    const float2* G = reinterpret_cast<const float2*>(Gn) + c;  // this plane's, stride 2
+    float2* o2 = out + (size_t)p * P + (size_t)c * n;
     const float fn = (float)n;
-    float2 x[PPT], h[PPT];
-    if constexpr (CROP) {
+    float2 x[PPT], e[PPT];
+    load_window<NTB, CROP>(x, a, base, win, c ? mod : nullptr, nr);
 #pragma unroll 1
-        for (int ph = 0; ph < 6; ++ph) {
-            if (ph == 0 || ph == 2)
-                load_window<NTB, true>(x, a, base, win, ph == 2 ? mod : nullptr, nr);
-            if (ph == 5) {
+    for (int ph = 0; ph < 3; ++ph) {
+        fft_regs<NTB>(s, x, lad);
+        const int tid = opaque_tid();
+        float2* own = s + pad16(tid);
+        const float2* other = sm[1 - c] + pad16(tid);
+        if (ph == 0) {
 #pragma unroll
-                for (int q = 0; q < PPT; ++q) x[q] = h[q];
+            for (int q = 0; q < PPT; ++q) {
+                e[q] = x[q];
+                x[q] = conjf2(cmul(x[q], G[2 * (tid + q * NTB)]));
             }
-            fft_regs<NTB>(s, x, lad);
-            const int tid = opaque_tid();
+        } else if (CROP && ph == 1) {
+            // z = u - conj(m) v with x = conj(u), conj(v): conj(x0 - m x1)
+#pragma unroll
+            for (int q = 0; q < PPT; ++q) {
+                if (c) x[q] = cmul(mod[tid + q * NTB], x[q]);
+                own[q * (NTB + NTB / 16)] = x[q];
+            }
+            __syncthreads();
 #pragma unroll
             for (int q = 0; q < PPT; ++q) {
                 const int i = tid + q * NTB;
-                if (ph == 0) {
-                    const float4 g = Gn[i];
-                    o2[i] = x[q];
-                    x[q] = conjf2(cmul(x[q], make_float2(g.x, g.y)));
-                } else if (ph == 1) {
-                    h[q] = conjf2(x[q]);
-                } else if (ph == 2) {
-                    const float4 g = Gn[i];
-                    o2[n + i] = x[q];
-                    x[q] = conjf2(cmul(x[q], make_float2(g.z, g.w)));
-                } else if (ph == 3) {
-                    // v = conj(x); z = u - conj(m) v = u - conj(m x)
-                    const float2 mx = cmul(mod[i], x[q]);
-                    const float2 z = i < nr ? make_float2(h[q].x - mx.x, h[q].y + mx.y)
-                                            : make_float2(0.f, 0.f);
-                    x[q] = z;
-                    h[q] = cmul(z, mod[i]);
-                } else if (ph == 4) {
-                    o2[i] = cmul(o2[i], x[q]);
-                } else {
-                    o2[n + i] = cmul(o2[n + i], x[q]);
-                }
+                const float2 y = other[q * (NTB + NTB / 16)];
+                const float2 d = make_float2(x[q].x - y.x, x[q].y - y.y);
+                const float2 z = i < nr ? conjf2(d) : make_float2(0.f, 0.f);
+                // group 1 holds m x1 and read x0: its difference is -z's
+                x[q] = c ? cmul(make_float2(-z.x, -z.y), mod[i]) : z;
             }
-        }
-        return;
-    }
-    // Phase: input -> forward transform -> use; an inverse transform is
-    // fft(conj(.)) with the conjugates folded into the neighbouring steps
-    //   0: a          -> E        -> even plane = E (kept there); x = conj(E G_e)
-    //   1: x          -> conj(u)  -> x = m u
-    //   2: x          -> T2       -> h = T2
-    //   3: a m        -> O        -> odd plane = O (T2 - n O G_o); x = conj(O G_o)
-    //   4: x          -> conj(v)  -> x = conj(m) v
-    //   5: x          -> T1       -> h = T1
-    //   6: E read back from the even plane -> even plane = E (n E G_e - T1)
-    // Each thread reads back only the elements it wrote, so phase 6 needs no
-    // barrier and saves the seventh transform.
-#pragma unroll 1
-    for (int ph = 0; ph < 7; ++ph) {
-        if (ph == 0 || ph == 3) load_window<NTB>(x, a, base, win, ph == 3 ? mod : nullptr);
-        if (ph != 6) fft_regs<NTB>(s, x, lad);
-        const int tid = opaque_tid();
+        } else if (CROP) {
 #pragma unroll
-        for (int q = 0; q < PPT; ++q) {
-            const int i = tid + q * NTB;
-            if (ph == 0) {
-                const float4 g = Gn[i];
-                o2[i] = x[q];
-                x[q] = conjf2(cmul(x[q], make_float2(g.x, g.y)));
-            } else if (ph == 1) {
-                x[q] = cmul(conjf2(x[q]), mod[i]);
-            } else if (ph == 2 || ph == 5) {
-                h[q] = x[q];
-            } else if (ph == 3) {
-                const float4 g = Gn[i];
-                const float2 og = cmul(x[q], make_float2(g.z, g.w));
-                o2[n + i] = cmul(x[q], make_float2(h[q].x - fn * og.x, h[q].y - fn * og.y));
-                x[q] = conjf2(og);
-            } else if (ph == 4) {
-                x[q] = conjf2(cmul(x[q], mod[i]));
-            } else {
-                const float4 g = Gn[i];
-                const float2 e = o2[i];
-                const float2 eg = cmul(e, make_float2(g.x, g.y));
-                o2[i] = cmul(e, make_float2(fn * eg.x - h[q].x, fn * eg.y - h[q].y));
+            for (int q = 0; q < PPT; ++q) o2[tid + q * NTB] = cmul(e[q], x[q]);
+        } else if (ph == 1) {
+#pragma unroll
+            for (int q = 0; q < PPT; ++q) {
+                const float2 m = mod[tid + q * NTB];
+                x[q] = c ? conjf2(cmul(x[q], m)) : cmul(conjf2(x[q]), m);
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < PPT; ++q) own[q * (NTB + NTB / 16)] = x[q];
+            __syncthreads();
+#pragma unroll
+            for (int q = 0; q < PPT; ++q) {
+                const int i = tid + q * NTB;
+                const float2 t = other[q * (NTB + NTB / 16)];
+                const float2 eg = cmul(e[q], G[2 * i]);
+                const float2 d = make_float2(fn * eg.x - t.x, fn * eg.y - t.y);
+                o2[i] = cmul(e[q], c ? make_float2(-d.x, -d.y) : d);
             }
         }
     }
@@ -1383,9 +1365,12 @@ __global__ void k_wl_perm_table(float4* __restrict__ Gp, const float4* __restric
     if (p < n) Gp[p] = Gn[wl_perm(p, lw)];
 }
 
-// k_tpair_half with the wave-local transforms (n = 1024 W): the same
-// phases, with F where a transform takes natural input and G where it takes
-// permuted input (plain: F G F F G F; cropped: F G F G F F).  Gn is the
+// The chain with the wave-local transforms (n = 1024 W), one group running
+// both halves: E is parked in the even half of the pair's output row (which
+// only the last step writes) instead of being transformed again, and at most
+// one register array is held across a transform.  F where a transform takes
+// natural input and G where it takes permuted input (plain: F G F F G F;
+// cropped: F G F G F F).  Gn is the
 // permuted spectrum (k_wl_perm_table), the output planes are written in the
 // permuted layout, and the inputs, m(j) and the cropped z stay natural.
 template <int W, bool MT = false, bool CROP = false>
@@ -1804,8 +1789,10 @@ int target_half_slice() { return SLICE; }
 
 // the wave-local chain from n = 8192 (one or two workgroups per CU, whose
 // barriers idle it); below, several workgroups share a CU and hide the
-// barriers of k_tpair_half, which is then 2-3 % faster (fBm geometry,
-// 50 shots: n = 8192 13.4 against 14.7 ms; 4096 6.58 against 6.39)
+// barriers of k_tpair_half, which is then faster (1 681 targets, 24 shots:
+// n = 8192 9.02 against 9.60 ms with k_tpair_half<512>, whose one workgroup
+// per CU idles at each barrier; n = 4096 6.2 ms with k_tpair_half, whose
+// single-group form was already the faster of the two by 3 %)
 bool target_wl(const FftPlan& p) { return p.N / 2 >= 8192 && p.N / 2 <= 16384; }
 
 void wl_perm_table(const float2* Gnat, float2* Gwl, int P, hipStream_t st) {
@@ -1847,45 +1834,37 @@ void target_pairs_half(erp_ctx* ctx, const FftPlan& p, const float2* A, const in
     float2* o4 = work;
     // n: the pairs, or (multi-track, Gpair set) the bound of a grid whose
     // pairs past *npairs_dev exit at once
-    auto go = [&](auto kern, int nt) {
-        hipLaunchKernelGGL(kern, dim3(n), dim3(nt), 0, st, A, p.N, pbase, pwin, G4, o4, lad,
+    auto go = [&](auto kern, dim3 nt) {
+        hipLaunchKernelGGL(kern, dim3(n), nt, 0, st, A, p.N, pbase, pwin, G4, o4, lad,
                            Gpair, npairs_dev, nr);
     };
     const bool mt = Gpair != nullptr;
     const bool crop = nr < p.N / 2;
     // the 2 x 2 variants (multi-track, cropped) of one transform size
-    auto pick = [&](auto k00, auto k10, auto k01, auto k11, int nt) {
+    auto pick = [&](auto k00, auto k10, auto k01, auto k11, dim3 nt) {
         if (crop) mt ? go(k11, nt) : go(k01, nt);
         else mt ? go(k10, nt) : go(k00, nt);
     };
 #define ERP_TPAIR_VARIANTS(NTB)                                                       \
     pick(k_tpair_half<NTB, false, false>, k_tpair_half<NTB, true, false>,            \
          k_tpair_half<NTB, false, true>, k_tpair_half<NTB, true, true>, NTB)
-    if (target_wl(p)) {
-        // the wave-local transforms (Gnat in their layout)
-#define ERP_TPAIR_WL(W)                                                                \
-    pick(k_tpair_wl<W, false, false>, k_tpair_wl<W, true, false>,                     \
-         k_tpair_wl<W, false, true>, k_tpair_wl<W, true, true>, 64 * W)
-        switch (p.N / 2) {
-            case 1024: ERP_TPAIR_WL(1); break;
-            case 2048: ERP_TPAIR_WL(2); break;
-            case 4096: ERP_TPAIR_WL(4); break;
-            case 8192: ERP_TPAIR_WL(8); break;
-            default: ERP_TPAIR_WL(16); break;
-        }
-#undef ERP_TPAIR_WL
-        ERP_CHECK_LAUNCH("k_tpair_wl");
-        return;
-    }
+    // the wave-local transforms take Gnat in their layout
+#define ERP_TPAIR_HALF(NTB)                                                             \
+    pick(k_tpair_half<NTB, false, false>, k_tpair_half<NTB, true, false>,              \
+         k_tpair_half<NTB, false, true>, k_tpair_half<NTB, true, true>, dim3(NTB, 2))
+#define ERP_TPAIR_WL(W)                                                                 \
+    pick(k_tpair_wl<W, false, false>, k_tpair_wl<W, true, false>,                      \
+         k_tpair_wl<W, false, true>, k_tpair_wl<W, true, true>, dim3(64 * W))
     switch (p.N / 2) {
-        case 1024: ERP_TPAIR_VARIANTS(64); break;
-        case 2048: ERP_TPAIR_VARIANTS(128); break;
-        case 4096: ERP_TPAIR_VARIANTS(256); break;
-        case 8192: ERP_TPAIR_VARIANTS(512); break;
-        default: ERP_TPAIR_VARIANTS(1024); break;
+        case 1024: ERP_TPAIR_HALF(64); break;
+        case 2048: ERP_TPAIR_HALF(128); break;
+        case 4096: ERP_TPAIR_HALF(256); break;
+        case 8192: ERP_TPAIR_WL(8); break;
+        default: ERP_TPAIR_WL(16); break;
     }
-#undef ERP_TPAIR_VARIANTS
-    ERP_CHECK_LAUNCH("k_tpair_half");
+#undef ERP_TPAIR_HALF
+#undef ERP_TPAIR_WL
+    ERP_CHECK_LAUNCH("target_pairs_half");
 }
 
 // Per-shot sums of the per-pair rows of work: slice sums into partial
