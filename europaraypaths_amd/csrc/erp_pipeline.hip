@@ -658,6 +658,17 @@ struct Rec {
     int64_t cap;
 };
 
+// Threads per workgroup of k_surface for a grid of the given blocks.  A
+// thread takes its facets one after the other, some 4 us of FP64 latency
+// each, and up to two workgroups per CU (512) leave the SIMDs idle between
+// them: then 1024 threads with two facets each instead of 256 with eight.
+// k_surface, us: 2 blocks 32.3 to 22.3 (512 threads: 24.0), 448 blocks 42.5
+// to 33.8 (34.0), specular 240 blocks 46.1 to 44.3.  Above, the small
+// workgroups fill the CUs as well (16 waves either way, 117 registers) and
+// end in a finer last wave.
+constexpr int SURF_NT = 1024;
+int surface_threads(int64_t blocks) { return blocks <= 512 ? SURF_NT : NT; }
+
 // Facet records of a block of two consecutive shots for the shot-pair target
 // kernel: the facets that either shot illuminates (the union of the two
 // masks), laid out per block as rec_slot lays out one shot's, with the
@@ -812,7 +823,10 @@ __device__ __forceinline__ int rec_slot(int i, int V) {
     return (a < rem ? a * (q + 1) : rem * (q + 1) + (a - rem) * q) + c;
 }
 
-__global__ void __launch_bounds__(NT) k_surface(
+// One workgroup of NTS threads per block of FB facets and shot, FB / NTS
+// facets per thread one after the other.
+template <int NTS>
+__global__ void __launch_bounds__(NTS) k_surface(
     const float* __restrict__ mesh, int64_t Fpad, int64_t F, const erp_shot* __restrict__ shots,
     const unsigned long long* __restrict__ mask, const int* __restrict__ off,
     const int* __restrict__ Vs, const int64_t* __restrict__ rec_base, int nblk, KPar kp,
@@ -828,6 +842,7 @@ __global__ void __launch_bounds__(NT) k_surface(
     // double-float, and its LDS window sums in FP64 / FP32 / compensated
     // FP32 (the window partial sums enter the FP64 row as they are); the
     // facet records for the target kernels always keep the FP64 range
+    constexpr int FPT = FB / NTS, WPB = NTS / 64;
     const int blk = blockIdx.x, s = blockIdx.y;
     // the shot's index within its track (the incoherent phase hash)
     int64_t shot_id = shot0 + s;
@@ -857,27 +872,31 @@ __global__ void __launch_bounds__(NT) k_surface(
     __shared__ unsigned long long um_s[MASKW];
     __shared__ int upre_s[MASKW];
     const bool blk_rec = write_rec && brk.rec.qa;
-    if (threadIdx.x < MASKW) {
-        m_s[threadIdx.x] = mw[threadIdx.x];
-        if (blk_rec)
-            um_s[threadIdx.x] = brk.umask[((size_t)(s >> 1) * nblk + blk) * MASKW + threadIdx.x];
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int t = 0;
-        for (int w = 0; w < MASKW; ++w) {
-            pre_s[w] = t;
-            t += __popcll(m_s[w]);
+    if (threadIdx.x < 64) {
+        // the words' lit counts, prefixed over the first MASKW lanes
+        const int l = threadIdx.x;
+        unsigned long long m = 0, um = 0;
+        if (l < MASKW) {
+            m = mw[l];
+            if (blk_rec) um = brk.umask[((size_t)(s >> 1) * nblk + blk) * MASKW + l];
         }
-        pre_s[MASKW] = t;
-        wmin_s = 0x7FFFFFFF;
-        if (blk_rec) {
-            int u = 0;
-            for (int w = 0; w < MASKW; ++w) {
-                upre_s[w] = u;
-                u += __popcll(um_s[w]);
+        const int c = __popcll(m), uc = __popcll(um);
+        int t = c, u = uc;
+        for (int o = 1; o < MASKW; o <<= 1) {
+            const int pt = __shfl_up(t, o), pu = __shfl_up(u, o);
+            if (l >= o) {
+                t += pt;
+                u += pu;
             }
         }
+        if (l < MASKW) {
+            m_s[l] = m;
+            um_s[l] = um;
+            pre_s[l] = t - c;
+            upre_s[l] = u - uc;
+        }
+        if (l == MASKW - 1) pre_s[MASKW] = t;
+        if (l == 0) wmin_s = 0x7FFFFFFF;
     }
     __syncthreads();
     if (pre_s[MASKW] == 0) return;  // dark block (uniform exit)
@@ -908,7 +927,7 @@ __global__ void __launch_bounds__(NT) k_surface(
         const int w = q * WPB + wv;
         const unsigned long long m = m_s[w];
         if (!((m >> lane) & 1ull)) continue;
-        const int64_t i = facet_of(blk, q * NT + threadIdx.x, tile_nx);
+        const int64_t i = facet_of(blk, q * NTS + threadIdx.x, tile_nx);
         const int rank = pre_s[w] + __popcll(m & ((1ull << lane) - 1ull));
         float g[12];
 #pragma unroll
@@ -1101,7 +1120,7 @@ __global__ void __launch_bounds__(NT) k_surface(
         red_d[0][wv] = litmin; red_d[1][wv] = litmax;
     }
     // (FP64 window, or the FP32 layout of the study's sums in the same LDS)
-    for (int k = threadIdx.x; k < 2 * SWIN; k += NT) swin[k] = 0.0;
+    for (int k = threadIdx.x; k < 2 * SWIN; k += NTS) swin[k] = 0.0;
     __syncthreads();
     if (threadIdx.x == 0 && bounds) {
         float a[6];
@@ -1154,7 +1173,7 @@ __global__ void __launch_bounds__(NT) k_surface(
             }
         }
         __syncthreads();
-        for (int k = threadIdx.x; k < SWIN; k += NT) {
+        for (int k = threadIdx.x; k < SWIN; k += NTS) {
             const int b = base + k;
             const unsigned long long x = wux[k], y = wuy[k];
             if (b < nr && (x | y)) {
@@ -1186,7 +1205,7 @@ __global__ void __launch_bounds__(NT) k_surface(
         }
     }
     __syncthreads();
-    for (int k = threadIdx.x; k < SWIN; k += NT) {
+    for (int k = threadIdx.x; k < SWIN; k += NTS) {
         double vx, vy;
         if (prec_acc == ACC_F64) {
             vx = swin[k];
@@ -4551,6 +4570,8 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
         for (int s = 0; s < S; ++s) Vsum += hV[s];
         PT_.begin(ERP_STAGE_SURFACE, st, Vsum);
         const int write = (need_rec && Vtot > 0) ? 1 : 0;
+        const int nts = surface_threads((int64_t)nblk * S);
+        const auto ksurf = nts == NT ? k_surface<NT> : k_surface<SURF_NT>;
         if (T == 0 && !spec && !det && ph == PH_F64 && acc == ACC_F64) {
             // no targets: nothing reads records or bounds (shots are the fast
             // dimension where the blocks fit the other one)
@@ -4561,7 +4582,7 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
                                nblk, kp, srow, s0, tile_nx, shot_fast);
             ERP_CHECK_LAUNCH("k_surface_lean");
         } else {
-            hipLaunchKernelGGL(k_surface, dim3(nblk, S), dim3(NT), 0, st, mesh->soa.as<float>(),
+            hipLaunchKernelGGL(ksurf, dim3(nblk, S), dim3(nts), 0, st, mesh->soa.as<float>(),
                                mesh->Fpad, F, dshots, dmask, W.off.as<int>(), dV, dbase, nblk, kp, rec,
                                write, do_trace ? 1 : 0, srow, s0, dbounds, det ? 1 : 0, smax,
                                tile_nx, ph, acc, (const TrackK*)nullptr, (const RowK*)nullptr, brk,
@@ -4577,7 +4598,7 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
         if (det && do_trace) {
             // second pass: the same terms as fixed-point values scaled by the
             // per-shot maxima of the first
-            hipLaunchKernelGGL(k_surface, dim3(nblk, S), dim3(NT), 0, st, mesh->soa.as<float>(),
+            hipLaunchKernelGGL(ksurf, dim3(nblk, S), dim3(nts), 0, st, mesh->soa.as<float>(),
                                mesh->Fpad, F, dshots, dmask, W.off.as<int>(), dV, dbase, nblk, kp,
                                rec, 0, 1, srow, s0, (Bounds*)nullptr, 2, smax, tile_nx, 0,
                                0, (const TrackK*)nullptr, (const RowK*)nullptr, BlkRec{},
@@ -5430,6 +5451,8 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
         double Vsum = 0;
         for (size_t i = 0; i < r; ++i) Vsum += hV[i];
         PT_.begin(ERP_STAGE_SURFACE, st, Vsum);
+        const int nts = surface_threads((int64_t)nblk_max * R);
+        const auto ksurf = nts == NT ? k_surface<NT> : k_surface<SURF_NT>;
         mt_launch(m.gA2, direct, st, [&] {
             const size_t n1 = targ ? r * sumP : 0, ni = pairk ? 2 * m.key.reccap : 0;
             hipLaunchKernelGGL(k_batch_prep, dim3(grid_for(srow_f2 + n1 + ni, 256, 4096)),
@@ -5438,7 +5461,7 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
                                m.srow.as<double>(), srow_f2, m.Sacc.as<double>(), n1,
                                reinterpret_cast<double*>(brk.rec.itd), ni, dtrk, drows);
             ERP_CHECK_LAUNCH("k_batch_prep");
-            hipLaunchKernelGGL(k_surface, dim3(nblk_max, R), dim3(NT), 0, st,
+            hipLaunchKernelGGL(ksurf, dim3(nblk_max, R), dim3(nts), 0, st,
                                (const float*)nullptr, (int64_t)0, (int64_t)0, dshots,
                                m.mask.as<unsigned long long>(), m.off.as<int>(), dV, dbase,
                                nblk_max, kp0, rec, targ ? 1 : 0, 1, srow, (int64_t)0, dbounds,
@@ -5452,7 +5475,7 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
                 ERP_CHECK_LAUNCH("k_shot_sphere");
             }
             if (det) {
-                hipLaunchKernelGGL(k_surface, dim3(nblk_max, R), dim3(NT), 0, st,
+                hipLaunchKernelGGL(ksurf, dim3(nblk_max, R), dim3(nts), 0, st,
                                    (const float*)nullptr, (int64_t)0, (int64_t)0, dshots,
                                    m.mask.as<unsigned long long>(), m.off.as<int>(), dV, dbase,
                                    nblk_max, kp0, rec, 0, 1, srow, (int64_t)0, (Bounds*)nullptr,
