@@ -1083,6 +1083,8 @@ __device__ __forceinline__ void load_window(float2 (&x)[PPT], const float2* __re
 // runs of vhf chirps (us): 9 pairs per shot, 100 shots, n = 1024 624 to 570
 // (nr = n 736 to 684); 1 681 targets, 24 shots, n = 1024 4 041 to 3 932,
 // 2048 5 227 to 4 996, 4096 6 559 to 6 231, cropped 4096 6 827 to 6 392.
+// The kernel itself, us: n = 1024 a single pair 33 to 14, 64 shots of 9
+// pairs 50 to 20; n = 2048, many pairs 976 to 727 per launch.
 template <int NTB, bool MT = false, bool CROP = false>
 __global__ void __launch_bounds__(2 * NTB) k_tpair_half(const float2* __restrict__ A, int P,
                                                         const int* __restrict__ pbase,
