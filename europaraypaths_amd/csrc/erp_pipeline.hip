@@ -1344,8 +1344,12 @@ __global__ void __launch_bounds__(NT) k_surface_lean(
             Iv = e.y;
         }
         // sin(Ith) (cos Iph, sin Iph); (sI, 0) where both projections vanish
+        // or are too small for the hardware root, which takes no denormals:
+        // there the facet looks straight at the shot and the azimuth is
+        // immaterial (rounding leaves sI up to some 1e-4, where the two
+        // sincs' product turns by less than 1e-9)
         const float r2 = Iu * Iu + Iv * Iv;
-        const bool az = r2 > 0.f;
+        const bool az = r2 > 1e-30f;
         const float ri = sI * __builtin_amdgcn_rsqf(az ? r2 : 1.f);
         float n1, d1, n2, d2;
         pisinc(hL * (az ? Iv * ri : sI), &n1, &d1);
