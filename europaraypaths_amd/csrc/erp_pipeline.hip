@@ -269,6 +269,16 @@ __device__ __forceinline__ void pisinc_nd_hw(float x, float* num, float* den) {
     *den = xa;
 }
 
+// exp(x) from the hardware's exp2 (1 ulp): what rounding takes from x log2(e)
+// is put back to first order, so that the error does not grow with |x|
+__device__ __forceinline__ float exp_hw(float x) {
+    x = x < -200.f ? -200.f : x;  // zero anyway (and keeps an infinite x out of the difference)
+    const float t = x * 1.44269504f;
+    const float lo = fmaf(x, 1.92596303e-8f, fmaf(x, 1.44269504f, -t));
+    const float r = __builtin_amdgcn_exp2f(t);
+    return fmaf(r, 0.693147181f * lo, r);
+}
+
 // exp(-i pi t) for t = 2 r c given r and c (FP64): the half-cycle count
 // h = t / 2 = r c is formed directly, which is the same double as 0.5 (r 2c)
 __device__ __forceinline__ float2 phasor_rc_hw(double r, double c) {
@@ -1230,18 +1240,22 @@ __global__ void __launch_bounds__(NTS) k_surface(
 // needs about 100 instructions and reads 48 bytes.  So, as in the target
 // kernels: range and 1 / range by one FP64 Newton step from the hardware
 // reciprocal root, the oracle's exact root and division only within 1e-7 bin
-// of a bin edge (bin indices stay identical), hardware sine, exponential
-// and reciprocal on reduced arguments, sqrt(fRe) formed directly, the
-// azimuth from unnormalised projections (only their ratio enters).  No
+// of a bin edge (bin indices stay identical), hardware roots and
+// reciprocals (1 ulp), the phasor by the hardware sine on the exactly reduced
+// argument (1.2e-7 of its modulus), sqrt(fRe) formed directly, the
+// azimuth from unnormalised projections (only their ratio enters).  The
+// sincs' sines stay polynomials: the hardware sine is as good only relative
+// to 1, and facets small against the wavelength, whose terms add up
+// coherently, showed it (error of 2 to 8 m facets against 64 bits 7.4e-7 rms
+// instead of 2.3e-7 with k_surface and 1.6e-7 here).  No
 // bounds, no ranks; only the bins a block's terms reach are cleared and
 // flushed.  Shots are the fast grid dimension: the workgroups that read one
 // facet block run together and find it in their L2.
-// Measured on the 2048 x 2048 mesh at 60 degrees, 50 shots (1.9e8 terms):
-// k_surface took 4.2 ms per launch, this kernel 1.15 ms; VALU 82 % busy with
-// 142 instructions per facet (176 with vector addresses for the loads, 1.28
-// ms).  Windows of 1024 bins instead of 2048 and the next facet's loads
-// ahead of the arithmetic gave 1.38 to 1.28 ms.
-template <bool REDUCE>
+// Measured on the 2048 x 2048 mesh at 60 degrees, 50 shots (1.9e8 terms), a
+// whole run: 4.33 ms with k_surface, 1.45 with this kernel, 1.39 with
+// hardware sines and exponential.  Scalar bases for the loads, windows of
+// 1024 bins instead of 2048 and the next facet's loads ahead of the arithmetic
+// gave 0.2 ms of it.
 __global__ void __launch_bounds__(NT) k_surface_lean(
     const float* __restrict__ mesh, int64_t Fpad, const erp_shot* __restrict__ shots,
     const unsigned long long* __restrict__ mask, const int* __restrict__ cnt, int nblk, KPar kp,
@@ -1259,20 +1273,13 @@ __global__ void __launch_bounds__(NT) k_surface_lean(
     const double rst = (double)sh.rst, x0 = -rst * kp.inv_dr, two_cyc = 2.0 * kp.inv_cyc;
     // amplitude without G1 / Dmax / Itd^2 and the loss; the four factors pi
     // of the two pi-sincs squared
-    const float amp0 = kp.sqrtP * kp.lam * kp.lam * sh.grefr * kp.invK * kp.Dmax *
-                       (0.0102659823f * 0.0625f);
-    // exp(-2 (alpha1 Itd + (ks cI)^2)) as exp2
-    constexpr float m2l2e = -2.f * 1.44269504088896341f;
-    // pi-sincs from half their arguments h in revolutions, sin(2 pi |h|) / |h|
-    // (the four factors 2 in amp0); REDUCE: |h| may pass 256, up to which the
-    // hardware sine's own reduction is exact enough
-    const float hL = 0.5f * kp.piLlam;
-    auto pisinc = [](float h, float* num, float* den) {
-        const float ha = fmaxf(fabsf(h), 5e-7f);
-        *num = __builtin_amdgcn_sinf(REDUCE ? ha - rintf(ha) : ha);
-        *den = ha;
+    const float amp0 = kp.sqrtP * kp.lam * kp.lam * sh.grefr * kp.invK * kp.Dmax * 0.0102659823f;
+    // pi-sinc but for its sign (both are squared): sin(pi r) / |x|, r = x - rint(x)
+    auto pisinc_abs = [](float x, float* num, float* den) {
+        const float xa = fmaxf(fabsf(x), 1e-6f);
+        *num = sinpi_red(xa - rintf(xa));
+        *den = xa;
     };
-    const float la = m2l2e * kp.alpha1, lk = m2l2e * kp.ks * kp.ks;
 
     int bq[FPT];
     float wq[FPT];
@@ -1352,8 +1359,8 @@ __global__ void __launch_bounds__(NT) k_surface_lean(
         const bool az = r2 > 1e-30f;
         const float ri = sI * __builtin_amdgcn_rsqf(az ? r2 : 1.f);
         float n1, d1, n2, d2;
-        pisinc(hL * (az ? Iv * ri : sI), &n1, &d1);
-        pisinc(hL * (Iu * ri), &n2, &d2);
+        pisinc_abs(kp.piLlam * (az ? Iv * ri : sI), &n1, &d1);
+        pisinc_abs(kp.piLlam * (Iu * ri), &n2, &d2);
         const float sc = n1 * n2 * __builtin_amdgcn_rcpf(d1 * d2);
         float amp = amp0 * (sc * sc) * (rs * rs);
         if (!lossless) {
@@ -1363,7 +1370,8 @@ __global__ void __launch_bounds__(NT) k_surface_lean(
                                        : __builtin_amdgcn_sqrtf(fmaxf(0.f, 1.f - sR * sR));
             const float rho = (kp.nu2 * cI - kp.nu1 * cR) *
                               __builtin_amdgcn_rcpf(kp.nu2 * cI + kp.nu1 * cR);
-            amp *= fabsf(rho) * __builtin_amdgcn_exp2f(fmaf(lk * cI, cI, la * (float)Itd));
+            const float kc = kp.ks * cI;
+            amp *= fabsf(rho) * exp_hw(-2.f * fmaf(kp.alpha1, (float)Itd, kc * kc));
         }
         float2 ph;
         if (incoh) {
@@ -4580,7 +4588,7 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
             // no targets: nothing reads records or bounds (shots are the fast
             // dimension where the blocks fit the other one)
             const int shot_fast = nblk <= 65535 ? 1 : 0;
-            hipLaunchKernelGGL(kp.piLlam <= 512.f ? k_surface_lean<false> : k_surface_lean<true>,
+            hipLaunchKernelGGL(k_surface_lean,
                                shot_fast ? dim3(S, nblk) : dim3(nblk, S), dim3(NT), 0, st,
                                mesh->soa.as<float>(), mesh->Fpad, dshots, dmask, W.cnt.as<int>(),
                                nblk, kp, srow, s0, tile_nx, shot_fast);
