@@ -188,15 +188,6 @@ __device__ __forceinline__ float sinc_f(float x) {
     return sinpif(x) / (3.14159265358979f * x);
 }
 
-// sin(pi |x|) and |x| / 2, at least 5e-7 (where the sinc is 1 to 1e-12): the
-// sinc sin(pi x) / (pi x) is num / (2 pi den).  Hardware sine on the exactly
-// reduced argument in revolutions, 1.2e-7 absolute.
-__device__ __forceinline__ void pisinc(float x, float* num, float* den) {
-    const float h = fmaxf(fabsf(0.5f * x), 5e-7f);
-    *num = __builtin_amdgcn_sinf(__builtin_amdgcn_fractf(h));
-    *den = h;
-}
-
 // sin(pi r) and cos(pi r) for |r| <= 0.5 from their Taylor series (degree 13
 // and 14); truncation error < 7e-10, FP32 evaluation error < 2e-7.
 __device__ __forceinline__ void sincospi_red(float r, float* s, float* c) {
@@ -230,6 +221,16 @@ __device__ __forceinline__ float sinpi_red(float r) {
     ps = fmaf(ps, r2, -5.1677127800499694f);
     ps = fmaf(ps, r2, 3.1415926535897931f);
     return r * ps;
+}
+
+// sinc(x) but for its sign, num / (pi den): sin(pi r) with r = x - rint(x) and
+// |x|, at least 1e-6 (where the sinc is 1 to 2e-12).  The sine is good
+// relative to itself, for the smallest arguments too; the hardware's is 1.2e-7
+// absolute.
+__device__ __forceinline__ void pisinc_abs(float x, float* num, float* den) {
+    const float xa = fmaxf(fabsf(x), 1e-6f);
+    *num = sinpi_red(xa - rintf(xa));
+    *den = xa;
 }
 
 // sinc(x) of elementary_kernels.cu:50-53 as numerator / denominator so that a
@@ -1274,12 +1275,6 @@ __global__ void __launch_bounds__(NT) k_surface_lean(
     // amplitude without G1 / Dmax / Itd^2 and the loss; the four factors pi
     // of the two pi-sincs squared
     const float amp0 = kp.sqrtP * kp.lam * kp.lam * sh.grefr * kp.invK * kp.Dmax * 0.0102659823f;
-    // pi-sinc but for its sign (both are squared): sin(pi r) / |x|, r = x - rint(x)
-    auto pisinc_abs = [](float x, float* num, float* den) {
-        const float xa = fmaxf(fabsf(x), 1e-6f);
-        *num = sinpi_red(xa - rintf(xa));
-        *den = xa;
-    };
 
     int bq[FPT];
     float wq[FPT];
@@ -1696,7 +1691,7 @@ __device__ __forceinline__ float rerad_f(int fn, float th) {
 // (geometry_kernels.cu:530-539, 565-572): fs^2 / lam times
 //     sinc(fs / lam sin(Rth - Tth) cos dph) sinc(... sin dph),  dph = Iph - Tph,
 // and the same with sin(RrTh) for the way back (sinc is even, so its dph may
-// take either sign).  The angles enter through sines and cosines only: those
+// take either sign), without their signs.  The angles enter through sines and cosines only: those
 // of Iph and Rth are the facet record's, (sT, cT) and (Iu, Iv) the target
 // leg's, so no angle is formed; past a critical angle the reference takes
 // 1e4 for the angle.
@@ -1712,12 +1707,12 @@ __device__ __forceinline__ void spec_factors(float sT, float cT, float cph, floa
     const float so = back > 1.f ? s1e4 : back;
     const float cd = cI * cph + sI * sph, sd = sI * cph - cI * sph;
     float n1, d1, n2, d2;
-    pisinc(kp.fs_lam * si * cd, &n1, &d1);
-    pisinc(kp.fs_lam * si * sd, &n2, &d2);
-    *vi = kp.fs2_lam * 0.25f * (n1 * n2) * __builtin_amdgcn_rcpf(d1 * d2) * 0.101321184f;
-    pisinc(kp.fs_lam * so * cd, &n1, &d1);
-    pisinc(kp.fs_lam * so * sd, &n2, &d2);
-    *vo = kp.fs2_lam * 0.25f * (n1 * n2) * __builtin_amdgcn_rcpf(d1 * d2) * 0.101321184f;
+    pisinc_abs(kp.fs_lam * si * cd, &n1, &d1);
+    pisinc_abs(kp.fs_lam * si * sd, &n2, &d2);
+    *vi = kp.fs2_lam * fabsf(n1 * n2) * __builtin_amdgcn_rcpf(d1 * d2) * 0.101321184f;
+    pisinc_abs(kp.fs_lam * so * cd, &n1, &d1);
+    pisinc_abs(kp.fs_lam * so * sd, &n2, &d2);
+    *vo = kp.fs2_lam * fabsf(n1 * n2) * __builtin_amdgcn_rcpf(d1 * d2) * 0.101321184f;
 }
 
 // The same in the reference's steps, for the type-0 targets: their terms take
@@ -1758,9 +1753,12 @@ inline size_t accum_lds(int mode, int nr) {
 // targets of a shot add to the shot's row): pass 1 only takes the largest
 // component of each pair into tmax[shot]; pass 2 adds the terms, scaled by
 // the shot's bound, into the shot's row as fixed-point (int64) pairs.
-// MODE 1 is bound by its instructions (80 % busy): hardware sines, roots and
+// MODE 1 is bound by its instructions (80 % busy): hardware roots and
 // reciprocals and no angles, 359 to 219 us per 600 pairs, and no fence where the
-// window holds the pair, to 97.
+// window holds the pair, to 97.  Hardware sines and exponential instead of the
+// polynomials on reduced arguments save 2 of 340 us per run, but an echo from
+// facets of 2 m at 33 m wavelength was then 3e-6 of its peak off, against 6e-7
+// with the reference's steps and 2.5e-7 so.
 template <int MODE, bool DET = false>
 __global__ void __launch_bounds__(NTT) k_target_accum(
     const float* __restrict__ tg, int64_t Tpad, const int* __restrict__ pshot,
@@ -1864,12 +1862,12 @@ __global__ void __launch_bounds__(NTT) k_target_accum(
             const float ri = az ? __builtin_amdgcn_rsqf(q2) : 0.f;
             const float cph = az ? Iv * ri : 1.f, sph = Iu * ri;
             float n1, d1, n2, d2, n3, d3, n4, d4;
-            pisinc(kp.piLlam * (sT * cph), &n1, &d1);
-            pisinc(kp.piLlam * (sT * sph), &n2, &d2);
-            pisinc(kp.piLlam * (sTT * cph), &n3, &d3);
-            pisinc(kp.piLlam * (sTT * sph), &n4, &d4);
-            // 1 / (2 pi)^4
-            float amp = rec.F[r] * (kp.Dmax * 6.41623909e-4f) *
+            pisinc_abs(kp.piLlam * (sT * cph), &n1, &d1);
+            pisinc_abs(kp.piLlam * (sT * sph), &n2, &d2);
+            pisinc_abs(kp.piLlam * (sTT * cph), &n3, &d3);
+            pisinc_abs(kp.piLlam * (sTT * sph), &n4, &d4);
+            // 1 / pi^4
+            float amp = rec.F[r] * (kp.Dmax * 0.0102659823f) *
                         (fabsf((n1 * n2) * (n3 * n4)) *
                          __builtin_amdgcn_rcpf((d1 * d2) * (d3 * d4))) * rs;
             float ampB = amp / kp.sqrtP;
@@ -1883,13 +1881,13 @@ __global__ void __launch_bounds__(NTT) k_target_accum(
                 }
                 expo += kp.alpha2 * (Ttdf - tot);
                 const float kc = kp.ks * cT;
-                const float e = __builtin_amdgcn_exp2f(-2.885390082f * fmaf(kc, kc, expo));
+                const float e = exp_hw(-2.f * fmaf(kc, kc, expo));
                 // specular EI / EO facet reradiation factors
                 float vi, vo;
                 spec_factors(sT, cT, cph, sph, rec.ang[r], rec.ang[rec.cap + r],
                              rec.ang[2 * rec.cap + r], kp, &vi, &vo);
-                ampB *= e * fabsf(vo);
-                amp *= e * fabsf(vi);
+                ampB *= e * vo;
+                amp *= e * vi;
             }
             const float2 ph = phasor_rc_hw(rngt, kp.inv_cyc);
             // radiateTarget: phasor(rngt - lam / 2), P = 1 W
