@@ -182,6 +182,15 @@ __device__ __forceinline__ float2 sc_angles(float Iu, float Iv, float s) {
     return make_float2(s * Iv * ri, s * Iu * ri);
 }
 
+// Projections of which only the direction matters, atan2(u, v): where their
+// squares would be lost or denormal, both times 2^100
+__device__ __forceinline__ void lift_small(float& u, float& v) {
+    if (!(u * u + v * v > 1e-30f)) {
+        u *= 0x1p100f;
+        v *= 0x1p100f;
+    }
+}
+
 // elementary_kernels.cu:50-53
 __device__ __forceinline__ float sinc_f(float x) {
     if (fabsf(x) < 1e-6f) return 1.0f;
@@ -1033,9 +1042,11 @@ __global__ void __launch_bounds__(NTS) k_surface(
                 rec.fRfrC[r] = fRfrC;
                 // cos Iph, sin Iph (Iph = atan2(Iu, Iv): 0 where both vanish)
                 // and sin Rth (2: past the critical angle)
-                const float rI = sqrtf(Iu * Iu + Iv * Iv);
-                rec.ang[r] = rI > 0.f ? Iv / rI : 1.f;
-                rec.ang[rec.cap + r] = rI > 0.f ? Iu / rI : 0.f;
+                float au = Iu, av = Iv;
+                lift_small(au, av);
+                const float rI = sqrtf(au * au + av * av);
+                rec.ang[r] = rI > 0.f ? av / rI : 1.f;
+                rec.ang[rec.cap + r] = rI > 0.f ? au / rI : 0.f;
                 rec.ang[2 * rec.cap + r] = tir ? 2.f : sR;
             }
             if (rec.qa) {
@@ -1857,8 +1868,9 @@ __global__ void __launch_bounds__(NTT) k_target_accum(
                 Iu = e.x;
                 Iv = e.y;
             }
+            lift_small(Iu, Iv);  // the facet's reradiation turns on the azimuth
             const float q2 = Iu * Iu + Iv * Iv;
-            const bool az = q2 > 1e-30f;
+            const bool az = q2 > 0.f;
             const float ri = az ? __builtin_amdgcn_rsqf(q2) : 0.f;
             const float cph = az ? Iv * ri : 1.f, sph = Iu * ri;
             float n1, d1, n2, d2, n3, d3, n4, d4;
