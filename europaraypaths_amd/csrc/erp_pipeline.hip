@@ -2759,7 +2759,7 @@ __device__ __forceinline__ TLeg tri_leg(const BRecV& rv, int frame_ok, double tx
     // (sin from (Iu, Iv) themselves would save its root, but the reference's
     // sine is that of the rounded normal, which near the facet's axis differs
     // by up to 3e-6: 1e-5 of the strongest terms)
-    const float sTT = tn_up ? __builtin_amdgcn_sqrtf(Ix * Ix + Iy * Iy)
+    const float sTT = tn_up ? __builtin_amdgcn_sqrtf(fmaxf(0.f, (float)((1.0 + iz) * (1.0 - iz))))
                             : cos_sin_hw(ix, iy, iz, tnx, tny, tnz).y;
     // azimuth (cos Tph, sin Tph) = (Iv, Iu) / |(Iu, Iv)|, (1, 0) below 1e-30
     // (where every sinc argument is < 1e-6 whatever the azimuth)
