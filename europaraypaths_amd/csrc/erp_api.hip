@@ -173,8 +173,6 @@ void slot_main(erp_ctx* ctx, ErpSlot* s) {
             if (ctx->queue.empty()) return;  // stopping with nothing queued
             j = ctx->queue.front();
             ctx->queue.pop_front();
-            // counted before the job can take pointers into the table caches
-            ctx->active.fetch_add(1);
         }
         int rc = ERP_OK;
         std::string err;
@@ -191,7 +189,6 @@ void slot_main(erp_ctx* ctx, ErpSlot* s) {
             err = e.what();
         }
         if (rc != ERP_OK) hipStreamSynchronize(s->stream);  // drain what was queued
-        ctx->active.fetch_sub(1);
         {
             // notify under the lock: once it is released the caller may
             // free the job (erp_wait / erp_poll)
@@ -325,17 +322,8 @@ void erp_ctx_destroy(erp_ctx* ctx) {
     hipSetDevice(ctx->device);
     stop_slots(ctx);
     if (ctx->stream) hipStreamSynchronize(ctx->stream);
-    for (auto* c : ctx->chirps) delete c;
-    for (auto* b : ctx->bands) {
-        b->tab.release();
-        delete b;
-    }
     ctx->chirps.clear();
     ctx->bands.clear();
-    for (auto* t : ctx->narrows) {
-        t->tab.release();
-        delete t;
-    }
     ctx->narrows.clear();
     release_work(ctx->work);
     mt_state_free(ctx->mt);
@@ -586,13 +574,6 @@ int erp_run_tracks(erp_ctx* ctx, const erp_track* tracks, int64_t ntracks, uint3
                                                   " belong to another context"};
         }
         set_device(ctx);
-        // the cached range kernel spectra and band tables the batches
-        // point to stay in the cache while the run holds them
-        ctx->active.fetch_add(1);
-        struct Hold {
-            erp_ctx* c;
-            ~Hold() { c->active.fetch_sub(1); }
-        } hold{ctx};
         erp_run_tracks_impl(ctx, tracks, ntracks, flags, ctx->stream);
         ERP_HIP_TRY(hipStreamSynchronize(ctx->stream));
         ctx->prof.resolve();

@@ -10,6 +10,7 @@
 #include <atomic>
 #include <condition_variable>
 #include <deque>
+#include <memory>
 #include <mutex>
 #include <thread>
 
@@ -155,6 +156,17 @@ struct FftPlan {
     bool two_pass = false;
 };
 
+// A cached table: entries are shared between the context's cache and the runs
+// that read them (TableHold), so a cache can drop an entry at any time.  Freed
+// with the last reference; hipFree waits for the device, which covers work
+// that a run has queued and not waited for.
+struct Table {
+    Table() = default;
+    Table(const Table&) = delete;
+    Table& operator=(const Table&) = delete;
+};
+using TableHold = std::vector<std::shared_ptr<void>>;
+
 // Per-(nr, dr, res) chirp spectra
 struct ChirpKey {
     int nr;
@@ -166,11 +178,17 @@ struct ChirpKey {
     }
 };
 
-struct ChirpSpec {
+struct ChirpSpec : Table {
     ChirpKey key;
     DevBuf spec;  // P complex64, permuted forward order, scaled by 1/P
     DevBuf nat;   // the same spectrum in natural order (filled on first use)
     DevBuf wl;    // the natural one in the layout of k_tpair_wl (first use)
+    size_t bytes() const { return spec.bytes + nat.bytes + wl.bytes; }
+    ~ChirpSpec() {
+        spec.release();
+        nat.release();
+        wl.release();
+    }
 };
 
 // Band crop and decimation of a shot's summed spectrum (convolveComplex's
@@ -183,10 +201,12 @@ struct ChirpSpec {
 // D[2 d] and D[2 d - 1], which fit the P >= 2 nr - 1 point transforms.
 // tab: the spectra of those two kernels (output i at P / 2 + i), P complex64
 // each in fft_forward's order, scaled by 1 / P^2 (the two inverses).
-struct BandTables {
+struct BandTables : Table {
     int nr = 0, P = 0;
     float smpl = 0, B = 0;
     DevBuf tab;
+    size_t bytes() const { return tab.bytes; }
+    ~BandTables() { tab.release(); }
 };
 
 // Narrow-band chain of typed targets (erp_narrow.hip): band, decimation and
@@ -201,11 +221,13 @@ struct NarrowPlan {
     const float* tab;        // rows of e_k and M_k (k_narrow_table)
     const float* fir;        // filter operand of k_narrow_fir
 };
-struct NarrowTables {
+struct NarrowTables : Table {
     int nr = 0;
     float dr = 0, res = 0, smpl = 0, B = 0;
     NarrowPlan plan{};
     DevBuf tab;
+    size_t bytes() const { return tab.bytes; }
+    ~NarrowTables() { tab.release(); }
 };
 constexpr int kNarrowSlice = 32;  // pairs per slice
 // entries from one pair row to the next: 256 bytes past a power of two, so
@@ -279,9 +301,9 @@ struct erp_ctx {
     std::string last_error;
     DevBuf twiddle;  // ladder table of the LDS FFT stages (65536 complex64)
     std::vector<std::pair<int, DevBuf*>> inter;  // inter-pass twiddles per size
-    std::vector<ChirpSpec*> chirps;
-    std::vector<BandTables*> bands;
-    std::vector<NarrowTables*> narrows;
+    std::vector<std::shared_ptr<ChirpSpec>> chirps;
+    std::vector<std::shared_ptr<BandTables>> bands;
+    std::vector<std::shared_ptr<NarrowTables>> narrows;
     WorkBufs work;
     std::mutex mu;        // serialises the synchronous entry points
     // guards inter / chirps / bands / narrows (shared by all streams); recursive because
@@ -295,7 +317,6 @@ struct erp_ctx {
     std::mutex qmu;
     std::condition_variable qcv;
     bool stopping = false;
-    std::atomic<int> active{0};  // jobs running in slots
     // caps on the batch shapes (erp_set_tuning; 0 = default)
     std::atomic<int64_t> tune_shots{0}, tune_pairs{0};
     // multi-track batches: rows per batch (0 = default), launch directly

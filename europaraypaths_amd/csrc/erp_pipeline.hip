@@ -3562,40 +3562,50 @@ void build_chirp(erp_ctx* ctx, float2* dst, int nr, float dr, float res, int kin
     ERP_CHECK_LAUNCH("k_scale");
 }
 
-// Range-compression kernel spectrum, cached per context.  natural = true
-// returns it in natural frequency order (the per-pair LDS chain), otherwise
-// in the order fft_forward produces.  Only kind-1 entries (one per receive
-// window start) are evicted, so kind-0 pointers held by a run stay valid.
-// layout: 0 the forward FFT's order, 1 natural, 2 natural in the layout of
-// k_tpair_wl (wl_perm_table)
-const float2* get_chirp(erp_ctx* ctx, int nr, float dr, float res, int kind, float rst, int P,
-                        const FftPlan& plan, hipStream_t st, int layout = 0) {
+// What the caches keep, oldest entries dropped first: small tables by their
+// number (0.5 MB a layout of a spectrum at most), the narrow-band ones (up to 64
+// MB) by their bytes too.
+constexpr size_t kKeepChirps = 64;   // of kinds 0 and 2
+constexpr size_t kKeepCirc = 16;     // of kind 1, one per receive window start
+constexpr size_t kKeepBands = 32;
+constexpr size_t kKeepNarrows = 16;
+constexpr size_t kKeepNarrowBytes = (size_t)256 << 20;
+
+// Adds t to a cache and drops the oldest entries of its class past `most`
+// entries or `most_bytes` (never t).  Under cache_mu.
+template <class T, class Class>
+void keep_table(std::vector<std::shared_ptr<T>>& cache, const std::shared_ptr<T>& t, size_t most,
+                size_t most_bytes, Class&& same_class) {
+    size_t n = 1, bytes = t->bytes();
+    for (size_t i = cache.size(); i-- > 0;) {
+        if (!same_class(*cache[i])) continue;
+        bytes += cache[i]->bytes();
+        if (++n > most || bytes > most_bytes) cache.erase(cache.begin() + (long)i);
+    }
+    cache.push_back(t);
+}
+
+// Range-compression kernel spectrum, cached per context and kept alive by
+// hold.  layout: 0 the forward FFT's order, 1 natural (the per-pair LDS chain),
+// 2 natural in the layout of k_tpair_wl (wl_perm_table)
+const float2* get_chirp(erp_ctx* ctx, TableHold& hold, int nr, float dr, float res, int kind,
+                        float rst, int P, const FftPlan& plan, hipStream_t st, int layout = 0) {
     ChirpKey key{nr, dr, res, kind, kind == 1 ? rst : 0.f};
     std::lock_guard<std::recursive_mutex> lk(ctx->cache_mu);
-    ChirpSpec* c = nullptr;
-    for (ChirpSpec* e : ctx->chirps)
+    std::shared_ptr<ChirpSpec> c;
+    for (const auto& e : ctx->chirps)
         if (e->key == key) c = e;
     if (!c) {
-        c = new ChirpSpec();
+        c = std::make_shared<ChirpSpec>();
         c->key = key;
         c->spec.ensure(sizeof(float2) * (size_t)P);
         build_chirp(ctx, c->spec.as<float2>(), nr, dr, res, kind, rst, P, plan, st);
         // other streams may use the new spectrum as soon as the lock is released
         ERP_HIP_TRY(hipStreamSynchronize(st));
-        int n1 = 0;
-        for (ChirpSpec* e : ctx->chirps) n1 += e->key.kind == 1;
-        // evict only while no asynchronous job can hold a pointer into the cache
-        if (n1 > 16 && ctx->active.load() == 0) {
-            for (size_t i = 0; i < ctx->chirps.size(); ++i)
-                if (ctx->chirps[i]->key.kind == 1) {
-                    ERP_HIP_TRY(hipStreamSynchronize(st));
-                    delete ctx->chirps[i];
-                    ctx->chirps.erase(ctx->chirps.begin() + (long)i);
-                    break;
-                }
-        }
-        ctx->chirps.push_back(c);
+        keep_table(ctx->chirps, c, kind == 1 ? kKeepCirc : kKeepChirps, SIZE_MAX,
+                   [&](const ChirpSpec& e) { return (e.key.kind == 1) == (kind == 1); });
     }
+    hold.push_back(c);
     if (layout == 0) return c->spec.as<float2>();
     if (!c->nat.p) {
         c->nat.ensure(sizeof(float2) * (size_t)P);
@@ -3611,64 +3621,51 @@ const float2* get_chirp(erp_ctx* ctx, int nr, float dr, float res, int kind, flo
     return c->wl.as<float2>();
 }
 
-// band tables of (nr, smpl, B), cached per context
-const float2* get_band(erp_ctx* ctx, int nr, float smpl, float B, const FftPlan& plan,
-                       hipStream_t st) {
+// band tables of (nr, smpl, B), cached per context and kept alive by hold
+const float2* get_band(erp_ctx* ctx, TableHold& hold, int nr, float smpl, float B,
+                       const FftPlan& plan, hipStream_t st) {
     std::lock_guard<std::recursive_mutex> lk(ctx->cache_mu);
-    for (BandTables* b : ctx->bands)
-        if (b->nr == nr && b->smpl == smpl && b->B == B) return b->tab.as<float2>();
-    BandTables* b = new BandTables();
+    for (const auto& b : ctx->bands)
+        if (b->nr == nr && b->smpl == smpl && b->B == B) {
+            hold.push_back(b);
+            return b->tab.as<float2>();
+        }
+    auto b = std::make_shared<BandTables>();
     b->nr = nr;
     b->P = plan.N;
     b->smpl = smpl;
     b->B = B;
     b->tab.ensure(sizeof(float2) * 2 * (size_t)plan.N);
     build_band(ctx, plan, b->tab.as<float2>(), nr, smpl, B, st);
-    ctx->bands.push_back(b);
     ERP_HIP_TRY(hipStreamSynchronize(st));
+    keep_table(ctx->bands, b, kKeepBands, SIZE_MAX, [](const BandTables&) { return true; });
+    hold.push_back(b);
     return b->tab.as<float2>();
 }
 
-// plan and tables of the narrow-band chain, cached per context
-NarrowPlan get_narrow(erp_ctx* ctx, const NarrowPlan& plan, float dr, float res, float smpl,
-                      float B, hipStream_t st) {
+// plan and tables of the narrow-band chain, cached per context and kept alive
+// by hold
+NarrowPlan get_narrow(erp_ctx* ctx, TableHold& hold, const NarrowPlan& plan, float dr, float res,
+                      float smpl, float B, hipStream_t st) {
     std::lock_guard<std::recursive_mutex> lk(ctx->cache_mu);
-    for (NarrowTables* t : ctx->narrows)
-        if (t->nr == plan.nr && t->dr == dr && t->res == res && t->smpl == smpl && t->B == B)
+    for (const auto& t : ctx->narrows)
+        if (t->nr == plan.nr && t->dr == dr && t->res == res && t->smpl == smpl && t->B == B) {
+            hold.push_back(t);
             return t->plan;
-    NarrowTables* t = new NarrowTables();
+        }
+    auto t = std::make_shared<NarrowTables>();
     t->nr = plan.nr;
     t->dr = dr;
     t->res = res;
     t->smpl = smpl;
     t->B = B;
     t->plan = plan;
-    try {
-        t->tab.ensure(sizeof(float) * narrow_table_floats(plan));
-        narrow_build(t->plan, t->tab.as<float>(), st);
-    } catch (...) {
-        t->tab.release();
-        delete t;
-        throw;
-    }
-    ctx->narrows.push_back(t);
+    t->tab.ensure(sizeof(float) * narrow_table_floats(plan));
+    narrow_build(t->plan, t->tab.as<float>(), st);
+    keep_table(ctx->narrows, t, kKeepNarrows, kKeepNarrowBytes,
+               [](const NarrowTables&) { return true; });
+    hold.push_back(t);
     return t->plan;
-}
-
-// Drops the oldest tables past 8 of each kind.  Called where a synchronous
-// run begins: it holds no pointer yet, and no asynchronous job is active.
-void trim_tables(erp_ctx* ctx) {
-    std::lock_guard<std::recursive_mutex> lk(ctx->cache_mu);
-    if (ctx->active.load() != 0) return;
-    auto trim = [](auto& v) {
-        while (v.size() > 8) {
-            v.front()->tab.release();  // hipFree waits for the device
-            delete v.front();
-            v.erase(v.begin());
-        }
-    };
-    trim(ctx->bands);
-    trim(ctx->narrows);
 }
 
 void zero(float2* p, size_t n, hipStream_t st) {
@@ -4143,7 +4140,7 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
         throw ErpError{ERP_E_UNSUPPORTED,
                        "non-specular runs need convolution and convolution_linear "
                        "(sim.cu:431-439,778 otherwise write past the chirp buffer)"};
-    if (!arena) trim_tables(ctx);
+    TableHold hold;  // cached tables this run reads
     const int64_t F = mesh->F;
     const int64_t T = targets ? targets->T : 0;
     const bool any_t0 = T > 0 && targets->n0 > 0, any_typed = T > 0 && targets->n0 < T;
@@ -4186,7 +4183,7 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
 
     // chirp spectra: cached per context, or (arena) built into the region
     auto chirp = [&](float res, int layout, int kind = 0) -> const float2* {
-        if (!arena) return get_chirp(ctx, nr, p.dr, res, kind, 0.f, P, planP, st, layout);
+        if (!arena) return get_chirp(ctx, hold, nr, p.dr, res, kind, 0.f, P, planP, st, layout);
         float2* spec_ = arena->take_n<float2>((size_t)P, "chirp spectrum");
         build_chirp(ctx, spec_, nr, p.dr, res, kind, 0.f, P, planP, st);
         if (layout == 0) return spec_;
@@ -4217,7 +4214,7 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
     if (nar.ok && arena)
         narrow_build(nar, arena->take_n<float>(narrow_table_floats(nar), "narrow-band tables"), st);
     else if (nar.ok)
-        nar = get_narrow(ctx, nar, p.dr, res_t, p.smpl, p.B, st);
+        nar = get_narrow(ctx, hold, nar, p.dr, res_t, p.smpl, p.B, st);
     const bool nb = nar.ok;
     if (nb) {
         kp.row_live = nr;
@@ -4241,7 +4238,7 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
             build_band(ctx, planP, tab, nr, p.smpl, p.B, st);
             band = tab;
         } else {
-            band = get_band(ctx, nr, p.smpl, p.B, planP, st);
+            band = get_band(ctx, hold, nr, p.smpl, p.B, planP, st);
         }
     }
 
@@ -4992,12 +4989,13 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
                         std::vector<erp_shot> hs(shots + s0, shots + s0 + S);
                         for (int s = 0; s < S; ++s) {
                             const float2* gc = g_circ;
+                            TableHold one;  // not all of a long track's at once
                             if (g_circ)  // rebuilt in place: stream order keeps the last use
                                 build_chirp(ctx, g_circ, nr, p.dr, p.rng_res, 1, hs[s].rst, P,
                                             planP, st);
                             else
-                                gc = get_chirp(ctx, nr, p.dr, p.rng_res, 1, hs[s].rst, P, planP,
-                                               st);
+                                gc = get_chirp(ctx, one, nr, p.dr, p.rng_res, 1, hs[s].rst, P,
+                                               planP, st);
                             window_conv(ctx, planP, t0 + (size_t)s * P, 1, gc,
                                         refr0 + (size_t)s * nr, nr, st);
                         }
@@ -5173,7 +5171,8 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
     const int tkind = nr < P / 2 ? 2 : 0;  // the cropped pair chain's kernel placement
     const int ntr = (int)trk_idx.size();
 
-    // track descriptors
+    // track descriptors, and the cached tables they point to
+    TableHold hold;
     std::vector<TrackK> tk((size_t)ntr);
     int nblk_max = 1, Tcap = 0;
     bool targ = false;
@@ -5203,14 +5202,14 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
             d.ttype = t.targets->type.as<unsigned char>();
             // sim.cu:853-858: the target range kernel has twice the surface's
             if (!narrow)
-                d.g_targ_nat = get_chirp(ctx, nr, p.dr, 2.f * p.rng_res, tkind, 0.f, P, planP, st,
-                                         target_wl(planP) ? 2 : 1);
+                d.g_targ_nat = get_chirp(ctx, hold, nr, p.dr, 2.f * p.rng_res, tkind, 0.f, P,
+                                         planP, st, target_wl(planP) ? 2 : 1);
             targ = true;
         }
         // a disabled surface echo: no spectrum, so the row's echo is zero
         d.g_surf = (p.mode & ERP_MODE_DISABLE_SURFACE)
                        ? nullptr
-                       : get_chirp(ctx, nr, p.dr, p.rng_res, 0, 0.f, P, planP, st);
+                       : get_chirp(ctx, hold, nr, p.dr, p.rng_res, 0, 0.f, P, planP, st);
         d.out = static_cast<float2*>(t.out_dev);
         d.nvalid = static_cast<int32_t*>(t.nvalid_dev);
         d.tscale = -1.0f / d.kp.sqrtP;  // outward trace = -A / sqrt(P)
@@ -5228,11 +5227,11 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
             const erp_track& t = tracks[trk_idx[k]];
             const erp_params& p = *t.par;
             if (!narrow) {
-                tk[k].band = get_band(ctx, nr, p.smpl, p.B, planP, st);
+                tk[k].band = get_band(ctx, hold, nr, p.smpl, p.B, planP, st);
                 continue;
             }
-            tk[k].narrow = get_narrow(ctx, mt_narrow(t, det), p.dr, 2.f * p.rng_res, p.smpl, p.B,
-                                      st);
+            tk[k].narrow = get_narrow(ctx, hold, mt_narrow(t, det), p.dr, 2.f * p.rng_res, p.smpl,
+                                      p.B, st);
             nar.nr = nr;
             nar.Nu = std::max(nar.Nu, tk[k].narrow.Nu);
             nar.K = std::max(nar.K, tk[k].narrow.K);
@@ -5686,7 +5685,6 @@ void erp_run_tracks_impl(erp_ctx* ctx, const erp_track* tracks, int64_t ntracks,
                            ERP_RUN_PHASE_DF | ERP_RUN_ACC_F32 | ERP_RUN_ACC_COMP;
     if (flags & ~known) throw ErpError{ERP_E_INVALID, "unknown run flags"};
     const bool det = flags & ERP_RUN_DETERMINISTIC;
-    trim_tables(ctx);
     // groups of one range length, second-medium setting and spectral chain,
     // in track order
     std::vector<std::pair<std::tuple<int, bool, bool>, std::vector<int64_t>>> groups;
