@@ -5218,24 +5218,28 @@ void mt_run_group(erp_ctx* ctx, const erp_track* tracks, const std::vector<int64
         nrows += t.ns;
     }
 
-    // band tables (or the narrow-band chain's) of every track once any has
-    // targets: the tail runs over all rows of a batch (a row without targets
-    // crops a zero sum).  nar: the launches' bounds; rows read their own plan.
+    // band tables (or the narrow-band chain's) of the tracks with targets.  The
+    // tail runs over all rows of a batch; a row without targets crops a zero
+    // sum, for which any band of the group does (or the plan's zeros: k = 0
+    // alone).  nar: the launches' bounds; rows read their own plan.
     NarrowPlan nar{};
-    if (targ)
-        for (int k = 0; k < ntr; ++k) {
-            const erp_track& t = tracks[trk_idx[k]];
-            const erp_params& p = *t.par;
-            if (!narrow) {
-                tk[k].band = get_band(ctx, hold, nr, p.smpl, p.B, planP, st);
-                continue;
-            }
-            tk[k].narrow = get_narrow(ctx, hold, mt_narrow(t, det), p.dr, 2.f * p.rng_res, p.smpl,
-                                      p.B, st);
-            nar.nr = nr;
-            nar.Nu = std::max(nar.Nu, tk[k].narrow.Nu);
-            nar.K = std::max(nar.K, tk[k].narrow.K);
+    const float2* band = nullptr;
+    for (int k = 0; k < ntr; ++k) {
+        if (tk[k].T == 0) continue;
+        const erp_track& t = tracks[trk_idx[k]];
+        const erp_params& p = *t.par;
+        if (!narrow) {
+            tk[k].band = band = get_band(ctx, hold, nr, p.smpl, p.B, planP, st);
+            continue;
         }
+        tk[k].narrow = get_narrow(ctx, hold, mt_narrow(t, det), p.dr, 2.f * p.rng_res, p.smpl,
+                                  p.B, st);
+        nar.nr = nr;
+        nar.Nu = std::max(nar.Nu, tk[k].narrow.Nu);
+        nar.K = std::max(nar.K, tk[k].narrow.K);
+    }
+    for (int k = 0; k < ntr; ++k)
+        if (tk[k].T == 0) tk[k].band = band;
     const size_t sumP = narrow ? 2 * ((size_t)nar.K + 1) : (size_t)P;
     const int rowP = narrow ? narrow_stride(P) : P;
 
@@ -5685,14 +5689,19 @@ void erp_run_tracks_impl(erp_ctx* ctx, const erp_track* tracks, int64_t ntracks,
                            ERP_RUN_PHASE_DF | ERP_RUN_ACC_F32 | ERP_RUN_ACC_COMP;
     if (flags & ~known) throw ErpError{ERP_E_INVALID, "unknown run flags"};
     const bool det = flags & ERP_RUN_DETERMINISTIC;
-    // groups of one range length, second-medium setting and spectral chain,
-    // in track order
+    // groups of one range length, second-medium setting and spectral chain, in
+    // track order.  A track without targets runs no chain: it joins the first
+    // group of its range length and medium.
     std::vector<std::pair<std::tuple<int, bool, bool>, std::vector<int64_t>>> groups;
-    std::vector<int64_t> solo;
+    std::vector<int64_t> solo, plain;
     for (int64_t i = 0; i < ntracks; ++i) {
         const erp_track& t = tracks[i];
         if (!mt_eligible(t, flags)) {
             solo.push_back(i);
+            continue;
+        }
+        if (!t.targets || t.targets->T == 0) {
+            plain.push_back(i);
             continue;
         }
         const std::tuple<int, bool, bool> gk{t.par->nr, t.par->eps_3 > 0.f,
@@ -5702,6 +5711,16 @@ void erp_run_tracks_impl(erp_ctx* ctx, const erp_track* tracks, int64_t ntracks,
         if (it == groups.end()) groups.push_back({gk, {i}});
         else it->second.push_back(i);
     }
+    for (int64_t i : plain) {
+        const int nr = tracks[i].par->nr;
+        const bool s3 = tracks[i].par->eps_3 > 0.f;
+        auto it = std::find_if(groups.begin(), groups.end(), [&](const auto& g) {
+            return std::get<0>(g.first) == nr && std::get<1>(g.first) == s3;
+        });
+        if (it == groups.end()) groups.push_back({{nr, s3, false}, {i}});
+        else it->second.push_back(i);
+    }
+    for (auto& g : groups) std::sort(g.second.begin(), g.second.end());
     for (int64_t i : solo) {
         const erp_track& t = tracks[i];
         erp_run_impl(ctx, t.par, t.mesh, t.targets, t.shots, t.ns, nullptr, 0,
