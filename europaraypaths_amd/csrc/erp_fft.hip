@@ -1847,9 +1847,6 @@ void target_pairs_half(erp_ctx* ctx, const FftPlan& p, const float2* A, const in
         if (crop) mt ? go(k11, nt) : go(k01, nt);
         else mt ? go(k10, nt) : go(k00, nt);
     };
-#define ERP_TPAIR_VARIANTS(NTB)                                                       \
-    pick(k_tpair_half<NTB, false, false>, k_tpair_half<NTB, true, false>,            \
-         k_tpair_half<NTB, false, true>, k_tpair_half<NTB, true, true>, NTB)
     // the wave-local transforms take Gnat in their layout
 #define ERP_TPAIR_HALF(NTB)                                                             \
     pick(k_tpair_half<NTB, false, false>, k_tpair_half<NTB, true, false>,              \

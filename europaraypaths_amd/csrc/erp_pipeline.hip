@@ -4701,8 +4701,6 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
                 float2* Bq = A + (size_t)C * P;                 // y / Y' (and MODE 1: B)
                 float2* Bs = spec ? Bq + (size_t)C * P : nullptr;
                 float2* Z = W.tC.as<float2>();                  // Z or fused workspace
-                // each shot's list holds Tcap slots of which htc[2s] are used:
-                // copy only the leading columns that some shot uses
                 W.pairs.ensure(sizeof(int) * ((size_t)C * 4 + 2 * gcap + 3 * (size_t)S + 16));
                 int* dps = W.pairs.as<int>();
                 int* dpt = dps + C;
@@ -4739,6 +4737,7 @@ void erp_run_impl(erp_ctx* ctx, const erp_params* par, const erp_mesh* mesh,
                     for (int s = 0; s < S; ++s) maxc = std::max(maxc, htc[2 * s]);
                     std::vector<int> hl(short_lists ? 0 : (size_t)S * maxc);
                     if (maxc > 0 && !short_lists) {
+                        // a list holds Tcap slots: the columns that some shot uses
                         ERP_HIP_TRY(hipMemcpy2DAsync(hl.data(), sizeof(int) * maxc, list1,
                                                      sizeof(int) * Tcap, sizeof(int) * maxc, S,
                                                      hipMemcpyDeviceToHost, st));
