@@ -1727,8 +1727,8 @@ __device__ __forceinline__ void spec_factors(float sT, float cT, float cph, floa
 }
 
 // The same in the reference's steps, for the type-0 targets: their terms take
-// the factors squared, and the hardware functions' errors with them (the sinc
-// sums' error against 64 bits would be 1.8e-6 instead of 1.2e-6).
+// the factors squared, and their errors with them (with spec_factors on hardware
+// sines the sinc sums' error against 64 bits was 1.8e-6 instead of 1.2e-6).
 __device__ __forceinline__ void spec_factors_angles(float sT, float cT, float Iu, float Iv,
                                                     const Rec& rec, int64_t r, const KPar& kp,
                                                     float* vi, float* vo) {
@@ -3288,7 +3288,11 @@ __global__ void k_pair_targets_rows(int* __restrict__ ptgt, const int* __restric
 // ---------------------------------------------------------------------------
 constexpr int DS_BINS = 4;             // bins per thread
 constexpr int DS_TILE = NT * DS_BINS;  // bins per workgroup
-constexpr int DS_MIN_ITEMS = 4;        // term groups (of NT) worth a workgroup of their own
+// Term groups (of NT) per workgroup at least, so that a shot's few groups are
+// not split into partial rows of little each.  With few shots the facets' own
+// sums are then too few workgroups for the device: 16 shots of 1000 bins and
+// 8.8e3 facets, 144 of them, a run of 1.02 ms (1 group: 0.75, 2: 0.84, 8: 1.58).
+constexpr int DS_MIN_ITEMS = 4;
 // Partial rows a shot's terms are split into at most: enough workgroups for
 // one shot to fill the device, 1 MB of partial rows per shot.
 __host__ __device__ inline int direct_splits_max(int nr) {
