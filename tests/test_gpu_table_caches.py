@@ -9,6 +9,7 @@ Bounds: the caches keep at most 256 MB of narrow-band tables (45 MB each here),
 reads besides.  384 MB covers that and what the work buffers grow by; the
 tables of one pass would take 1080 MB."""
 import ctypes
+import threading
 
 import numpy as np
 import pytest
@@ -133,3 +134,30 @@ def test_a_context_gives_its_tables_back():
     used = before - free_bytes()
     print(used // MB, flush=True)
     assert used <= 16 * MB  # 6 x 8 range kernels in three layouts would take 36
+
+
+def test_dropped_beside_running_tracks(ctx):
+    """Jobs drop and build tables while another thread's multi-track calls,
+    which capture and replay graphs, hold some of them."""
+    jobs = jobs_of(ctx)
+    ref = run_all(ctx, "run", jobs)
+    got, errors = [], []
+
+    def tracks():
+        try:
+            for _ in range(4):
+                got.append(run_all(ctx, "tracks", jobs[:6]))
+        except Exception as e:  # noqa: BLE001 - reported by the main thread
+            errors.append(e)
+
+    th = threading.Thread(target=tracks)
+    th.start()
+    served = [run_all(ctx, "submit", jobs[k:] + jobs[:k]) for k in (0, 12)]
+    th.join()
+    assert not errors, errors
+    for g in got:
+        for a, b in zip(g, ref):
+            compare_traces(a, b)
+    for k, g in zip((0, 12), served):
+        for a, b in zip(g, ref[k:] + ref[:k]):
+            compare_traces(a, b)
